@@ -1,0 +1,90 @@
+"""The kernels that give a system several lanes (kernels_row.h) against the lane-per-system kernels and the oracle:
+bit-identical states, sub-step counts and status in exact mode, at the edges of their ranges."""
+import numpy as np
+import pytest
+
+import oracle_lib as O
+from wind_amd import api
+from wind_amd import networks as W
+
+pytestmark = pytest.mark.gpu
+
+
+def same(a, b):
+    na, nb = np.isnan(a), np.isnan(b)
+    return np.array_equal(na, nb) and np.array_equal(a[~na].view(np.uint32), b[~nb].view(np.uint32))
+
+
+def run(net, n, y0, c, kernel, **kw):
+    y = y0.copy()
+    steps, status = np.zeros(n, np.int32), np.full(n, -1, np.int32)
+    kw = {"tend": 1.0, "nfix": 1, "tol": 1e-3, **kw}
+    total, _ = api.integrate(net, 0.0, kw.pop("tend"), kw.pop("nfix"), c, y, n, kw["tol"], kw.pop("tol"), kernel=kernel,
+                             steps_out=steps, status_out=status, **kw)
+    assert total == int(steps.astype(np.int64).sum())
+    return y, steps, status
+
+
+NETS = {
+    "nr_test": (lambda: api.Network.builtin(api.NET_NR_TEST), lambda n: W.nr_test_systems(n, 5)[:2],
+                {"tend": 1.0, "nfix": 1000}),
+    "katz96": (lambda: api.Network.builtin(api.NET_KATZ96),
+               lambda n: tuple(np.resize(a, n * k) for a, k in ((W.KATZ96_FIXTURE_Y, 5), (W.KATZ96_FIXTURE_C, 10))),
+               {"tend": 200.0, "tol": 5e-3}),
+    "hhe6": (lambda: api.Network.builtin(api.NET_HHE6, W.hhe6_params()), lambda n: W.hhe6_systems(n, 9),
+             {"tend": 1e4}),
+    "mixed5": (lambda: api.Network.plugin("mixed5"),
+               lambda n: W.mass_action_systems(n, 5, 11, W.MIXED_SCALE_RANGE), {"tend": 1e7}),
+}
+
+
+@pytest.mark.parametrize("name", list(NETS))
+@pytest.mark.parametrize("method", [api.SIE, api.RK2])
+@pytest.mark.parametrize("controller", [api.CTRL_REFERENCE, api.CTRL_ADAPTIVE])
+@pytest.mark.parametrize("n", [1, 3, 4, 5, 67])
+def test_row_kernel_equals_lane_kernel(name, method, controller, n):
+    make, systems, kw = NETS[name]
+    net, (y0, c) = make(), systems(n)
+    kw = dict(kw, method=method, controller=controller, max_attempts=3000)
+    a, b = (run(net, n, y0, c, k, **kw) for k in (api.KERNEL_LANE, api.KERNEL_AUTO))
+    assert same(a[0], b[0]) and np.array_equal(a[1], b[1]) and np.array_equal(a[2], b[2])
+
+
+def test_row_kernel_strides_hints_and_non_finite_states():
+    net, n = api.Network.builtin(api.NET_HHE6, W.hhe6_params()), 129
+    y0, c = W.hhe6_systems(n, 21)
+    y0[6 * 7 + 5] = np.inf
+    y0[6 * 8 + 1] = np.nan
+    y0[6 * 9:6 * 10] = 3e38
+    wide = np.full(3 * n, 7.0, np.float32)
+    wide[::3] = c
+    kw = {"tend": 1e3, "max_attempts": 500, "tol": 1e-3}
+    ref = run(net, n, y0, c, api.KERNEL_LANE, **kw)
+    hint = np.random.default_rng(0).integers(1, 1000, n).astype(np.int32)
+    for extra in ({"const_stride": 3}, {"cost_hint": hint}):
+        got = run(net, n, y0, wide if "const_stride" in extra else c, api.KERNEL_AUTO, **kw, **extra)
+        assert same(ref[0], got[0]) and np.array_equal(ref[1], got[1]) and np.array_equal(ref[2], got[2])
+
+
+@pytest.mark.parametrize("tiles", [4, 5, 50])
+@pytest.mark.parametrize("method", [O.SIE, O.RK2])
+@pytest.mark.parametrize("controller", [api.CTRL_REFERENCE, api.CTRL_ADAPTIVE])
+def test_tiled_network_equals_oracle_also_where_a_tile_overflows(tiles, method, controller):
+    """A tile whose state overflows: in the dense elimination its infinities reach the other tiles' equations."""
+    n, N, name = 4, 5 * tiles, f"katz96_t{tiles}"
+    c = W.KATZ96_FIXTURE_C.copy()
+    y0 = np.tile(W.KATZ96_FIXTURE_Y.reshape(4, 5), (1, tiles)).astype(np.float32)
+    rng = np.random.default_rng(tiles)
+    y0 *= rng.uniform(0.5, 1.5, y0.shape).astype(np.float32)  # tiles that differ
+    y0[1, 5 * (tiles - 1) + 1] = 3e38
+    y0[2, 5 * (tiles // 2)] = np.inf
+    y0 = y0.reshape(-1)
+    yr = y0.copy()
+    tend = 0.5
+    _, sr, tr = O.gold_integrate(method, O.generated(name), 0.0, tend, 1, c, yr, n, 5e-3, 5e-3, const_stride=10,
+                                 max_attempts=40, controller=controller)
+    y, steps, status = run(api.Network.plugin(name), n, y0, c, api.KERNEL_AUTO, tend=tend, tol=5e-3, method=method,
+                           controller=controller, max_attempts=40)
+    if method == O.SIE and controller == api.CTRL_REFERENCE:
+        assert np.isnan(yr.reshape(n, N)[2]).sum() > 5  # it does reach them
+    assert same(y, yr) and np.array_equal(steps, sr) and np.array_equal(status, tr)

@@ -208,6 +208,12 @@ def _check_expr_network(spec, N, C):
         _check_tokens(_tokens(e), f"jac[{k}]", N, C, jnames, True)
 
 
+def _jidx(k, NB, S):
+    """Index text of base entry k = j*NB + i with column stride S (a number, or the name of one)."""
+    j, i = divmod(int(k), NB)
+    return str(j * S + i) if isinstance(S, int) else f"{j} * {S} + {i}"
+
+
 def _emit(toks, NB, S, tile_scope):
     """C text of a token list; y[i] and J[k] reindexed for the tile scope."""
     out, i = [], 0
@@ -220,7 +226,7 @@ def _emit(toks, NB, S, tile_scope):
             elif v == "c":
                 out.append(f"c[{k}]")
             else:
-                out.append(f"Jt[{(k // NB) * S + k % NB}]")
+                out.append(f"Jt[{_jidx(k, NB, S)}]")
             i += 4
             continue
         out.append(v)
@@ -249,7 +255,7 @@ def _expr_body(spec, N, S, real):
     fj = sum(_count_ops(_tokens(e)) for _, e in spec.get("jac", []))
     fj_t = sum(_count_ops(_tokens(e)) for _, e in spec.get("jac_temps", spec.get("temps", [])))
     rhs = [f"ft[{i}] = {_emit(_tokens(e), N, S, True)};" for i, e in enumerate(spec["rhs"])]
-    jac = [f"Jt[{(int(k) // N) * S + int(k) % N}] = {_emit(_tokens(e), N, S, True)};" for k, e in spec.get("jac", [])]
+    jac = [f"Jt[{_jidx(k, N, S)}] = {_emit(_tokens(e), N, S, True)};" for k, e in spec.get("jac", [])]
     return temps, rhs, jtemps, jac, (fr, fr_t), (fj, fj_t)
 
 
@@ -293,12 +299,14 @@ def _reaction_body(spec, N, S, real):
             js += [f"const auto da = ks * yt[{b}];", f"const auto db = ks * yt[{a}];"]
             fj += 2
             for t, sg in targets:
-                js += [f"Jt[{a * S + t}] = Jt[{a * S + t}] {sg} da;", f"Jt[{b * S + t}] = Jt[{b * S + t}] {sg} db;"]
+                ja, jb = _jidx(a * N + t, N, S), _jidx(b * N + t, N, S)
+                js += [f"Jt[{ja}] = Jt[{ja}] {sg} da;", f"Jt[{jb}] = Jt[{jb}] {sg} db;"]
                 fj += 2
         else:
             js += ["const auto da = ks;"]
             for t, sg in targets:
-                js += [f"Jt[{a * S + t}] = Jt[{a * S + t}] {sg} da;"]
+                ja = _jidx(a * N + t, N, S)
+                js += [f"Jt[{ja}] = Jt[{ja}] {sg} da;"]
                 fj += 1
         jac.append("{ " + " ".join(js) + " }")
     return [], rhs, [], jac, (fr, 0), (fj, 0)
@@ -320,7 +328,7 @@ def generate(spec) -> dict:
     expr = "rhs" in spec
     R = 0 if expr else len(spec["reactions"]) * T
     body = _expr_body if expr else _reaction_body
-    temps, rhs, jtemps, jac, (fr, fr_t), (fj, fj_t) = body(spec, NB, N, "float")
+    temps, rhs, jtemps, jac, (fr, fr_t), (fj, fj_t) = body(spec, NB, "LD", "float")
     flops_rhs, flops_jac = fr * T + fr_t, fj * T + fj_t
     unroll = "#pragma unroll" if N <= LANE_MAX_N else "#pragma unroll 1"
     ind = "        "
@@ -339,20 +347,27 @@ struct Net {{
     static constexpr int N = {N};
     static constexpr int NCONST = {C};
     struct Params {{}};
-    // tile t of the RHS / Jacobian (the tiles are independent)
+    // whether the tiles read the first tile's state (the temporaries)
+    static constexpr bool kFirstTile = {"true" if temps or jtemps else "false"};
+    // One tile of the RHS / Jacobian (the tiles are independent) from the
+    // first tile's state y and the tile's own yt; Jacobian columns LD apart.
+    template <class M>
+    __device__ static inline void rhs_at(const float *c, const float *y, const float *yt, float *ft) {{
+{chr(10).join(ind + l for l in temps)}
+{chr(10).join(ind + l for l in rhs)}
+    }}
+    template <class M, int LD>
+    __device__ static inline void jac_at(const float *c, const float *y, const float *yt, float *Jt) {{
+{chr(10).join(ind + l for l in jtemps)}
+{chr(10).join(ind + l for l in jac)}
+    }}
     template <class M>
     __device__ static inline void rhs_tile(const Params &, const float *c, const float *y, float *f, int t) {{
-{chr(10).join(ind + l for l in temps)}
-        const float *yt = y + t * NB;
-        float *ft = f + t * NB;
-{chr(10).join(ind + l for l in rhs)}
+        rhs_at<M>(c, y, y + t * NB, f + t * NB);
     }}
     template <class M>
     __device__ static inline void jac_tile(const Params &, const float *c, const float *y, float *J, int t) {{
-{chr(10).join(ind + l for l in jtemps)}
-        const float *yt = y + t * NB;
-        float *Jt = J + (size_t)t * NB * (N + 1);
-{chr(10).join(ind + l for l in jac)}
+        jac_at<M, N>(c, y, y + t * NB, J + (size_t)t * NB * (N + 1));
     }}
     template <class M>
     __device__ static inline void rhs(const Params &p, const float *c, const float *y, float *f) {{

@@ -13,6 +13,7 @@
 #include <type_traits>
 
 #include "kernels_mass_action.h"
+#include "kernels_row.h"
 
 namespace wind {
 
@@ -49,10 +50,8 @@ __host__ __device__ constexpr int gen_block_base_floats() {
     return 5 * Net::N + ((Net::NCONST + 3) & ~3);
 }
 
-template <class Net, int METHOD, bool FAST, bool PIVOT = false>
-__global__ void __launch_bounds__(256) gen_block_integrate(IntegrateArgs a, typename Net::Params p, float *gscratch,
-                                                           int mat_in_lds) {
-    extern __shared__ float lds[];
+template <class Net, bool FAST>
+__device__ inline MALayout gen_block_layout(float *lds, float *gscratch, int mat_in_lds) {
     constexpr int N = Net::N;
     MALayout L;
     L.y = lds;
@@ -61,14 +60,50 @@ __global__ void __launch_bounds__(256) gen_block_integrate(IntegrateArgs a, type
     L.f = L.y1 + N;
     L.g = L.f + N;
     L.w = L.da = L.db = nullptr;
-    float *cc = L.g + N;
     constexpr size_t per_block = (size_t)(FAST ? 1 : 2) * N * N;
     float *mats = mat_in_lds ? lds + gen_block_base_floats<Net>() : gscratch + (size_t)blockIdx.x * per_block;
     L.M = mats;
     L.Inv = FAST ? nullptr : mats + (size_t)N * N;
+    return L;
+}
+
+template <class Net, int METHOD, bool FAST, bool PIVOT = false>
+__global__ void __launch_bounds__(256) gen_block_integrate(IntegrateArgs a, typename Net::Params p, float *gscratch,
+                                                           int mat_in_lds) {
+    extern __shared__ float lds[];
+    MALayout L = gen_block_layout<Net, FAST>(lds, gscratch, mat_in_lds);
     using Ev = GenEval<Net, typename std::conditional<FAST, MathFast, MathExact>::type>;
-    Ev ev{p, cc};
-    block_integrate_systems<METHOD, FAST, Ev, PIVOT>(a, N, L, ev);
+    Ev ev{p, L.g + Net::N};
+    block_integrate_systems<METHOD, FAST, Ev, PIVOT>(a, Net::N, L, ev);
+}
+
+// Exact mode, tiled networks: a row of lanes per tile (row_tile_integrate),
+// the dense path of gen_block_integrate for systems that meet a non-finite
+// value.  Bound by the latency of one attempt's instruction stream and its
+// two barriers, not by the N^3 of a dense inverse: 80 Katz96 systems, one
+// call through the drop-in, N = 50 (t = 200) 44.5 -> 0.35 ms, N = 250
+// (t = 5) 767 -> 0.21 ms.
+template <class Net, int METHOD>
+__global__ void __launch_bounds__(row_tile_threads<Net>()) gen_tile_integrate(IntegrateArgs a, typename Net::Params p,
+                                                                             float *gscratch, int mat_in_lds) {
+    extern __shared__ float lds[];
+    row_tile_integrate<Net, METHOD>(a, p, [&](int sid) {
+        MALayout L = gen_block_layout<Net, false>(lds, gscratch, mat_in_lds);
+        GenEval<Net, MathExact> ev{p, L.g + Net::N};
+        return block_integrate_system<METHOD, false>(a, Net::N, L, ev, sid);
+    });
+}
+
+// The kernel of a launch and its threads per workgroup.
+template <class Net, int METHOD, bool FAST, bool PIVOT>
+inline auto gen_block_kernel(int nsys, int num_cu, int *threads) {
+    if constexpr (!FAST && row_tile_network<Net>()) {
+        *threads = row_tile_threads<Net>();
+        return gen_tile_integrate<Net, METHOD>;
+    } else {
+        *threads = block_threads(Net::N, nsys, num_cu);
+        return gen_block_integrate<Net, METHOD, FAST, PIVOT>;
+    }
 }
 
 // Launch shape of gen_block_integrate: threads, grid, LDS bytes, and the
@@ -88,10 +123,9 @@ inline int gen_block_shape(int nsys, int num_cu, float share, int grid_cap, GenB
         return WIND_ERR_DEVICE;
     const size_t base = sizeof(float) * (size_t)gen_block_base_floats<Net>();
     const size_t mats = sizeof(float) * (FAST ? 1 : 2) * (size_t)N * N;
-    s->T = block_threads(N, nsys, num_cu);
+    auto kfn = gen_block_kernel<Net, METHOD, FAST, PIVOT>(nsys, num_cu, &s->T);
     s->in_lds = base + mats + 256 <= (size_t)max_lds;
     s->lds = base + (s->in_lds ? mats : 0);
-    auto kfn = gen_block_integrate<Net, METHOD, FAST, PIVOT>;
     if (s->lds > 65536 &&
         hipFuncSetAttribute((const void *)kfn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)s->lds) != hipSuccess)
         return WIND_ERR_DEVICE;
@@ -112,7 +146,8 @@ inline int gen_block_launch(const IntegrateArgs &a, const typename Net::Params &
     int rc = gen_block_shape<Net, METHOD, FAST, PIVOT>(a.nsys, num_cu, share, grid_cap, &s);
     if (rc) return rc;
     if (s.scratch > 0 && (!scratch || scratch_bytes < s.scratch)) return WIND_ERR_ARGUMENT;
-    hipLaunchKernelGGL((gen_block_integrate<Net, METHOD, FAST, PIVOT>), dim3(s.grid), dim3(s.T), s.lds, st, a, p,
+    auto kfn = gen_block_kernel<Net, METHOD, FAST, PIVOT>(a.nsys, num_cu, &s.T);
+    hipLaunchKernelGGL(kfn, dim3(s.grid), dim3(s.T), s.lds, st, a, p,
                        s.in_lds ? nullptr : scratch, s.in_lds ? 1 : 0);
     return hipGetLastError() == hipSuccess ? WIND_OK : WIND_ERR_DEVICE;
 }

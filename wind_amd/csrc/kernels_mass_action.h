@@ -205,94 +205,100 @@ __device__ inline void block_lu_fast(int N, MALayout &L) {
     }
 }
 
-// The per-system loop of the one-workgroup-per-system kernels: each
-// workgroup takes systems blockIdx.x, blockIdx.x + gridDim.x, ... and runs
-// the step-doubling attempts of common_gold.c:77-148 with the solver of the
-// mode.  `ev` evaluates the network: ev.load(a, sid) reads the system's
-// constants, ev.eval(yv, L, nh, want_jac) writes f(yv) to L.f and, with
-// want_jac, L.M = I + nh J(yv) (column-major), ending with a barrier.
+// One system by a whole workgroup: the step-doubling attempts of
+// common_gold.c:77-148 with the solver of the mode.  `ev` evaluates the
+// network: ev.load(a, sid) reads the system's constants,
+// ev.eval(yv, L, nh, want_jac) writes f(yv) to L.f and, with want_jac,
+// L.M = I + nh J(yv) (column-major), ending with a barrier.  Returns the
+// attempts made.
 template <int METHOD, bool FAST, class Eval, bool PIVOT = false>
-__device__ inline void block_integrate_systems(const IntegrateArgs &a, int N, MALayout &L, Eval &ev) {
+__device__ inline int block_integrate_system(const IntegrateArgs &a, int N, MALayout &L, Eval &ev, int sid) {
     const int t = threadIdx.x, T = blockDim.x;
     __shared__ int s_flag;
-    __shared__ double s_err[4];
-    unsigned long long steps = 0;
-    for (int sid = blockIdx.x; sid < a.nsys; sid += gridDim.x) {
-        for (int i = t; i < N; i += T) L.y[i] = a.equations[(size_t)sid * N + i];
-        ev.load(a, sid);
-        __syncthreads();
-        float tnow = a.tnow, h = a.h0;
-        int unsolved = 0, attempts = 0, status = WIND_STATUS_OK;
-        while (tnow < a.tend) {
-            const float hh = fminf(a.tend - tnow, h);
-            const float tb = tnow + hh;
-            const float hs_full = tb - tnow, hs_half = (tb - tnow) / 2.0f;
-            for (int pass = 0; pass < 3; pass++) {
-                const float hs = pass == 0 ? hs_full : hs_half;
-                if (pass != 2) {
-                    for (int i = t; i < N; i += T) L.yw[i] = L.y[i];
-                    __syncthreads();
-                }
-                ev.eval(L.yw, L, -hs, METHOD == WIND_SIE);
-                if (METHOD == WIND_SIE) {
-                    if (FAST)
-                        block_lu_fast<PIVOT>(N, L);
-                    else
-                        block_gje_exact(N, L);
-                    for (int i = t; i < N; i += T)
-                        L.yw[i] = FAST ? fmaf(hs, L.g[i], L.yw[i]) : L.yw[i] + hs * L.g[i];
-                } else {
-                    __syncthreads();
-                    for (int i = t; i < N; i += T)
-                        L.yw[i] = FAST ? fmaf(hs, L.f[i], L.yw[i]) : L.yw[i] + hs * L.f[i];
-                }
+    __shared__ double s_err[16];
+    for (int i = t; i < N; i += T) L.y[i] = a.equations[(size_t)sid * N + i];
+    ev.load(a, sid);
+    __syncthreads();
+    float tnow = a.tnow, h = a.h0;
+    int unsolved = 0, attempts = 0, status = WIND_STATUS_OK;
+    while (tnow < a.tend) {
+        const float hh = fminf(a.tend - tnow, h);
+        const float tb = tnow + hh;
+        const float hs_full = tb - tnow, hs_half = (tb - tnow) / 2.0f;
+        for (int pass = 0; pass < 3; pass++) {
+            const float hs = pass == 0 ? hs_full : hs_half;
+            if (pass != 2) {
+                for (int i = t; i < N; i += T) L.yw[i] = L.y[i];
                 __syncthreads();
-                if (pass == 0)
-                    for (int i = t; i < N; i += T) L.y1[i] = L.yw[i];
             }
-            if (t == 0) s_flag = 0;
-            __syncthreads();
-            bool fail = false;
-            double err = 0.0;
-            if (a.controller == WIND_CTRL_REFERENCE) {
+            ev.eval(L.yw, L, -hs, METHOD == WIND_SIE);
+            if (METHOD == WIND_SIE) {
+                if (FAST)
+                    block_lu_fast<PIVOT>(N, L);
+                else
+                    block_gje_exact(N, L);
                 for (int i = t; i < N; i += T)
-                    fail = fail || species_fails<METHOD>(L.y1[i], L.yw[i], a.ABS, a.REL);
-                if (fail) s_flag = 1;
+                    L.yw[i] = FAST ? fmaf(hs, L.g[i], L.yw[i]) : L.yw[i] + hs * L.g[i];
             } else {
-                for (int i = t; i < N; i += T) err = err_max(err, err_term(L.y1[i], L.yw[i], a.ABS, a.REL));
+                __syncthreads();
+                for (int i = t; i < N; i += T)
+                    L.yw[i] = FAST ? fmaf(hs, L.f[i], L.yw[i]) : L.yw[i] + hs * L.f[i];
+            }
+            __syncthreads();
+            if (pass == 0)
+                for (int i = t; i < N; i += T) L.y1[i] = L.yw[i];
+        }
+        if (t == 0) s_flag = 0;
+        __syncthreads();
+        bool fail = false;
+        double err = 0.0;
+        if (a.controller == WIND_CTRL_REFERENCE) {
+            for (int i = t; i < N; i += T)
+                fail = fail || species_fails<METHOD>(L.y1[i], L.yw[i], a.ABS, a.REL);
+            if (fail) s_flag = 1;
+        } else {
+            for (int i = t; i < N; i += T) err = err_max(err, err_term(L.y1[i], L.yw[i], a.ABS, a.REL));
 #pragma unroll
-                for (int off = 32; off > 0; off >>= 1) err = err_max(err, __shfl_xor(err, off));
-                if (__lane_id() == 0) s_err[t >> 6] = err;
-            }
-            __syncthreads();
-            const bool flag = s_flag != 0;
-            if (a.controller != WIND_CTRL_REFERENCE) {
-                err = s_err[0];
-                for (int wv = 1; wv < (T + 63) / 64; wv++) err = err_max(err, s_err[wv]);
-            }
-            attempts++;
-            const bool acc = control_step<METHOD>(a.controller, a.tend, hh, flag, err, tnow, h, unsolved, status);
-            if (acc) {
-                const bool extrap = METHOD == WIND_RK2 || a.controller != WIND_CTRL_REFERENCE;
-                for (int i = t; i < N; i += T) L.y[i] = extrap ? 2.0f * L.yw[i] - L.y1[i] : L.yw[i];
-            }
-            __syncthreads();
-            if (status != WIND_STATUS_OK) break;
-            if (attempts >= a.max_attempts && tnow < a.tend) {
-                status = WIND_STATUS_EXHAUSTED;
-                break;
-            }
+            for (int off = 32; off > 0; off >>= 1) err = err_max(err, __shfl_xor(err, off));
+            if (__lane_id() == 0) s_err[t >> 6] = err;
         }
         __syncthreads();
-        for (int i = t; i < N; i += T) a.equations[(size_t)sid * N + i] = L.y[i];
-        if (t == 0) {
-            if (a.steps_out) a.steps_out[sid] = 3 * attempts;
-            if (a.status_out) a.status_out[sid] = status;
-            steps += 3ull * (unsigned long long)attempts;
+        const bool flag = s_flag != 0;
+        if (a.controller != WIND_CTRL_REFERENCE) {
+            err = s_err[0];
+            for (int wv = 1; wv < (T + 63) / 64; wv++) err = err_max(err, s_err[wv]);
+        }
+        attempts++;
+        const bool acc = control_step<METHOD>(a.controller, a.tend, hh, flag, err, tnow, h, unsolved, status);
+        if (acc) {
+            const bool extrap = METHOD == WIND_RK2 || a.controller != WIND_CTRL_REFERENCE;
+            for (int i = t; i < N; i += T) L.y[i] = extrap ? 2.0f * L.yw[i] - L.y1[i] : L.yw[i];
         }
         __syncthreads();
+        if (status != WIND_STATUS_OK) break;
+        if (attempts >= a.max_attempts && tnow < a.tend) {
+            status = WIND_STATUS_EXHAUSTED;
+            break;
+        }
     }
-    if (t == 0 && steps) atomicAdd(a.counters + 1, steps);
+    __syncthreads();
+    for (int i = t; i < N; i += T) a.equations[(size_t)sid * N + i] = L.y[i];
+    if (t == 0) {
+        if (a.steps_out) a.steps_out[sid] = 3 * attempts;
+        if (a.status_out) a.status_out[sid] = status;
+    }
+    __syncthreads();
+    return attempts;
+}
+
+// The per-system loop of the one-workgroup-per-system kernels: each
+// workgroup takes systems blockIdx.x, blockIdx.x + gridDim.x, ...
+template <int METHOD, bool FAST, class Eval, bool PIVOT = false>
+__device__ inline void block_integrate_systems(const IntegrateArgs &a, int N, MALayout &L, Eval &ev) {
+    unsigned long long steps = 0;
+    for (int sid = blockIdx.x; sid < a.nsys; sid += gridDim.x)
+        steps += 3ull * (unsigned long long)block_integrate_system<METHOD, FAST, Eval, PIVOT>(a, N, L, ev, sid);
+    if (threadIdx.x == 0 && steps) atomicAdd(a.counters + 1, steps);
 }
 
 // Network evaluation of the table-driven mass-action networks (one constant

@@ -223,6 +223,10 @@ struct NetHHe6 {
     __device__ static inline void rhs(const Params &p, const float *c, const float *y, float *f) {
         State s;
         state<M>(p, c, y, s, false);
+        rhs_of(s, y, f);
+    }
+
+    __device__ static inline void rhs_of(const State &s, const float *y, float *f) {
         const float xe = s.xe;
         float Rr = s.Rj[4] + s.Rj[5];
         float w0 = (s.Rj[0] * xe + s.G[0]) * y[0];
@@ -246,17 +250,53 @@ struct NetHHe6 {
         f[5] = heat - ((cci + crec) + cff) * s.phi;
     }
 
-    // d/dy_k of w = (R xe + G) y_s.
-    __device__ static inline void dw(const State &s, float Rv, float g, float G, int sidx,
-                                     const float *y, float *out) {
-        const float dxe[6] = {0.0f, 1.0f, 0.0f, 1.0f, 2.0f, 0.0f};
-#pragma unroll
-        for (int k = 0; k < 6; k++) {
-            float t = (g * s.dT[k]) * s.xe + Rv * dxe[k];
-            float v = t * y[sidx];
-            if (k == sidx) v = v + (Rv * s.xe + G);
-            out[k] = v;
-        }
+    // d/dy_k of w = (R xe + G) y_sidx.
+    __device__ static inline float dw(const State &s, float Rv, float g, float G, int sidx, const float *y, int k,
+                                      float dT, float dxe) {
+        const float t = (g * dT) * s.xe + Rv * dxe;
+        const float v = t * y[sidx];
+        return k == sidx ? v + (Rv * s.xe + G) : v;
+    }
+
+    // Column k of the exact Jacobian, from the derivatives by y_k of T, phi,
+    // xe and the ion sum, and the photoheating per y_k.
+    __device__ static inline void jac_col(const State &s, const float *y, int k, float dT, float dphi, float dxe,
+                                          float dion, float heat, float *col) {
+        const float xe = s.xe;
+        const float Rr = s.Rj[4] + s.Rj[5];
+        const float gr = s.gj[4] + s.gj[5];
+        const float dw0 = dw(s, s.Rj[0], s.gj[0], s.G[0], 0, y, k, dT, dxe);
+        const float dw1 = dw(s, s.Rj[1], s.gj[1], s.G[1], 2, y, k, dT, dxe);
+        const float dw2 = dw(s, s.Rj[2], s.gj[2], s.G[2], 3, y, k, dT, dxe);
+        const float dw3 = dw(s, s.Rj[3], s.gj[3], 0.0f, 1, y, k, dT, dxe);
+        const float dw4 = dw(s, Rr, gr, 0.0f, 3, y, k, dT, dxe);
+        const float dw5 = dw(s, s.Rj[6], s.gj[6], 0.0f, 4, y, k, dT, dxe);
+        const float dc0 = dw(s, s.Rj[0], s.gj[0], 0.0f, 0, y, k, dT, dxe);
+        const float dc1 = dw(s, s.Rj[1], s.gj[1], 0.0f, 2, y, k, dT, dxe);
+        const float dc2 = dw(s, s.Rj[2], s.gj[2], 0.0f, 3, y, k, dT, dxe);
+        const float w3 = (s.Rj[3] * xe) * y[1];
+        const float w4 = (Rr * xe) * y[3];
+        const float w5 = (s.Rj[6] * xe) * y[4];
+        const float W = (w3 + w4) + w5;
+        const float T4 = s.T * 1.0e-4f;
+        const float recT = RECC * T4;
+        const float ion = (y[1] + y[3]) + 4.0f * y[4];
+        const float LN = LFF * s.nHyr;
+        const float LNs = LN * s.sqT;
+        const float xion = xe * ion;
+        const float dsqc = (0.5f * s.sqT) * s.invT;
+        const float cci = (((s.Rj[0] * xe) * y[0]) * CHI0 + ((s.Rj[1] * xe) * y[2]) * CHI1) +
+                          ((s.Rj[2] * xe) * y[3]) * CHI2;
+        const float cool = (cci + W * recT) + LNs * xion;
+        col[0] = dw3 - dw0;
+        col[1] = dw0 - dw3;
+        col[2] = dw4 - dw1;
+        col[3] = (dw1 + dw5) - (dw2 + dw4);
+        col[4] = dw2 - dw5;
+        const float dcci = (dc0 * CHI0 + dc1 * CHI1) + dc2 * CHI2;
+        const float dcrec = ((dw3 + dw4) + dw5) * recT + W * (RECC * (dT * 1.0e-4f));
+        const float dcff = (LN * (dsqc * dT)) * xion + LNs * (dxe * ion + xe * dion);
+        col[5] = heat - (((dcci + dcrec) + dcff) * s.phi + cool * dphi);
     }
 
     // Fast-mode Jacobian from its structure (other rounding than jac's exact
@@ -327,52 +367,11 @@ struct NetHHe6 {
             jac_fast(s, y, J);
             return;
         }
-        const float xe = s.xe;
-        float Rr = s.Rj[4] + s.Rj[5];
-        float gr = s.gj[4] + s.gj[5];
-        float dw0[6], dw1[6], dw2[6], dw3[6], dw4[6], dw5[6], dc0[6], dc1[6], dc2[6];
-        dw(s, s.Rj[0], s.gj[0], s.G[0], 0, y, dw0);
-        dw(s, s.Rj[1], s.gj[1], s.G[1], 2, y, dw1);
-        dw(s, s.Rj[2], s.gj[2], s.G[2], 3, y, dw2);
-        dw(s, s.Rj[3], s.gj[3], 0.0f, 1, y, dw3);
-        dw(s, Rr, gr, 0.0f, 3, y, dw4);
-        dw(s, s.Rj[6], s.gj[6], 0.0f, 4, y, dw5);
-        dw(s, s.Rj[0], s.gj[0], 0.0f, 0, y, dc0);
-        dw(s, s.Rj[1], s.gj[1], 0.0f, 2, y, dc1);
-        dw(s, s.Rj[2], s.gj[2], 0.0f, 3, y, dc2);
-        float w3 = (s.Rj[3] * xe) * y[1];
-        float w4 = (Rr * xe) * y[3];
-        float w5 = (s.Rj[6] * xe) * y[4];
-        float W = (w3 + w4) + w5;
-        float T4 = s.T * 1.0e-4f;
-        float recT = RECC * T4;
-        float ion = (y[1] + y[3]) + 4.0f * y[4];
-        float LN = LFF * s.nHyr;
-        float LNs = LN * s.sqT;
-        float xion = xe * ion;
-        float dsqc = (0.5f * s.sqT) * s.invT;
-        float cci = (((s.Rj[0] * xe) * y[0]) * CHI0 + ((s.Rj[1] * xe) * y[2]) * CHI1) +
-                    ((s.Rj[2] * xe) * y[3]) * CHI2;
-        float cool = (cci + W * recT) + LNs * xion;
         const float dxe[6] = {0.0f, 1.0f, 0.0f, 1.0f, 2.0f, 0.0f};
         const float dion[6] = {0.0f, 1.0f, 0.0f, 1.0f, 4.0f, 0.0f};
+        const float heat[6] = {s.G[0] * E0, 0.0f, s.G[1] * E1, s.G[2] * E2, 0.0f, 0.0f};
 #pragma unroll
-        for (int k = 0; k < 6; k++) {
-            float *col = J + 6 * k;
-            col[0] = dw3[k] - dw0[k];
-            col[1] = dw0[k] - dw3[k];
-            col[2] = dw4[k] - dw1[k];
-            col[3] = (dw1[k] + dw5[k]) - (dw2[k] + dw4[k]);
-            col[4] = dw2[k] - dw5[k];
-            float heat = 0.0f;
-            if (k == 0) heat = s.G[0] * E0;
-            if (k == 2) heat = s.G[1] * E1;
-            if (k == 3) heat = s.G[2] * E2;
-            float dcci = (dc0[k] * CHI0 + dc1[k] * CHI1) + dc2[k] * CHI2;
-            float dcrec = ((dw3[k] + dw4[k]) + dw5[k]) * recT + W * (RECC * (s.dT[k] * 1.0e-4f));
-            float dcff = (LN * (dsqc * s.dT[k])) * xion + LNs * (dxe[k] * ion + xe * dion[k]);
-            col[5] = heat - (((dcci + dcrec) + dcff) * s.phi + cool * s.dphi[k]);
-        }
+        for (int k = 0; k < 6; k++) jac_col(s, y, k, s.dT[k], s.dphi[k], dxe[k], dion[k], heat[k], J + 6 * k);
     }
 };
 
@@ -392,8 +391,14 @@ __device__ inline bool species_fails(float y1, float y2, float ABS, float REL) {
         den = (double)(2.0f * y2 - y1) + 1e-12;
     else
         den = (double)y2 + 1e-12;
-    double rel = fabs((double)d / den);
-    return rel >= (double)REL && fabsf(y1) > ABS && fabsf(y2) > ABS;
+    if (!(fabsf(y1) > ABS && fabsf(y2) > ABS)) return false;
+    // fabs(d / den) >= REL, decided by the product where the rounded
+    // quotient cannot lie on the other side of REL (the margin is 2^13 times
+    // the rounding errors), by the division only within the margin
+    const double ad = fabs((double)d), lim = (double)REL * fabs(den);
+    if (ad < lim * (1.0 - 0x1p-40)) return false;
+    if (ad > lim * (1.0 + 0x1p-40)) return true;
+    return fabs((double)d / den) >= (double)REL;
 }
 
 // ---------------------------------------------------------------------------
