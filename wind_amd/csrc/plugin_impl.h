@@ -76,6 +76,16 @@ int plugin_launch_method(const IntegrateArgs &a, int mode, int kernel, int num_c
         }
     } else if (choice == 0) {
         if constexpr (Net::N <= kGenLaneMaxN) {
+            if constexpr (row_network<Net>()) {
+                if (kernel == WIND_KERNEL_AUTO && a.nsys <= row_max_systems<Net, METHOD>(num_cu)) {
+                    auto k = row_integrate<Net, METHOD>;
+                    int grid = 0;
+                    const int rc = plugin_grid(k, 256, a.nsys * 16, num_cu, share, grid_cap, &grid);
+                    if (rc) return rc;
+                    hipLaunchKernelGGL(k, dim3(grid), dim3(256), 0, st, a, p);
+                    return hipGetLastError() == hipSuccess ? WIND_OK : WIND_ERR_DEVICE;
+                }
+            }
             auto k = lane_integrate<Net, METHOD, MathExact>;
             int grid = 0;
             const int rc = plugin_grid(k, 256, a.nsys, num_cu, share, grid_cap, &grid);

@@ -19,6 +19,7 @@
 #include <tuple>
 #include <vector>
 
+#include "kernels_row.h"
 #include "kernels_small.h"
 #include "plugin_abi.h"
 #include "wind_internal.h"
@@ -307,6 +308,13 @@ int launch_small(int num_cu, const wind_network *net, const IntegrateArgs &a, in
         if (a.trace.capacity > 0) return fail(WIND_ERR_UNSUPPORTED, "trace: the block kernel has no trace");
         const int grid = scaled_grid(num_cu, 32, sc, a.nsys);
         hipLaunchKernelGGL((block_integrate<Net, METHOD>), dim3(grid), dim3(64), 0, st, a, p);
+    } else if (mode == WIND_MODE_EXACT && kernel == WIND_KERNEL_AUTO && a.trace.capacity == 0 &&
+               a.nsys <= row_max_systems<Net, METHOD>(num_cu)) {
+        auto k = row_integrate<Net, METHOD>;
+        int grid = 0;
+        int rc = persistent_grid(num_cu, k, 256, a.nsys * 16, &grid, sc);
+        if (rc) return rc;
+        hipLaunchKernelGGL(k, dim3(grid), dim3(256), 0, st, a, p);
     } else if (mode == WIND_MODE_EXACT) {
         auto k = a.trace.capacity > 0 ? lane_integrate<Net, METHOD, MathExact, true>
                                       : lane_integrate<Net, METHOD, MathExact>;
