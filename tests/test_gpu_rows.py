@@ -50,6 +50,19 @@ def test_row_kernel_equals_lane_kernel(name, method, controller, n):
     assert same(a[0], b[0]) and np.array_equal(a[1], b[1]) and np.array_equal(a[2], b[2])
 
 
+@pytest.mark.parametrize("name,n,method,controller", [
+    ("katz96", 16385, api.SIE, api.CTRL_REFERENCE), ("katz96", 4097, api.RK2, api.CTRL_ADAPTIVE),
+    ("hhe6", 17001, api.SIE, api.CTRL_ADAPTIVE), ("hhe6", 140001, api.RK2, api.CTRL_REFERENCE),
+    ("mixed5", 70001, api.SIE, api.CTRL_REFERENCE)])
+def test_tail_on_rows_equals_lane_kernel(name, n, method, controller):
+    """Batches whose last systems the lane kernel hands over; an attempt cap that some reach."""
+    make, systems, kw = NETS[name]
+    net, (y0, c) = make(), systems(n)
+    kw = dict(kw, method=method, controller=controller, max_attempts=60)
+    a, b = (run(net, n, y0, c, k, **kw) for k in (api.KERNEL_LANE, api.KERNEL_AUTO))
+    assert same(a[0], b[0]) and np.array_equal(a[1], b[1]) and np.array_equal(a[2], b[2])
+
+
 def test_row_kernel_strides_hints_and_non_finite_states():
     net, n = api.Network.builtin(api.NET_HHE6, W.hhe6_params()), 129
     y0, c = W.hhe6_systems(n, 21)

@@ -314,14 +314,16 @@ inline int row_max_systems(int num_cu) {
     return (METHOD == WIND_SIE && Net::N >= 5 ? 64 : 16) * num_cu;
 }
 
-// One system per row, four per wave, taken from the device queue.
-template <class Net, int METHOD>
+// One system per row, four per wave, taken from the device queue; or (TAIL)
+// the systems that the lane kernel before it handed over (a.spill).
+template <class Net, int METHOD, bool TAIL = false>
 __global__ void __launch_bounds__(256) row_integrate(IntegrateArgs a, typename Net::Params p) {
     constexpr int N = Net::N, NC = Net::NCONST;
     static_assert(N <= 16, "one equation per lane of a 16-lane row");
     const int li = threadIdx.x & 15;
     const bool mine = li < N;
-    unsigned int *head = reinterpret_cast<unsigned int *>(a.counters);
+    unsigned int *head = reinterpret_cast<unsigned int *>(a.counters + (TAIL ? 3 : 0));
+    const int count = TAIL ? (int)*reinterpret_cast<const unsigned *>(a.counters + 2) : a.nsys;
     RowEval<Net, MathExact> ev(p, li);
     float y[N], c[NC > 0 ? NC : 1], yo = 0.0f, tnow = 0.0f, h = 0.0f;
     int sid = 0, unsolved = 0, attempts = 0, status = WIND_STATUS_OK;
@@ -334,17 +336,27 @@ __global__ void __launch_bounds__(256) row_integrate(IntegrateArgs a, typename N
     int next = (blockIdx.x * blockDim.x + threadIdx.x) >> 4;
     for (;;) {
         if (__any(need)) {
-            const int got = next >= 0 ? next : rows + row_get_i<0>(queue_fetch(head, need && li == 0 && rows < a.nsys));
+            const int got = next >= 0 ? next : rows + row_get_i<0>(queue_fetch(head, need && li == 0 && rows < count));
             next = -1;
             if (need) {
                 need = false;
-                active = got < a.nsys;
+                active = got < count;
                 if (active) {
-                    sid = a.index ? a.index[got] : got;
-                    yo = a.equations[(size_t)sid * N + (mine ? li : 0)];
-                    tnow = a.tnow;
-                    h = a.h0;
-                    unsolved = attempts = 0;
+                    if constexpr (TAIL) {
+                        const float *r = a.spill + (size_t)got * spill_record_words(N);
+                        yo = r[mine ? li : 0];
+                        tnow = r[N];
+                        h = r[N + 1];
+                        unsolved = __float_as_int(r[N + 2]);
+                        attempts = __float_as_int(r[N + 3]);
+                        sid = __float_as_int(r[N + 4]);
+                    } else {
+                        sid = a.index ? a.index[got] : got;
+                        yo = a.equations[(size_t)sid * N + (mine ? li : 0)];
+                        tnow = a.tnow;
+                        h = a.h0;
+                        unsolved = attempts = 0;
+                    }
                     status = WIND_STATUS_OK;
                     row_gather<N>(yo, y);
 #pragma unroll

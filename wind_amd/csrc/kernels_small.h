@@ -374,7 +374,32 @@ __device__ inline void wave_add_steps(unsigned long long *total, unsigned long l
 
 // The body of lane_integrate, shared with kernels that set other launch
 // bounds or are compiled with other floating-point contraction.
-template <class Net, int METHOD, class M, bool TRACE = false>
+// Hands the wave's unfinished systems (lanes `busy`) to the row kernel.
+template <int N>
+__device__ inline void spill_systems(const IntegrateArgs &a, const LaneSys<N> &s, int sid, bool active,
+                                     unsigned long long busy) {
+    constexpr int R = spill_record_words(N);
+    const int lane = __lane_id();
+    unsigned base = 0;
+    if (lane == 0) base = atomicAdd(reinterpret_cast<unsigned *>(a.counters + 2), (unsigned)__popcll(busy));
+    base = __shfl(base, 0);
+    if (!active) return;
+    const unsigned long long below = lane ? (~0ull >> (64 - lane)) : 0ull;
+    float r[R] = {};
+#pragma unroll
+    for (int i = 0; i < N; i++) r[i] = s.y[i];
+    r[N] = s.tnow;
+    r[N + 1] = s.h;
+    r[N + 2] = __int_as_float(s.unsolved);
+    r[N + 3] = __int_as_float(s.attempts);
+    r[N + 4] = __int_as_float(sid);
+    float4 *out = reinterpret_cast<float4 *>(a.spill + (size_t)(base + (unsigned)__popcll(busy & below)) * R);
+#pragma unroll
+    for (int v = 0; v < R / 4; v++) out[v] = make_float4(r[4 * v], r[4 * v + 1], r[4 * v + 2], r[4 * v + 3]);
+}
+
+// SPILL: with a.spill set, the wave's last systems go to the row kernel.
+template <class Net, int METHOD, class M, bool TRACE = false, bool SPILL = false>
 __device__ inline void lane_integrate_body(const IntegrateArgs &a, const typename Net::Params &p) {
     constexpr int N = Net::N;
     constexpr int NC = Net::NCONST;
@@ -382,10 +407,11 @@ __device__ inline void lane_integrate_body(const IntegrateArgs &a, const typenam
     LaneSys<N> s;
     float c[NC];
     int sid = 0;
-    bool active = false, need = true;
+    bool active = false, need = true, dry = false;
     unsigned long long steps = 0;
     for (;;) {
         const int got = queue_fetch(head, need);
+        if constexpr (SPILL) dry = dry || __any(need && got >= a.nsys);
         if (need) {
             need = false;
             active = got < a.nsys;
@@ -423,7 +449,14 @@ __device__ inline void lane_integrate_body(const IntegrateArgs &a, const typenam
                 s.status = WIND_STATUS_OK;
             }
         }
-        if (!__any(active)) break;
+        const unsigned long long busy = __ballot(active);
+        if (busy == 0ull) break;
+        if constexpr (SPILL) {
+            if (dry && __popcll(busy) <= a.spill_at) {
+                spill_systems<N>(a, s, sid, active, busy);
+                break;
+            }
+        }
         if (active && attempt<Net, METHOD, M, TRACE>(p, a, c, s, sid)) {
             float *ys = a.equations + (size_t)sid * N;
             store_state<N>(ys, s.y);
@@ -437,9 +470,9 @@ __device__ inline void lane_integrate_body(const IntegrateArgs &a, const typenam
     wave_add_steps(a.counters + 1, steps);
 }
 
-template <class Net, int METHOD, class M, bool TRACE = false>
+template <class Net, int METHOD, class M, bool TRACE = false, bool SPILL = false>
 __global__ void __launch_bounds__(256) lane_integrate(IntegrateArgs a, typename Net::Params p) {
-    lane_integrate_body<Net, METHOD, M, TRACE>(a, p);
+    lane_integrate_body<Net, METHOD, M, TRACE, SPILL>(a, p);
 }
 
 // ---------------------------------------------------------------------------

@@ -85,6 +85,17 @@ int plugin_launch_method(const IntegrateArgs &a, int mode, int kernel, int num_c
                     hipLaunchKernelGGL(k, dim3(grid), dim3(256), 0, st, a, p);
                     return hipGetLastError() == hipSuccess ? WIND_OK : WIND_ERR_DEVICE;
                 }
+                if (a.spill) {
+                    auto k = lane_integrate<Net, METHOD, MathExact, false, true>;
+                    auto kt = row_integrate<Net, METHOD, true>;
+                    int grid = 0, grid_t = 0;
+                    int rc = plugin_grid(k, 256, a.nsys, num_cu, share, grid_cap, &grid);
+                    if (!rc) rc = plugin_grid(kt, 256, a.nsys, num_cu, share, grid_cap, &grid_t);
+                    if (rc) return rc;
+                    hipLaunchKernelGGL(k, dim3(grid), dim3(256), 0, st, a, p);
+                    hipLaunchKernelGGL(kt, dim3(grid_t), dim3(256), 0, st, a, p);
+                    return hipGetLastError() == hipSuccess ? WIND_OK : WIND_ERR_DEVICE;
+                }
             }
             auto k = lane_integrate<Net, METHOD, MathExact>;
             int grid = 0;

@@ -74,6 +74,7 @@ struct CallSlot {
     Pool hint, order;  // cost hints copied from the host; start order and class counts
     Pool records;      // systems packed in start order (lane kernels of compiled-in networks)
     Pool activity;     // initial-state work estimates (start order without caller hints)
+    Pool spill;        // systems that a lane kernel hands over to the row kernel
     Pool trace;        // per-attempt trace arrays of host-pointer calls
     bool busy = false;
 };
@@ -289,6 +290,20 @@ int activity_hints(int num_cu, const wind_network *net, const IntegrateArgs &a, 
     }
 }
 
+// Lanes of a wave at which, its queue empty, its last systems go to the row
+// kernel (kernels_row.h): a lane wave costs three row waves' instructions
+// whatever its lanes do, and a row attempt takes a third of the time.  With
+// none / 8 / 16 / 24 / 32 / 48 lanes handed over, hhe6 SIE (reference
+// controller, t = 1 Myr) took 100,003 systems 475 / 225 / 160 / 154 / 167 /
+// 164 ms and 1,000,003 (t = 10^4) 634 / 415 / 384 / 374 / 385 / 410; katz96
+// 200,000 2.92 / 2.56 / 2.48 / 2.43 / 2.45 / 2.55; NR_test (N = 2) 200,000
+// 0.50 / 0.52 / 0.64 / 0.89, so only systems of five equations on do it.
+constexpr int kSpillAt = 24;
+bool spills(const wind_network *net, int mode, int nsys, int num_cu) {
+    const bool lanes = net->builtin == WIND_NET_KATZ96 || net->builtin == WIND_NET_HHE6 || net->builtin == WIND_NET_PLUGIN;
+    return mode == WIND_MODE_EXACT && lanes && net->N >= 5 && net->N <= 8 && nsys > 16 * num_cu;
+}
+
 template <class K>
 int persistent_grid(int num_cu, K kernel, int block, int nsys, int *grid, const SolverChoice &sc) {
     int per_cu = 0;
@@ -315,6 +330,15 @@ int launch_small(int num_cu, const wind_network *net, const IntegrateArgs &a, in
         int rc = persistent_grid(num_cu, k, 256, a.nsys * 16, &grid, sc);
         if (rc) return rc;
         hipLaunchKernelGGL(k, dim3(grid), dim3(256), 0, st, a, p);
+    } else if (mode == WIND_MODE_EXACT && a.spill) {
+        auto k = lane_integrate<Net, METHOD, MathExact, false, true>;
+        auto kt = row_integrate<Net, METHOD, true>;
+        int grid = 0, grid_t = 0;
+        int rc = persistent_grid(num_cu, k, 256, a.nsys, &grid, sc);
+        if (!rc) rc = persistent_grid(num_cu, kt, 256, a.nsys, &grid_t, sc);
+        if (rc) return rc;
+        hipLaunchKernelGGL(k, dim3(grid), dim3(256), 0, st, a, p);
+        hipLaunchKernelGGL(kt, dim3(grid_t), dim3(256), 0, st, a, p);
     } else if (mode == WIND_MODE_EXACT) {
         auto k = a.trace.capacity > 0 ? lane_integrate<Net, METHOD, MathExact, true>
                                       : lane_integrate<Net, METHOD, MathExact>;
@@ -917,6 +941,14 @@ int wind_integrate(const wind_network *net, float tnow, float tend, int n_integr
         if (rc) return rc;
     }
     a.records = pk.rec;
+    if (opts.kernel == WIND_KERNEL_AUTO && !opts.trace && spills(net, opts.mode, Nsystems, c.num_cu)) {
+        a.spill_at = kSpillAt;
+        // at most 32 waves per CU, each of which hands over once
+        const size_t most = std::min((size_t)Nsystems, (size_t)c.num_cu * 32 * kSpillAt);
+        rc = reserve(sl->spill, sizeof(float) * spill_record_words(Neqn) * most);
+        if (rc) return rc;
+        a.spill = (float *)sl->spill.ptr;
+    }
     std::vector<TraceCopy> trace_back;
     if (opts.trace) {
         rc = setup_trace(sl->trace, opts, Nsystems, Neqn, &a.trace, &trace_back, st);

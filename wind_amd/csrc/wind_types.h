@@ -47,10 +47,21 @@ struct IntegrateArgs {
     // bits) of system index[q], packed in queue order, so that lanes read the
     // systems they take contiguously instead of gathering them
     const float *records = nullptr;
+    // optional (lane kernels with a row-kernel tail, kernels_row.h): a wave
+    // whose queue is empty and whose unfinished systems are at most
+    // spill_at hands them over: system k's state to record k of
+    // spill_record_words(N) floats, k counted in the low word of counters[2];
+    // the row kernel that follows takes them through counters[3].
+    float *spill = nullptr;
+    int32_t spill_at = 0;
 };
 
 // Floats per packed record: state, constants and the system id, rounded up
 // to whole 32-byte sectors.
 constexpr int lane_record_words(int N, int NC) { return (N + NC + 1 + 7) / 8 * 8; }
+
+// Floats per handed-over system: state, tnow, h, refinements in a row,
+// attempts and the system id, rounded up to whole 16-byte pieces.
+constexpr int spill_record_words(int N) { return (N + 5 + 3) / 4 * 4; }
 
 }  // namespace wind
