@@ -19,7 +19,8 @@ def run(net, n, y0, c, kernel, **kw):
     y = y0.copy()
     steps, status = np.zeros(n, np.int32), np.full(n, -1, np.int32)
     kw = {"tend": 1.0, "nfix": 1, "tol": 1e-3, **kw}
-    total, _ = api.integrate(net, 0.0, kw.pop("tend"), kw.pop("nfix"), c, y, n, kw["tol"], kw.pop("tol"), kernel=kernel,
+    tol = kw.pop("tol")
+    total, _ = api.integrate(net, 0.0, kw.pop("tend"), kw.pop("nfix"), c, y, n, tol, kw.pop("rel", tol), kernel=kernel,
                              steps_out=steps, status_out=status, **kw)
     assert total == int(steps.astype(np.int64).sum())
     return y, steps, status
@@ -61,6 +62,24 @@ def test_tail_on_rows_equals_lane_kernel(name, n, method, controller):
     kw = dict(kw, method=method, controller=controller, max_attempts=60)
     a, b = (run(net, n, y0, c, k, **kw) for k in (api.KERNEL_LANE, api.KERNEL_AUTO))
     assert same(a[0], b[0]) and np.array_equal(a[1], b[1]) and np.array_equal(a[2], b[2])
+
+
+@pytest.mark.parametrize("N", [1, 2, 7, 8, 9, 16, 31, 33, 40, 41, 55, 57, 63, 64])
+@pytest.mark.parametrize("controller", [api.CTRL_REFERENCE, api.CTRL_ADAPTIVE])
+def test_register_kernel_equals_oracle(N, controller):
+    """Mass-action networks with the matrix in registers, at the edges of the sizes it is built for; a state that
+    overflows, whose infinities pass through the elimination."""
+    n = 5
+    rx, k = W.mass_action_network(N, 300 + N, R=max(4 * N, 3) if N != 9 else 0)
+    y0, sc = W.mass_action_systems(n, N, 5, W.MIXED_SCALE_RANGE)
+    y0[N:2 * N] *= np.float32(1e30)
+    y0[2 * N] = np.inf
+    yr = y0.copy()
+    _, sr, tr = O.gold_integrate(O.SIE, O.mass_action(N, rx, k), 0.0, 1e5, 1, sc, yr, n, 1e-6, 1e-4, const_stride=1,
+                                 max_attempts=60, controller=controller)
+    y, steps, status = run(api.Network.mass_action(N, rx, k), n, y0, sc, api.KERNEL_AUTO, tend=1e5, tol=1e-6,
+                           rel=1e-4, controller=controller, max_attempts=60)
+    assert same(y, yr) and np.array_equal(steps, sr) and np.array_equal(status, tr)
 
 
 def test_row_kernel_strides_hints_and_non_finite_states():

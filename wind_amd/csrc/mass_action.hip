@@ -9,6 +9,7 @@
 
 #include "kernels_dense.h"
 #include "kernels_dense_reg.h"
+#include "kernels_ma_wave.h"
 #include "kernels_mass_action.h"
 #include "wind_internal.h"
 
@@ -34,6 +35,34 @@ struct Scratch {
 Scratch g_scratch;  // per-process matrix scratch; callers hold the context lock
 
 }  // namespace
+
+// The exact register kernel (ma_wave_integrate): N <= 64, its LDS within the
+// default limit.
+static bool ma_wave_fits(int N, int R) {
+    return N <= 64 && sizeof(float) * ma_wave_lds_floats((N + 7) & ~7, R) <= 65536 - 64;
+}
+
+// Deals elements (their terms' words) to `threads` streams, most terms first
+// to the least-loaded thread; streams padded with zero words to the longest,
+// rounded up to `batch`, and interleaved: word j of thread t at
+// [j * threads + t].
+static std::vector<int32_t> deal_streams(std::vector<std::vector<uint32_t>> &items, int threads, int batch, int *len) {
+    std::stable_sort(items.begin(), items.end(), [](const auto &p1, const auto &p2) { return p1.size() > p2.size(); });
+    std::vector<std::vector<uint32_t>> per(threads);
+    for (auto &it : items) {
+        size_t th = 0;
+        for (size_t u = 1; u < per.size(); u++)
+            if (per[u].size() < per[th].size()) th = u;
+        per[th].insert(per[th].end(), it.begin(), it.end());
+    }
+    size_t n = batch;
+    for (auto &p : per) n = std::max(n, (p.size() + batch - 1) / batch * batch);
+    std::vector<int32_t> out(n * threads, 0);
+    for (int th = 0; th < threads; th++)
+        for (size_t j = 0; j < per[th].size(); j++) out[j * threads + th] = (int32_t)per[th][j];
+    *len = (int)n;
+    return out;
+}
 
 int mass_action_build(wind_network *n, int N, int R, const int32_t *rx, const float *k) {
     n->rx.assign(rx, rx + 4 * (size_t)R);
@@ -80,14 +109,12 @@ int mass_action_build(wind_network *n, int N, int R, const int32_t *rx, const fl
     // the order dense_eval applies them (the row's reactions in sweep order,
     // the reaction's first reactant before its second), summed from 1 on the
     // diagonal; the elements are dealt to the workgroup's 256
-    // threads, most terms first to the least-loaded thread, and a thread's
-    // stream is its elements' terms, one word each:
+    // threads (deal_streams), and a thread's stream is its elements' terms,
+    // one word each:
     //   (LDS float index of the term's h dJ value) << 16 | (buffer offset of
     //   the element) << 3 | (element on the diagonal) << 2 | (element's last
     //   term) << 1 | (reactant row: the term adds)
-    // Streams are padded with zero words (which store nothing) to the
-    // longest, rounded up to kDenseRegBatch words, and interleaved: word j
-    // of thread t at sc_ent[j * 256 + t].
+    // The padding's zero words store nothing.
     const int NT = (N + 15) / 16;
     std::vector<int32_t> sc_ent;
     std::vector<uint32_t> sc_tile;
@@ -125,7 +152,7 @@ int mass_action_build(wind_network *n, int N, int R, const int32_t *rx, const fl
         // (+1: an owner lane reads one place past its elements, unused)
         sc_cap = (int)((nnz + 1 + 3) & ~3u);
         ok = ok && sc_cap < 8192;
-        std::vector<std::pair<int, std::vector<uint32_t>>> items;  // (count, words)
+        std::vector<std::vector<uint32_t>> items;
         for (auto &kv : elem) {
             int tl, q;
             slot(kv.first.first, kv.first.second, &tl, &q);
@@ -133,28 +160,39 @@ int mass_action_build(wind_network *n, int N, int R, const int32_t *rx, const fl
             std::vector<uint32_t> w = kv.second;
             for (auto &x : w) x |= dest << 3;
             w.back() |= 2u;
-            items.push_back({(int)w.size(), std::move(w)});
+            items.push_back(std::move(w));
         }
-        std::stable_sort(items.begin(), items.end(),
-                         [](const auto &p1, const auto &p2) { return p1.first > p2.first; });
-        std::vector<std::vector<uint32_t>> per(256);
-        for (auto &it : items) {
-            size_t th = 0;
-            for (size_t u = 1; u < per.size(); u++)
-                if (per[u].size() < per[th].size()) th = u;
-            per[th].insert(per[th].end(), it.second.begin(), it.second.end());
-        }
-        size_t len = kDenseRegBatch;
-        for (auto &p : per) len = std::max(len, (p.size() + kDenseRegBatch - 1) / kDenseRegBatch * kDenseRegBatch);
-        sc_ent.assign(len * 256, 0);
-        for (int th = 0; th < 256; th++)
-            for (size_t j = 0; j < per[th].size(); j++) sc_ent[j * 256 + th] = (int32_t)per[th][j];
-        sc_len = (int)len;
+        sc_ent = deal_streams(items, 256, kDenseRegBatch, &sc_len);
         if (!ok) {
             sc_ent.clear();
             sc_tile.clear();
             sc_len = sc_cap = 0;
         }
+    }
+    // Assembly of the exact register kernel (ma_wave_integrate): f's and the
+    // Jacobian's elements, each its terms in sweep order, one word per term:
+    //   (LDS float index of the term's w, da or db) << 16 | (LDS float index
+    //   of the element) << 3 | (element's last term) << 1 | (subtracted)
+    std::vector<int32_t> ex_ent;
+    int ex_len = 0;
+    if (ma_wave_fits(N, R)) {
+        const int NP = (N + 7) & ~7;
+        const uint32_t f0 = NP * NP + 3 * NP, w0 = f0 + NP;
+        std::vector<std::vector<uint32_t>> items;
+        for (int i = 0; i < N; i++) {
+            std::vector<uint32_t> w;
+            for (int32_t e : flist[i]) w.push_back((w0 + (uint32_t)(e >> 1)) << 16 | (f0 + i) << 3 | (uint32_t)(e & 1));
+            if (!w.empty()) items.push_back(std::move(w));
+        }
+        for (auto &kv : jlist) {
+            const uint32_t dest = (uint32_t)(kv.first / N * NP + kv.first % N);
+            std::vector<uint32_t> w;
+            for (int32_t e : kv.second)
+                w.push_back((w0 + (uint32_t)(R * ((e & 2) ? 2 : 1) + (e >> 2))) << 16 | dest << 3 | (uint32_t)(e & 1));
+            items.push_back(std::move(w));
+        }
+        for (auto &w : items) w.back() |= 2u;
+        ex_ent = deal_streams(items, 128, kMaWaveBatch, &ex_len);
     }
     MassActionDevice &d = n->ma;
     d.N = N;
@@ -171,6 +209,8 @@ int mass_action_build(wind_network *n, int N, int R, const int32_t *rx, const fl
     if (!rc) rc = upload((void **)&d.r_z, r_z.data(), sizeof(int32_t) * r_z.size());
     if (!rc && !sc_ent.empty()) rc = upload((void **)&d.sc_ent, sc_ent.data(), sizeof(int32_t) * sc_ent.size());
     if (!rc && !sc_ent.empty()) rc = upload((void **)&d.sc_tile, sc_tile.data(), sizeof(uint32_t) * sc_tile.size());
+    if (!rc && !ex_ent.empty()) rc = upload((void **)&d.ex_ent, ex_ent.data(), sizeof(int32_t) * ex_ent.size());
+    d.ex_len = ex_len;
     d.sc_len = sc_len;
     d.sc_cap = sc_cap;
     return rc;
@@ -178,7 +218,7 @@ int mass_action_build(wind_network *n, int N, int R, const int32_t *rx, const fl
 
 void mass_action_release(wind_network *n) {
     MassActionDevice &d = n->ma;
-    void *ptrs[] = {d.rx, d.k, d.f_ptr, d.f_ent, d.j_pos, d.j_ptr, d.j_ent, d.r_ptr, d.r_z, d.sc_ent, d.sc_tile};
+    void *ptrs[] = {d.rx, d.k, d.f_ptr, d.f_ent, d.j_pos, d.j_ptr, d.j_ent, d.r_ptr, d.r_z, d.sc_ent, d.sc_tile, d.ex_ent};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     d = MassActionDevice();
@@ -264,6 +304,18 @@ size_t scratch_bytes(const MassActionDevice &d, const BlockShape &s) {
     return s.in_lds ? 0 : sizeof(float) * 2 * (size_t)d.N * d.N * s.grid;
 }
 
+template <int NP>
+int launch_ma_wave(int num_cu, const MassActionDevice &d, const IntegrateArgs &a, const SolverChoice &sc, hipStream_t st) {
+    const size_t lds = sizeof(float) * ma_wave_lds_floats(NP, d.R);
+    int per_cu = 0;
+    hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, ma_wave_integrate<NP>, 128, lds);
+    if (e != hipSuccess) return wind_fail(WIND_ERR_DEVICE, hipGetErrorString(e));
+    hipLaunchKernelGGL(ma_wave_integrate<NP>, dim3(scaled_grid(num_cu, per_cu, sc, a.nsys)), dim3(128), lds, st, a, d);
+    e = hipGetLastError();
+    if (e != hipSuccess) return wind_fail(WIND_ERR_DEVICE, hipGetErrorString(e));
+    return WIND_OK;
+}
+
 }  // namespace
 
 template <int METHOD>
@@ -323,6 +375,18 @@ int launch_mass_action(int num_cu, const wind_network *net, const IntegrateArgs 
     if (a.trace.capacity > 0)
         return wind_fail(WIND_ERR_UNSUPPORTED, "trace: mass-action networks are traced by the dense solver "
                                                "(fast mode, N <= 176) only");
+    if (METHOD == WIND_SIE && !fast && kernel == WIND_KERNEL_AUTO && d.ex_ent) {
+        switch ((N + 7) / 8) {
+        case 1: return launch_ma_wave<8>(num_cu, d, a, sc, st);
+        case 2: return launch_ma_wave<16>(num_cu, d, a, sc, st);
+        case 3: return launch_ma_wave<24>(num_cu, d, a, sc, st);
+        case 4: return launch_ma_wave<32>(num_cu, d, a, sc, st);
+        case 5: return launch_ma_wave<40>(num_cu, d, a, sc, st);
+        case 6: return launch_ma_wave<48>(num_cu, d, a, sc, st);
+        case 7: return launch_ma_wave<56>(num_cu, d, a, sc, st);
+        default: return launch_ma_wave<64>(num_cu, d, a, sc, st);
+        }
+    }
     BlockShape s;
     int rc = block_shape<METHOD>(num_cu, d, plan, fast, sc, a.nsys, &s);
     if (rc) return rc;
