@@ -13,11 +13,18 @@
 // Per pass (step-doubling sub-step) of an attempt:
 // * assembly: the per-reaction rate terms and f as in the LDS solver
 //   (kernels_dense.h, dense_eval, same order, so f and every matrix element
-//   round identically); the matrix elements with Jacobian terms are summed
-//   into a compact LDS buffer (the elements dealt to all 256 threads on the
-//   host, each element its terms in sweep order), and the owner lanes of
-//   the tiles read them into registers through per-lane offset and mask
-//   words (1 on the diagonal, 0 elsewhere where absent);
+//   round identically); f and the matrix elements with Jacobian terms are
+//   summed into a compact LDS buffer (dealt to all 256 threads on the host,
+//   each element its terms in sweep order, one branch-free stream of term
+//   words per thread), and the owner lanes of the tiles read them into
+//   registers through per-lane offset and mask words (1 on the diagonal, 0
+//   elsewhere where absent), loaded ahead while the tiles' registers are
+//   free.  Against f summed from lists of its own by the first N threads,
+//   words loaded a tile row at a time and tile addresses and conditions kept
+//   in (spilled) registers across the phases, a sub-step went from 21.7 to
+//   19.1 us per CU at N = 157, 3.37 to 3.30 at N = 64 and 1.84 to 1.72 at
+//   N = 32 with the CU full, and from 51.5 / 12.4 / 7.4 to 46.8 / 10.5 /
+//   5.7 us for a system alone on it;
 // * block LU without pivoting, A = [I 0; A21 G I][A11 A12; 0 A22 - A21 G A12],
 //   G = A11^-1, per 16-column panel k, with two barriers:
 //     B: W_kj = G_k A_kj for the row panel (G_k from LDS, A_kj in the
@@ -52,7 +59,7 @@ namespace wind {
 
 // Assembly stream words a thread loads at a time (streams are padded to a
 // multiple of it).
-constexpr int kDenseRegBatch = 4;
+constexpr int kDenseRegBatch = 8;
 
 // Row-panel tiles a wave holds at a time in the trailing update: two from
 // eight tiles per dimension (N = 157: 2.26 k -> 2.31 k systems/s; N = 64,
@@ -62,10 +69,11 @@ constexpr int kDenseRegGW = NT >= 8 ? 2 : 1;
 
 // LDS layout of the register-resident solver (offsets in floats, 16-byte
 // aligned): per-system vectors, per-reaction rate terms, reactant indices
-// and rate constants, and a work area shared by the compact element buffer
-// of the assembly (cap floats) and the factorisation's panel buffers.  The term lists stay in global memory.
+// and rate constants, and a work area shared by the assembly's compact
+// element buffer (cap floats) with f behind it, and the factorisation's panel
+// buffers.  The term lists stay in global memory.
 struct DenseRegOffsets {
-    int y, yw, y1, f, r, w, hda, hdb, k, ab, fptr, work, total;
+    int y, yw, y1, r, w, hda, hdb, k, ab, work, total;
 };
 
 __host__ __device__ inline DenseRegOffsets dense_reg_offsets(int NT, int R, int WGS, int cap) {
@@ -79,8 +87,6 @@ __host__ __device__ inline DenseRegOffsets dense_reg_offsets(int NT, int R, int 
     p = up(p + NP);
     o.y1 = p;
     p = up(p + NP);
-    o.f = p;
-    p = up(p + NP);
     o.r = p;
     p = up(p + NP);
     o.w = p;
@@ -93,11 +99,9 @@ __host__ __device__ inline DenseRegOffsets dense_reg_offsets(int NT, int R, int 
     if (WGS == 3) p = up(p + R);  // rate constants in LDS
     o.ab = p;
     p = up(p + 2 * R);
-    o.fptr = p;
-    p = up(p + NP + 1);
     o.work = p;
-    const int lu = (2 * NT + 1) * 256;
-    p = up(p + (cap > lu ? cap : lu));
+    const int lu = (2 * NT + 1) * 256, el = cap + NP;
+    p = up(p + (el > lu ? el : lu));
     o.total = p;
     return o;
 }
@@ -164,41 +168,44 @@ __device__ inline void tile_matvec_store(const f32x4 &m, float v, float *dst, in
     }
 }
 
+__device__ inline float uniform(float v) {
+    return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
+}
+
 // TRACE: per-attempt trace and replay through a.trace, as in the other
 // kernels.
 template <int NT, int WGS, bool TRACE = false>
 __global__ void __launch_bounds__(256, WGS) ma_dense_reg_integrate(IntegrateArgs a, MassActionDevice net) {
-    constexpr int NP = 16 * NT, NL = (NT + 1) / 2;
+    constexpr int WR = 2, WC = 2;  // the waves' grid
+    constexpr int NP = 16 * NT, T = 64 * WR * WC, NR = (NT + WR - 1) / WR, NC = (NT + WC - 1) / WC;
     extern __shared__ float lds[];
     const int N = net.N, R = net.R, t = threadIdx.x;
     const int lane = t & 63;
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
-    const int wi = wave >> 1, wj = wave & 1;
+    const int wi = wave / WC, wj = wave % WC;
     const int lr = lane & 15, g = lane >> 4;
     const DenseRegOffsets o = dense_reg_offsets(NT, R, WGS, net.sc_cap);
-    float *y = lds + o.y, *yw = lds + o.yw, *y1 = lds + o.y1, *f = lds + o.f, *rv = lds + o.r;
+    float *y = lds + o.y, *yw = lds + o.yw, *y1 = lds + o.y1, *rv = lds + o.r;
     float *w = lds + o.w, *hda = lds + o.hda, *hdb = lds + o.hdb, *kk = lds + o.k;
     int2 *ab = reinterpret_cast<int2 *>(lds + o.ab);
-    int *fptr = reinterpret_cast<int *>(lds + o.fptr);
-    const int *__restrict__ fent = net.f_ent;
     const int *__restrict__ scent = net.sc_ent;
     const unsigned *__restrict__ sctile = net.sc_tile;
-    float *work = lds + o.work;
+    float *work = lds + o.work, *f = work + net.sc_cap;
     float *Gbuf = work, *Cbuf = work + 256, *Wbuf = work + 256 * (NT + 1);
-    // Per-lane bases of this wave's tiles (tile row i = 2 ta + wi, column
-    // j = 2 tb + wj): the accesses below add compile-time offsets.
-    float *const cA = Cbuf + wi * 256 + lr * 16 + 4 * g;  // A-operand reads of Cbuf tile i: + ta * 512
-    float *const cS = Cbuf + wi * 256 + 64 * g + lr;      // stores to Cbuf tile i: + ta * 512 + q * 16
-    float *const wB = Wbuf + wj * 256 + lane * 4;          // Wbuf tile j: + tb * 512
-    float *const rI = rv + 16 * wi;                        // rows of tile row i: + 32 * ta
-    for (int r = t; r < R; r += 256) {
+    // Per-lane bases of this wave's tiles (tile row i = WR ta + wi, column
+    // j = WC tb + wj): the accesses below add compile-time offsets.
+    constexpr int RS = 256 * WR, CS = 256 * WC;
+    float *const cA = Cbuf + wi * 256 + lr * 16 + 4 * g;  // A-operand reads of Cbuf tile i: + ta * RS
+    float *const cS = Cbuf + wi * 256 + 64 * g + lr;      // stores to Cbuf tile i: + ta * RS + q * 16
+    float *const wB = Wbuf + wj * 256 + lane * 4;          // Wbuf tile j: + tb * CS
+    float *const rI = rv + 16 * wi;                        // rows of tile row i: + 16 * WR * ta
+    for (int r = t; r < R; r += T) {
         ab[r] = make_int2(net.rx[4 * r], net.rx[4 * r + 1]);
         if (WGS == 3) kk[r] = net.k[r];
     }
-    for (int i = t; i <= N; i += 256) fptr[i] = net.f_ptr[i];
     __shared__ int s_flag, s_sid;
-    __shared__ double s_err[4];
-    f32x4 M[NL][NL];
+    __shared__ double s_err[WR * WC];
+    f32x4 M[NR][NC];
     unsigned long long steps = 0;
     unsigned int *head = reinterpret_cast<unsigned int *>(a.counters);
     __syncthreads();
@@ -207,19 +214,39 @@ __global__ void __launch_bounds__(256, WGS) ma_dense_reg_integrate(IntegrateArgs
     // barrier).
     auto assemble = [&](const float *yv, float scale, float hs) __attribute__((always_inline)) {
         constexpr int B = kDenseRegBatch;
+        // (the wave's place made opaque, so that the compiler derives the
+        // tiles' conditions and offsets here instead of keeping them all)
+        int wv = wave;
+        asm volatile("" : "+s"(wv));
+        const int wi = wv / WC, wj = wv % WC;
         // the tiles' old values are dead (every tile is stored again below,
         // under conditions the compiler cannot prove cover all of them)
 #pragma unroll
-        for (int ta = 0; ta < NL; ta++)
+        for (int ta = 0; ta < NR; ta++)
 #pragma unroll
-            for (int tb = 0; tb < NL; tb++) M[ta][tb] = __builtin_nondeterministic_value(M[ta][tb]);
+            for (int tb = 0; tb < NC; tb++) M[ta][tb] = __builtin_nondeterministic_value(M[ta][tb]);
+        // This lane's word of each tile: offset << 4 | the mask of its q
+        // present; loaded here, the tiles' registers being free, and used
+        // after the elements are summed.  (An opaque offset per pass, so that
+        // the compiler does not keep them across passes.)
+        int tsel = 0;
+        asm volatile("" : "+s"(tsel));
+        const unsigned *tpass = sctile + tsel + lane;
+        unsigned wt[NR][NC];
+#pragma unroll
+        for (int ta = 0; ta < NR; ta++)
+#pragma unroll
+            for (int tb = 0; tb < NC; tb++) {
+                const int i = WR * ta + wi, jb = WC * tb + wj;
+                wt[ta][tb] = (i < NT && jb < NT) ? tpass[(i * NT + jb) * 64] : 0u;
+            }
         // the first words of the term stream, loaded while the rate terms
         // and f are formed
         int en[B];
         const int *sp = scent + t;
 #pragma unroll
-        for (int u = 0; u < B; u++) en[u] = sp[u * 256];
-        for (int r = t; r < R; r += 256) {
+        for (int u = 0; u < B; u++) en[u] = sp[u * T];
+        for (int r = t; r < R; r += T) {
             const int2 x = ab[r];
             const float ks = (WGS == 3 ? kk[r] : net.k[r]) * scale;
             const float ya = yv[x.x], yb = yv[x.y];
@@ -227,80 +254,51 @@ __global__ void __launch_bounds__(256, WGS) ma_dense_reg_integrate(IntegrateArgs
             hda[r] = hs * (ks * yb);
             hdb[r] = hs * (ks * ya);
         }
+        if (t < NP) f[t] = 0.0f;  // species without reactions, and the padding
         __syncthreads();
-        // f: the row's reaction list in order, its loads issued 8 at a time
-        if (t < NP) {
-            float acc = 0.0f;
-            if (t < N) {
-                const int e1 = fptr[t + 1];
-                for (int e = fptr[t]; e < e1; e += 8) {
-                    int fe[8];
-                    float wv[8];
-#pragma unroll
-                    for (int u = 0; u < 8; u++) fe[u] = e + u < e1 ? fent[e + u] : 0;
-#pragma unroll
-                    for (int u = 0; u < 8; u++) wv[u] = w[fe[u] >> 1];
-#pragma unroll
-                    for (int u = 0; u < 8; u++)
-                        if (e + u < e1) acc = (fe[u] & 1) ? acc - wv[u] : acc + wv[u];
-                }
-            }
-            f[t] = acc;
-        }
-        // The matrix's non-zero elements through a compact buffer: each
+        // f and the matrix's non-zero elements through a compact buffer: each
         // thread walks its term stream (the elements dealt to the 256
         // threads on the host, interleaved so that a batch of words is one
         // coalesced load per word); an element is its terms summed in order
-        // in a register (from 1 on the diagonal), stored once at its offset.
+        // in a register (from 1 on the diagonal), stored at its offset.
         // The owner lane of each tile element then reads it from the buffer
         // through its per-lane offset and mask word (1 on the diagonal, 0
         // elsewhere where the element is absent).
         {
             const int len = net.sc_len;
             float acc = 0.0f;
-            bool start = true;
             for (int j = 0;;) {
                 float v[B];
-#pragma unroll
-                for (int u = 0; u < B; u++) v[u] = lds[(unsigned)en[u] >> 16];
+                int e[B];
 #pragma unroll
                 for (int u = 0; u < B; u++) {
-                    // zero words (padding) load and store nothing that matters
-                    const int e = en[u];
-                    acc = start ? ((e & 4) ? 1.0f : 0.0f) : acc;
-                    acc = (e & 1) ? acc + v[u] : acc - v[u];
-                    start = (e & 2) != 0;
-                    if (start) work[(e >> 3) & 8191] = acc;
+                    e[u] = en[u];
+                    v[u] = lds[(unsigned)e[u] >> 16];
                 }
                 j += B;
-                if (j >= len) break;
+                if (j < len)
 #pragma unroll
-                for (int u = 0; u < B; u++) en[u] = sp[(j + u) * 256];
+                    for (int u = 0; u < B; u++) en[u] = sp[(j + u) * T];
+#pragma unroll
+                for (int u = 0; u < B; u++) {
+                    // the running sum is stored at every term (the element's
+                    // last store stays); padding stores where nothing reads
+                    acc = (e[u] & 2) ? ((e[u] & 4) ? 1.0f : 0.0f) : acc;
+                    acc += __uint_as_float(__float_as_uint(v[u]) ^ ((unsigned)e[u] << 31));
+                    work[(e[u] >> 3) & 8191] = acc;
+                }
+                if (j >= len) break;
             }
         }
         __syncthreads();
-        // (an opaque offset per pass, so that the compiler does not keep
-        // every tile's words live across passes)
-        int tsel = 0;
-        asm volatile("" : "+s"(tsel));
-        const unsigned *tpass = sctile + tsel;
 #pragma unroll
-        for (int ta = 0; ta < NL; ta++) {
-            const int i = 2 * ta + wi;
-            // this lane's word of each tile in the row: offset << 4 | the
-            // mask of its q present (a row of tiles at a time, so that few
-            // loads are in flight beside the tiles already filled)
-            unsigned wrow[NL];
+        for (int ta = 0; ta < NR; ta++) {
+            const int i = WR * ta + wi;
 #pragma unroll
-            for (int tb = 0; tb < NL; tb++) {
-                const int jb = 2 * tb + wj;
-                wrow[tb] = (i < NT && jb < NT) ? tpass[(i * NT + jb) * 64 + lane] : 0u;
-            }
-#pragma unroll
-            for (int tb = 0; tb < NL; tb++) {
-                const int jb = 2 * tb + wj;
+            for (int tb = 0; tb < NC; tb++) {
+                const int jb = WC * tb + wj;
                 if (i >= NT || jb >= NT) continue;
-                const unsigned wd = wrow[tb];
+                const unsigned wd = wt[ta][tb];
                 unsigned p = wd >> 4;
                 f32x4 m;
 #pragma unroll
@@ -317,7 +315,7 @@ __global__ void __launch_bounds__(256, WGS) ma_dense_reg_integrate(IntegrateArgs
     };
 
     // Diagonal tile (k, k) of its owner: invert, publish G_k, c_k = G_k r_k.
-    auto diag_step = [&](f32x4 &m, int k) __attribute__((always_inline)) {
+    auto diag_step = [&](f32x4 m, int k) __attribute__((always_inline)) {
         tile_invert_acc(m, lane);
 #pragma unroll
         for (int q = 0; q < 4; q++) Gbuf[(4 * g + q) * 16 + lr] = m[q];
@@ -332,82 +330,91 @@ __global__ void __launch_bounds__(256, WGS) ma_dense_reg_integrate(IntegrateArgs
     // cores, the owner of the next diagonal tile updating it first, inverting
     // it and forming c_{k+1} = G_{k+1} r_{k+1}.  Leaves c in rv.
     auto factor = [&]() __attribute__((always_inline)) {
+        int wv = wave;
+        asm volatile("" : "+s"(wv));
+        const int wi = wv / WC, wj = wv % WC;
         if (t < NP) rv[t] = f[t];
         __syncthreads();
         if (wave == 0) diag_step(M[0][0], 0);
         __syncthreads();
         for (int k = 0; k < NT - 1; k++) {
-            if (wi == (k & 1)) {
+            if (wi == k % WR) {
                 const f32x4 gr = *reinterpret_cast<const f32x4 *>(Gbuf + lr * 16 + 4 * g);
 #pragma unroll
-                for (int ta = 0; ta < NL; ta++) {
-                    if (2 * ta + wi != k) continue;
+                for (int ta = 0; ta < NR; ta++) {
+                    if (WR * ta + wi != k) continue;
 #pragma unroll
-                    for (int tb = 0; tb < NL; tb++) {
-                        const int j = 2 * tb + wj;
+                    for (int tb = 0; tb < NC; tb++) {
+                        const int j = WC * tb + wj;
                         if (j <= k || j >= NT) continue;
                         f32x4 z = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
                         for (int q = 0; q < 4; q++) z = __builtin_amdgcn_mfma_f32_16x16x4f32(gr[q], M[ta][tb][q], z, 0, 0, 0);
                         M[ta][tb] = z;
-                        *reinterpret_cast<f32x4 *>(wB + tb * 512) = z;
+                        *reinterpret_cast<f32x4 *>(wB + tb * CS) = z;
                     }
                 }
             }
-            if (wj == (k & 1)) {
+            if (wj == k % WC) {
                 const float ck = rv[16 * k + lr];
 #pragma unroll
-                for (int tb = 0; tb < NL; tb++) {
-                    if (2 * tb + wj != k) continue;
+                for (int tb = 0; tb < NC; tb++) {
+                    if (WC * tb + wj != k) continue;
 #pragma unroll
-                    for (int ta = 0; ta < NL; ta++) {
-                        const int i = 2 * ta + wi;
+                    for (int ta = 0; ta < NR; ta++) {
+                        const int i = WR * ta + wi;
                         if (i <= k || i >= NT) continue;
                         const f32x4 m = M[ta][tb];
 #pragma unroll
-                        for (int q = 0; q < 4; q++) cS[ta * 512 + q * 16] = -m[q];
-                        tile_matvec_store<true>(m, ck, rI + 32 * ta, lane);
+                        for (int q = 0; q < 4; q++) cS[ta * RS + q * 16] = -m[q];
+                        tile_matvec_store<true>(m, ck, rI + 16 * WR * ta, lane);
                     }
                 }
             }
             __syncthreads();
             const int k1 = k + 1;
-            if (wi == (k1 & 1) && wj == (k1 & 1)) {
+            if (wi == k1 % WR && wj == k1 % WC) {
+                // in a copy, so that the inversion's code exists once; the
+                // tile itself is not read again
+                f32x4 d = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-                for (int ta = 0; ta < NL; ta++) {
-                    if (2 * ta + wi != k1) continue;
-                    const f32x4 xa = *reinterpret_cast<const f32x4 *>(cA + ta * 512);
-                    const f32x4 wv = *reinterpret_cast<const f32x4 *>(wB + ta * 512);
+                for (int ta = 0; ta < NR; ta++)
 #pragma unroll
-                    for (int q = 0; q < 4; q++)
-                        M[ta][ta] = __builtin_amdgcn_mfma_f32_16x16x4f32(xa[q], wv[q], M[ta][ta], 0, 0, 0);
-                    diag_step(M[ta][ta], k1);
-                }
+                    for (int tb = 0; tb < NC; tb++) {
+                        if (WR * ta >= WC * (tb + 1) || WC * tb >= WR * (ta + 1)) continue;  // no diagonal tile
+                        if (WR * ta + wi != k1 || WC * tb + wj != k1) continue;
+                        const f32x4 xa = *reinterpret_cast<const f32x4 *>(cA + ta * RS);
+                        const f32x4 wv = *reinterpret_cast<const f32x4 *>(wB + tb * CS);
+                        d = M[ta][tb];
+#pragma unroll
+                        for (int q = 0; q < 4; q++) d = __builtin_amdgcn_mfma_f32_16x16x4f32(xa[q], wv[q], d, 0, 0, 0);
+                    }
+                diag_step(d, k1);
             }
             // GW row-panel tiles W_kj held at a time, each A_ik read once
             // per group (fewer LDS reads than one W read per tile update)
 #pragma unroll
-            for (int tb0 = 0; tb0 < NL; tb0 += kDenseRegGW<NT>) {
+            for (int tb0 = 0; tb0 < NC; tb0 += kDenseRegGW<NT>) {
                 constexpr int GW = kDenseRegGW<NT>;
                 f32x4 wv[GW];
                 bool vv[GW], any = false;
 #pragma unroll
                 for (int u = 0; u < GW; u++) {
-                    const int j = 2 * (tb0 + u) + wj;
-                    vv[u] = tb0 + u < NL && j > k && j < NT;
+                    const int j = WC * (tb0 + u) + wj;
+                    vv[u] = tb0 + u < NC && j > k && j < NT;
                     any = any || vv[u];
-                    wv[u] = vv[u] ? *reinterpret_cast<const f32x4 *>(wB + (tb0 + u) * 512) : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                    wv[u] = vv[u] ? *reinterpret_cast<const f32x4 *>(wB + (tb0 + u) * CS) : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
                 }
                 if (!any) continue;
 #pragma unroll
-                for (int ta = 0; ta < NL; ta++) {
-                    const int i = 2 * ta + wi;
+                for (int ta = 0; ta < NR; ta++) {
+                    const int i = WR * ta + wi;
                     if (i <= k || i >= NT) continue;
-                    const f32x4 xa = *reinterpret_cast<const f32x4 *>(cA + ta * 512);
+                    const f32x4 xa = *reinterpret_cast<const f32x4 *>(cA + ta * RS);
 #pragma unroll
                     for (int u = 0; u < GW; u++) {
-                        const int tb = tb0 + u < NL ? tb0 + u : NL - 1;
-                        const int j = 2 * (tb0 + u) + wj;
+                        const int tb = tb0 + u < NC ? tb0 + u : NC - 1;
+                        const int j = WC * (tb0 + u) + wj;
                         if (!vv[u] || (i == k1 && j == k1)) continue;
 #pragma unroll
                         for (int q = 0; q < 4; q++)
@@ -421,17 +428,20 @@ __global__ void __launch_bounds__(256, WGS) ma_dense_reg_integrate(IntegrateArgs
 
     // Backward sweep by columns: x_k = c_k, then c_i -= W_ik x_k above.
     auto back = [&]() __attribute__((always_inline)) {
+        int wv = wave;
+        asm volatile("" : "+s"(wv));
+        const int wi = wv / WC, wj = wv % WC;
         for (int k = NT - 1; k >= 1; k--) {
-            if (wj == (k & 1)) {
+            if (wj == k % WC) {
                 const float xk = rv[16 * k + lr];
 #pragma unroll
-                for (int tb = 0; tb < NL; tb++) {
-                    if (2 * tb + wj != k) continue;
+                for (int tb = 0; tb < NC; tb++) {
+                    if (WC * tb + wj != k) continue;
 #pragma unroll
-                    for (int ta = 0; ta < NL; ta++) {
-                        const int i = 2 * ta + wi;
+                    for (int ta = 0; ta < NR; ta++) {
+                        const int i = WR * ta + wi;
                         if (i >= k) continue;
-                        tile_matvec_store<true>(M[ta][tb], xk, rI + 32 * ta, lane);
+                        tile_matvec_store<true>(M[ta][tb], xk, rI + 16 * WR * ta, lane);
                     }
                 }
             }
@@ -445,9 +455,9 @@ __global__ void __launch_bounds__(256, WGS) ma_dense_reg_integrate(IntegrateArgs
             s_sid = q < (unsigned)a.nsys ? (a.index ? a.index[q] : (int)q) : a.nsys;
         }
         __syncthreads();
-        const int sid = s_sid;
+        const int sid = __builtin_amdgcn_readfirstlane(s_sid);
         if (sid >= a.nsys) break;
-        for (int i = t; i < N; i += 256) y[i] = a.equations[(size_t)sid * N + i];
+        for (int i = t; i < N; i += T) y[i] = a.equations[(size_t)sid * N + i];
         const float scale = a.constants[(size_t)sid * a.const_stride];
         __syncthreads();
         float tnow = a.tnow, h = a.h0;
@@ -457,7 +467,7 @@ __global__ void __launch_bounds__(256, WGS) ma_dense_reg_integrate(IntegrateArgs
         while (replay ? attempts < rcount : tnow < a.tend) {
             const size_t slot = TRACE ? (size_t)sid * a.trace.capacity + attempts : 0;
             if (replay && a.trace.y_start) {
-                for (int i = t; i < N; i += 256) y[i] = a.trace.y_start[slot * N + i];
+                for (int i = t; i < N; i += T) y[i] = a.trace.y_start[slot * N + i];
                 __syncthreads();
             }
             const float hh = replay ? a.trace.h[slot] : fminf(a.tend - tnow, h);
@@ -466,16 +476,16 @@ __global__ void __launch_bounds__(256, WGS) ma_dense_reg_integrate(IntegrateArgs
             for (int pass = 0; pass < 3; pass++) {
                 const float hs = pass == 0 ? hs_full : hs_half;
                 if (pass != 2) {
-                    for (int i = t; i < N; i += 256) yw[i] = y[i];
+                    for (int i = t; i < N; i += T) yw[i] = y[i];
                     __syncthreads();
                 }
                 assemble(yw, scale, hs);
                 factor();
                 back();
-                for (int i = t; i < N; i += 256) yw[i] = fmaf(hs, rv[i], yw[i]);
+                for (int i = t; i < N; i += T) yw[i] = fmaf(hs, rv[i], yw[i]);
                 __syncthreads();
                 if (pass == 0)
-                    for (int i = t; i < N; i += 256) y1[i] = yw[i];
+                    for (int i = t; i < N; i += T) y1[i] = yw[i];
             }
             if (t == 0) s_flag = 0;
             __syncthreads();
@@ -483,10 +493,10 @@ __global__ void __launch_bounds__(256, WGS) ma_dense_reg_integrate(IntegrateArgs
             double err = 0.0;
             if (a.controller == WIND_CTRL_REFERENCE) {
                 bool fail = false;
-                for (int i = t; i < N; i += 256) fail = fail || species_fails<WIND_SIE>(y1[i], yw[i], a.ABS, a.REL);
+                for (int i = t; i < N; i += T) fail = fail || species_fails<WIND_SIE>(y1[i], yw[i], a.ABS, a.REL);
                 if (fail) s_flag = 1;
             } else {
-                for (int i = t; i < N; i += 256) err = err_max(err, err_term(y1[i], yw[i], a.ABS, a.REL));
+                for (int i = t; i < N; i += T) err = err_max(err, err_term(y1[i], yw[i], a.ABS, a.REL));
 #pragma unroll
                 for (int off = 32; off > 0; off >>= 1) err = err_max(err, __shfl_xor(err, off));
                 if (lane == 0) s_err[wave] = err;
@@ -495,12 +505,12 @@ __global__ void __launch_bounds__(256, WGS) ma_dense_reg_integrate(IntegrateArgs
             flag = s_flag != 0;
             if (a.controller != WIND_CTRL_REFERENCE) {
                 err = s_err[0];
-                for (int wv = 1; wv < 4; wv++) err = err_max(err, s_err[wv]);
+                for (int wv = 1; wv < WR * WC; wv++) err = err_max(err, s_err[wv]);
             }
             const bool extrap = a.controller != WIND_CTRL_REFERENCE;
             if constexpr (TRACE) {
                 if (attempts < a.trace.capacity) {
-                    for (int i = t; i < N; i += 256) {
+                    for (int i = t; i < N; i += T) {
                         if (a.trace.y1) a.trace.y1[slot * N + i] = y1[i];
                         if (a.trace.y2) a.trace.y2[slot * N + i] = yw[i];
                     }
@@ -511,7 +521,7 @@ __global__ void __launch_bounds__(256, WGS) ma_dense_reg_integrate(IntegrateArgs
                     attempts++;
                     if (a.trace.accept[slot]) {
                         tnow = tnow + hh;
-                        for (int i = t; i < N; i += 256) y[i] = extrap ? 2.0f * yw[i] - y1[i] : yw[i];
+                        for (int i = t; i < N; i += T) y[i] = extrap ? 2.0f * yw[i] - y1[i] : yw[i];
                     }
                     __syncthreads();
                     continue;
@@ -519,8 +529,13 @@ __global__ void __launch_bounds__(256, WGS) ma_dense_reg_integrate(IntegrateArgs
             }
             attempts++;
             const bool acc = control_step<WIND_SIE, true>(a.controller, a.tend, hh, flag, err, tnow, h, unsolved, status);
+            // (the same in every lane: kept in scalar registers)
+            tnow = uniform(tnow);
+            h = uniform(h);
+            unsolved = __builtin_amdgcn_readfirstlane(unsolved);
+            status = __builtin_amdgcn_readfirstlane(status);
             if (acc)
-                for (int i = t; i < N; i += 256) y[i] = extrap ? 2.0f * yw[i] - y1[i] : yw[i];
+                for (int i = t; i < N; i += T) y[i] = extrap ? 2.0f * yw[i] - y1[i] : yw[i];
             __syncthreads();
             if (status != WIND_STATUS_OK) break;
             if (attempts >= a.max_attempts && tnow < a.tend) {
@@ -529,7 +544,7 @@ __global__ void __launch_bounds__(256, WGS) ma_dense_reg_integrate(IntegrateArgs
             }
         }
         __syncthreads();
-        for (int i = t; i < N; i += 256) a.equations[(size_t)sid * N + i] = y[i];
+        for (int i = t; i < N; i += T) a.equations[(size_t)sid * N + i] = y[i];
         if (t == 0) {
             if (a.steps_out) a.steps_out[sid] = 3 * attempts;
             if (a.status_out) a.status_out[sid] = status;

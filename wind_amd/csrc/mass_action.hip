@@ -43,10 +43,11 @@ static bool ma_wave_fits(int N, int R) {
 }
 
 // Deals elements (their terms' words) to `threads` streams, most terms first
-// to the least-loaded thread; streams padded with zero words to the longest,
+// to the least-loaded thread; streams padded with `pad` to the longest,
 // rounded up to `batch`, and interleaved: word j of thread t at
 // [j * threads + t].
-static std::vector<int32_t> deal_streams(std::vector<std::vector<uint32_t>> &items, int threads, int batch, int *len) {
+static std::vector<int32_t> deal_streams(std::vector<std::vector<uint32_t>> &items, int threads, int batch,
+                                         uint32_t pad, int *len) {
     std::stable_sort(items.begin(), items.end(), [](const auto &p1, const auto &p2) { return p1.size() > p2.size(); });
     std::vector<std::vector<uint32_t>> per(threads);
     for (auto &it : items) {
@@ -57,7 +58,7 @@ static std::vector<int32_t> deal_streams(std::vector<std::vector<uint32_t>> &ite
     }
     size_t n = batch;
     for (auto &p : per) n = std::max(n, (p.size() + batch - 1) / batch * batch);
-    std::vector<int32_t> out(n * threads, 0);
+    std::vector<int32_t> out(n * threads, (int32_t)pad);
     for (int th = 0; th < threads; th++)
         for (size_t j = 0; j < per[th].size(); j++) out[j * threads + th] = (int32_t)per[th][j];
     *len = (int)n;
@@ -112,9 +113,10 @@ int mass_action_build(wind_network *n, int N, int R, const int32_t *rx, const fl
     // threads (deal_streams), and a thread's stream is its elements' terms,
     // one word each:
     //   (LDS float index of the term's h dJ value) << 16 | (buffer offset of
-    //   the element) << 3 | (element on the diagonal) << 2 | (element's last
-    //   term) << 1 | (reactant row: the term adds)
-    // The padding's zero words store nothing.
+    //   the element) << 3 | (element on the diagonal) << 2 | (element's first
+    //   term) << 1 | (the term is subtracted: a product row)
+    // f's elements (from 0, their terms w) follow the matrix's in the buffer,
+    // at sc_cap + row; padding words go to a place that nothing reads.
     const int NT = (N + 15) / 16;
     std::vector<int32_t> sc_ent;
     std::vector<uint32_t> sc_tile;
@@ -129,7 +131,7 @@ int mass_action_build(wind_network *n, int N, int R, const int32_t *rx, const fl
                 const int32_t *x = rx + 4 * r;
                 for (int which = 0; which < 2; which++) {
                     const uint32_t hd = (uint32_t)((which ? lo.hdb : lo.hda) + r);
-                    elem[{i, x[which]}].push_back((hd << 16) | ((x[which] == i ? 1u : 0u) << 2) | (uint32_t)neg);
+                    elem[{i, x[which]}].push_back((hd << 16) | ((x[which] == i ? 1u : 0u) << 2) | (uint32_t)!neg);
                 }
             }
         // the q present per (tile, lane), then the offsets
@@ -151,7 +153,7 @@ int mass_action_build(wind_network *n, int N, int R, const int32_t *rx, const fl
         }
         // (+1: an owner lane reads one place past its elements, unused)
         sc_cap = (int)((nnz + 1 + 3) & ~3u);
-        ok = ok && sc_cap < 8192;
+        ok = ok && sc_cap + 16 * NT <= 8192;
         std::vector<std::vector<uint32_t>> items;
         for (auto &kv : elem) {
             int tl, q;
@@ -159,10 +161,18 @@ int mass_action_build(wind_network *n, int N, int R, const int32_t *rx, const fl
             const uint32_t dest = (sc_tile[tl] >> 4) + (uint32_t)__builtin_popcount(mask4[tl] & ((1u << q) - 1));
             std::vector<uint32_t> w = kv.second;
             for (auto &x : w) x |= dest << 3;
-            w.back() |= 2u;
+            w.front() |= 2u;
             items.push_back(std::move(w));
         }
-        sc_ent = deal_streams(items, 256, kDenseRegBatch, &sc_len);
+        for (int i = 0; i < N && ok; i++) {
+            std::vector<uint32_t> w;
+            for (int32_t e : flist[i])
+                w.push_back((uint32_t)(lo.w + (e >> 1)) << 16 | (uint32_t)(sc_cap + i) << 3 | (uint32_t)(e & 1));
+            if (w.empty()) continue;
+            w.front() |= 2u;
+            items.push_back(std::move(w));
+        }
+        sc_ent = deal_streams(items, 256, kDenseRegBatch, nnz << 3, &sc_len);
         if (!ok) {
             sc_ent.clear();
             sc_tile.clear();
@@ -192,7 +202,7 @@ int mass_action_build(wind_network *n, int N, int R, const int32_t *rx, const fl
             items.push_back(std::move(w));
         }
         for (auto &w : items) w.back() |= 2u;
-        ex_ent = deal_streams(items, 128, kMaWaveBatch, &ex_len);
+        ex_ent = deal_streams(items, 128, kMaWaveBatch, 0, &ex_len);
     }
     MassActionDevice &d = n->ma;
     d.N = N;
