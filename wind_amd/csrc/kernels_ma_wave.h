@@ -181,7 +181,7 @@ __global__ void __launch_bounds__(128) ma_wave_integrate(IntegrateArgs a, MassAc
                 bool flag = false;
                 double err = 0.0;
                 if (a.controller == WIND_CTRL_REFERENCE) {
-                    flag = __any(lane < N && species_fails<WIND_SIE>(y1[col], y2, a.ABS, a.REL));
+                    flag = __any(lane < N && species_fails<WIND_SIE, true>(y1[col], y2, a.ABS, a.REL));
                 } else {
                     if (lane < N) err = err_term(y1[col], y2, a.ABS, a.REL);
 #pragma unroll

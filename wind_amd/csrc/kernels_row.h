@@ -376,7 +376,7 @@ __global__ void __launch_bounds__(256) row_integrate(IntegrateArgs a, typename N
         bool flag = false;
         double err = 0.0;
         if (a.controller == WIND_CTRL_REFERENCE) {
-            const bool fail = mine && species_fails<METHOD>(y1, y2, a.ABS, a.REL);
+            const bool fail = mine && species_fails<METHOD, true>(y1, y2, a.ABS, a.REL);
             flag = ((__ballot(fail) >> (__lane_id() & 48)) & 0xFFFFull) != 0;
         } else {
             err = row_err_max(mine ? err_term(y1, y2, a.ABS, a.REL) : 0.0);
@@ -473,7 +473,7 @@ __device__ inline void row_tile_integrate(const IntegrateArgs &a, const typename
             if (TT::kFirstTile && t < NB) s_new[t] = ynew;
             bool fail = false;
             if (a.controller == WIND_CTRL_REFERENCE) {
-                fail = mine && species_fails<METHOD>(y1, y2, a.ABS, a.REL);
+                fail = mine && species_fails<METHOD, true>(y1, y2, a.ABS, a.REL);
             } else {
                 double e = row_err_max(mine ? err_term(y1, y2, a.ABS, a.REL) : 0.0);
                 e = err_max(e, __shfl_xor(e, 16));
