@@ -82,6 +82,20 @@ def test_register_kernel_equals_oracle(N, controller):
     assert same(y, yr) and np.array_equal(steps, sr) and np.array_equal(status, tr)
 
 
+@pytest.mark.parametrize("N", [50, 80, 96, 97, 113, 129, 157])
+def test_dense_solver_results_do_not_depend_on_the_batch(N):
+    """Fast dense solver: few systems run on eight waves each, many on four; the same bits."""
+    n = 560
+    net = api.Network.mass_action(N, *W.mass_action_network(N, 700 + N))
+    y0, sc = W.mass_action_systems(n, N, 7, W.MIXED_SCALE_RANGE)
+    kw = {"tend": 1e6, "tol": 1e-10, "rel": 8e-5, "mode": api.MODE_FAST, "controller": api.CTRL_ADAPTIVE,
+          "max_attempts": 60}
+    full = run(net, n, y0, sc, api.KERNEL_AUTO, **kw)
+    for m in (1, 200, 512):
+        part = run(net, m, y0[:m * N], sc[:m], api.KERNEL_AUTO, **kw)
+        assert same(part[0], full[0][:m * N]) and np.array_equal(part[1], full[1][:m])
+
+
 def test_row_kernel_strides_hints_and_non_finite_states():
     net, n = api.Network.builtin(api.NET_HHE6, W.hhe6_params()), 129
     y0, c = W.hhe6_systems(n, 21)
@@ -120,3 +134,19 @@ def test_tiled_network_equals_oracle_also_where_a_tile_overflows(tiles, method, 
     if method == O.SIE and controller == api.CTRL_REFERENCE:
         assert np.isnan(yr.reshape(n, N)[2]).sum() > 5  # it does reach them
     assert same(y, yr) and np.array_equal(steps, sr) and np.array_equal(status, tr)
+
+
+@pytest.mark.parametrize("n", [1, 3, 32000, 33500])
+def test_host_arrays_equal_device_arrays(n):
+    """Host-pointer calls on both sides of the staging limit (1 MiB; 32 bytes a system here), outputs optional."""
+    torch = pytest.importorskip("torch")
+    net = api.Network.builtin(api.NET_NR_TEST)
+    y0, c, _ = W.nr_test_systems(n, 3)
+    y, steps, status = run(net, n, y0, c, api.KERNEL_AUTO, nfix=1000)
+    d, dc = torch.from_numpy(y0).cuda(), torch.from_numpy(c).cuda()
+    torch.cuda.synchronize()
+    total, _ = api.integrate(net, 0.0, 1.0, 1000, dc, d, n, 1e-3, 1e-3, device_pointers=True)
+    assert total == int(steps.astype(np.int64).sum()) and np.all(status == 0)
+    assert same(y, d.cpu().numpy())
+    bare = y0.copy()
+    assert api.integrate(net, 0.0, 1.0, 1000, c, bare, n, 1e-3, 1e-3)[0] == total and same(bare, y)

@@ -62,20 +62,21 @@ bool dense_reg_eligible(const MassActionDevice &d, const SolverChoice &sc) {
     return dense_reg_wgs_dev(d) != 0;
 }
 
-template <int NT, int WGS>
+template <int NT, int WGS, int WR = 2, int WC = 2>
 int launch_dense_reg_nt(int num_cu, const MassActionDevice &d, const IntegrateArgs &a, const SolverChoice &sc,
                         hipStream_t st) {
-    auto kfn = a.trace.capacity > 0 ? ma_dense_reg_integrate<NT, WGS, true> : ma_dense_reg_integrate<NT, WGS>;
+    auto kfn = a.trace.capacity > 0 ? ma_dense_reg_integrate<NT, WGS, WR, WC, true>
+                                      : ma_dense_reg_integrate<NT, WGS, WR, WC>;
     const size_t lds = dense_reg_lds_bytes(NT, d.R, WGS, d.sc_cap);
     if (lds > 65536) {
         hipError_t e = hipFuncSetAttribute((const void *)kfn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return wind_fail(WIND_ERR_DEVICE, hipGetErrorString(e));
     }
     int per_cu = 0;
-    hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kfn, 256, lds);
+    hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kfn, 64 * WR * WC, lds);
     if (e != hipSuccess) return wind_fail(WIND_ERR_DEVICE, hipGetErrorString(e));
     const int grid = scaled_grid(num_cu, per_cu, sc, a.nsys);
-    hipLaunchKernelGGL(kfn, dim3(grid), dim3(256), lds, st, a, d);
+    hipLaunchKernelGGL(kfn, dim3(grid), dim3(64 * WR * WC), lds, st, a, d);
     e = hipGetLastError();
     if (e != hipSuccess) return wind_fail(WIND_ERR_DEVICE, hipGetErrorString(e));
     return WIND_OK;
@@ -83,7 +84,25 @@ int launch_dense_reg_nt(int num_cu, const MassActionDevice &d, const IntegrateAr
 
 int launch_dense_reg(int num_cu, const MassActionDevice &d, const IntegrateArgs &a, const SolverChoice &sc,
                      hipStream_t st) {
-    switch ((d.N + 15) / 16) {
+    // Few systems: eight waves each, two workgroups per CU, no register
+    // spilled.  A system alone on its CU: N = 160 46.6 -> 37.0 us per
+    // sub-step, 128 29.2 -> 24.6, 96 18.4 -> 16.7, 64 10.6 -> 9.8; two per
+    // CU: 56.1 -> 50.3, 35.1 -> 33.2, 21.6 -> 21.8, 12.2 -> 12.7 (512
+    // systems to the end, N = 160 512 -> 450 ms, 128 367 -> 320, 96 159 ->
+    // 152).  With the CU full the four-wave form is the better one (N = 160
+    // 19.1 us per sub-step and CU against 25.2).
+    const int NT = (d.N + 15) / 16;
+    if (a.nsys <= num_cu * (NT >= 6 ? 2 : 1)) switch (NT) {
+        case 4: return launch_dense_reg_nt<4, 2, 4, 2>(num_cu, d, a, sc, st);
+        case 5: return launch_dense_reg_nt<5, 2, 4, 2>(num_cu, d, a, sc, st);
+        case 6: return launch_dense_reg_nt<6, 2, 4, 2>(num_cu, d, a, sc, st);
+        case 7: return launch_dense_reg_nt<7, 2, 4, 2>(num_cu, d, a, sc, st);
+        case 8: return launch_dense_reg_nt<8, 2, 4, 2>(num_cu, d, a, sc, st);
+        case 9: return launch_dense_reg_nt<9, 2, 4, 2>(num_cu, d, a, sc, st);
+        case 10: return launch_dense_reg_nt<10, 2, 4, 2>(num_cu, d, a, sc, st);
+        default: break;
+    }
+    switch (NT) {
     case 2:
         return dense_reg_wgs_dev(d) == 8 ? launch_dense_reg_nt<2, 8>(num_cu, d, a, sc, st)
                                          : launch_dense_reg_nt<2, 3>(num_cu, d, a, sc, st);

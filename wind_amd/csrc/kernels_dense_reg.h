@@ -1,9 +1,9 @@
 // Register-resident dense SIE solver for mass-action networks with
-// 16 NT - 15 <= N <= 16 NT (fast mode).  One 256-thread workgroup (four
-// waves) owns one system at a time, systems taken from a device queue, and
-// the matrix A = I - hJ lives in the waves' registers instead of LDS: wave
-// (wi, wj) holds the 16x16 tiles (i, j) with i = wi, j = wj (mod 2), each in
-// the MFMA accumulator layout (lane l holds rows 4(l/16) + q, q = 0..3, of
+// 16 NT - 15 <= N <= 16 NT (fast mode).  One workgroup of WR x WC waves
+// (2 x 2, or 4 x 2 for few systems, dense.hip) owns one system at a time,
+// systems taken from a device queue, and the matrix A = I - hJ lives in the
+// waves' registers instead of LDS: wave (wi, wj) holds the 16x16 tiles (i, j)
+// with i = wi (mod WR), j = wj (mod WC), each in the MFMA accumulator layout (lane l holds rows 4(l/16) + q, q = 0..3, of
 // column l % 16).  Without the matrix in LDS a workgroup needs a third
 // (N > 144 and few enough reactions: a quarter) of a CU's LDS and
 // registers, so three (four) systems share a CU and each one's serial
@@ -14,7 +14,7 @@
 // * assembly: the per-reaction rate terms and f as in the LDS solver
 //   (kernels_dense.h, dense_eval, same order, so f and every matrix element
 //   round identically); f and the matrix elements with Jacobian terms are
-//   summed into a compact LDS buffer (dealt to all 256 threads on the host,
+//   summed into a compact LDS buffer (dealt to all threads on the host,
 //   each element its terms in sweep order, one branch-free stream of term
 //   words per thread), and the owner lanes of the tiles read them into
 //   registers through per-lane offset and mask words (1 on the diagonal, 0
@@ -174,9 +174,9 @@ __device__ inline float uniform(float v) {
 
 // TRACE: per-attempt trace and replay through a.trace, as in the other
 // kernels.
-template <int NT, int WGS, bool TRACE = false>
-__global__ void __launch_bounds__(256, WGS) ma_dense_reg_integrate(IntegrateArgs a, MassActionDevice net) {
-    constexpr int WR = 2, WC = 2;  // the waves' grid
+template <int NT, int WGS, int WR, int WC, bool TRACE = false>
+__global__ void __launch_bounds__(64 * WR * WC, WGS *WR *WC / 4)
+    ma_dense_reg_integrate(IntegrateArgs a, MassActionDevice net) {
     constexpr int NP = 16 * NT, T = 64 * WR * WC, NR = (NT + WR - 1) / WR, NC = (NT + WC - 1) / WC;
     extern __shared__ float lds[];
     const int N = net.N, R = net.R, t = threadIdx.x;
@@ -188,7 +188,7 @@ __global__ void __launch_bounds__(256, WGS) ma_dense_reg_integrate(IntegrateArgs
     float *y = lds + o.y, *yw = lds + o.yw, *y1 = lds + o.y1, *rv = lds + o.r;
     float *w = lds + o.w, *hda = lds + o.hda, *hdb = lds + o.hdb, *kk = lds + o.k;
     int2 *ab = reinterpret_cast<int2 *>(lds + o.ab);
-    const int *__restrict__ scent = net.sc_ent;
+    const int *__restrict__ scent = T == 256 ? net.sc_ent : net.sc_ent2;
     const unsigned *__restrict__ sctile = net.sc_tile;
     float *work = lds + o.work, *f = work + net.sc_cap;
     float *Gbuf = work, *Cbuf = work + 256, *Wbuf = work + 256 * (NT + 1);
@@ -257,7 +257,7 @@ __global__ void __launch_bounds__(256, WGS) ma_dense_reg_integrate(IntegrateArgs
         if (t < NP) f[t] = 0.0f;  // species without reactions, and the padding
         __syncthreads();
         // f and the matrix's non-zero elements through a compact buffer: each
-        // thread walks its term stream (the elements dealt to the 256
+        // thread walks its term stream (the elements dealt to the
         // threads on the host, interleaved so that a batch of words is one
         // coalesced load per word); an element is its terms summed in order
         // in a register (from 1 on the diagonal), stored at its offset.
@@ -265,7 +265,7 @@ __global__ void __launch_bounds__(256, WGS) ma_dense_reg_integrate(IntegrateArgs
         // through its per-lane offset and mask word (1 on the diagonal, 0
         // elsewhere where the element is absent).
         {
-            const int len = net.sc_len;
+            const int len = T == 256 ? net.sc_len : net.sc_len2;
             float acc = 0.0f;
             for (int j = 0;;) {
                 float v[B];

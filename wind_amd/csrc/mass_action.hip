@@ -109,8 +109,8 @@ int mass_action_build(wind_network *n, int N, int R, const int32_t *rx, const fl
     // that offset plus the present q below it.  An element is its terms in
     // the order dense_eval applies them (the row's reactions in sweep order,
     // the reaction's first reactant before its second), summed from 1 on the
-    // diagonal; the elements are dealt to the workgroup's 256
-    // threads (deal_streams), and a thread's stream is its elements' terms,
+    // diagonal; the elements are dealt to the workgroup's 256 or
+    // 512 threads (deal_streams), and a thread's stream is its elements' terms,
     // one word each:
     //   (LDS float index of the term's h dJ value) << 16 | (buffer offset of
     //   the element) << 3 | (element on the diagonal) << 2 | (element's first
@@ -118,9 +118,9 @@ int mass_action_build(wind_network *n, int N, int R, const int32_t *rx, const fl
     // f's elements (from 0, their terms w) follow the matrix's in the buffer,
     // at sc_cap + row; padding words go to a place that nothing reads.
     const int NT = (N + 15) / 16;
-    std::vector<int32_t> sc_ent;
+    std::vector<int32_t> sc_ent, sc_ent2;
     std::vector<uint32_t> sc_tile;
-    int sc_len = 0, sc_cap = 0;
+    int sc_len = 0, sc_len2 = 0, sc_cap = 0;
     if (dense_reg_tiles(NT)) {
         const DenseRegOffsets lo = dense_reg_offsets(NT, R, 3, 0);
         bool ok = lo.hdb + R < 65536;
@@ -173,10 +173,12 @@ int mass_action_build(wind_network *n, int N, int R, const int32_t *rx, const fl
             items.push_back(std::move(w));
         }
         sc_ent = deal_streams(items, 256, kDenseRegBatch, nnz << 3, &sc_len);
+        sc_ent2 = deal_streams(items, 512, kDenseRegBatch, nnz << 3, &sc_len2);
         if (!ok) {
             sc_ent.clear();
+            sc_ent2.clear();
             sc_tile.clear();
-            sc_len = sc_cap = 0;
+            sc_len = sc_len2 = sc_cap = 0;
         }
     }
     // Assembly of the exact register kernel (ma_wave_integrate): f's and the
@@ -221,6 +223,8 @@ int mass_action_build(wind_network *n, int N, int R, const int32_t *rx, const fl
     if (!rc && !sc_ent.empty()) rc = upload((void **)&d.sc_tile, sc_tile.data(), sizeof(uint32_t) * sc_tile.size());
     if (!rc && !ex_ent.empty()) rc = upload((void **)&d.ex_ent, ex_ent.data(), sizeof(int32_t) * ex_ent.size());
     d.ex_len = ex_len;
+    if (!rc && !sc_ent2.empty()) rc = upload((void **)&d.sc_ent2, sc_ent2.data(), sizeof(int32_t) * sc_ent2.size());
+    d.sc_len2 = sc_len2;
     d.sc_len = sc_len;
     d.sc_cap = sc_cap;
     return rc;
@@ -228,7 +232,7 @@ int mass_action_build(wind_network *n, int N, int R, const int32_t *rx, const fl
 
 void mass_action_release(wind_network *n) {
     MassActionDevice &d = n->ma;
-    void *ptrs[] = {d.rx, d.k, d.f_ptr, d.f_ent, d.j_pos, d.j_ptr, d.j_ent, d.r_ptr, d.r_z, d.sc_ent, d.sc_tile, d.ex_ent};
+    void *ptrs[] = {d.rx, d.k, d.f_ptr, d.f_ent, d.j_pos, d.j_ptr, d.j_ent, d.r_ptr, d.r_z, d.sc_ent, d.sc_tile, d.sc_ent2, d.ex_ent};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     d = MassActionDevice();

@@ -31,6 +31,8 @@ struct MassActionDevice {
     int32_t *sc_ent = nullptr;
     uint32_t *sc_tile = nullptr;
     int sc_len = 0, sc_cap = 0;
+    int32_t *sc_ent2 = nullptr;  // the streams of 512 threads, sc_len2 words each
+    int sc_len2 = 0;
     // Exact register kernel (N <= 64, format in mass_action_build): word j
     // of thread t's term stream at ex_ent[j * 128 + t], ex_len words each.
     int32_t *ex_ent = nullptr;
