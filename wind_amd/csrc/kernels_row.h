@@ -314,6 +314,54 @@ inline int row_max_systems(int num_cu) {
     return (METHOD == WIND_SIE && Net::N >= 5 ? 64 : 16) * num_cu;
 }
 
+// Start order of the row kernel's systems (SIE): most remaining attempts
+// first, as the attempts so far extrapolate over the time left (rank
+// correlation 0.7 to 0.76 with the true ones on hhe6 after 600 to 5000
+// attempts; RK2's steps grow too unevenly for it).  A counting sort into four
+// classes per octave, one workgroup.
+template <int N>
+__global__ void __launch_bounds__(1024) spill_order(IntegrateArgs a) {
+    constexpr int C = 64;
+    __shared__ unsigned start[C];
+    const unsigned *words = reinterpret_cast<const unsigned *>(a.counters);
+    const bool second = (int)words[SPILL_FIRST] > a.spill_pack;
+    const int n = (int)words[second ? SPILL_SECOND : SPILL_FIRST], t = threadIdx.x;
+    const float *list = a.spill + (size_t)(second ? a.spill_cap : 0) * spill_record_words(N);
+    auto cls = [&](int k) {
+        const float *r = list + (size_t)k * spill_record_words(N);
+        const float est = (float)__float_as_int(r[N + 3]) * (a.tend - r[N]) / fmaxf(r[N] - a.tnow, 1.0e-30f);
+        // exponent and two mantissa bits, from 2^4 up; NaN first, as longest
+        const int b = (int)(__float_as_uint(est) >> 21) - ((127 + 4) << 2);
+        return C - 1 - min(max(b, 0), C - 1);
+    };
+    if (t < C) start[t] = 0;
+    __syncthreads();
+    for (int k = t; k < n; k += 1024) atomicAdd(&start[cls(k)], 1u);
+    __syncthreads();
+    if (t == 0) {
+        unsigned run = 0;
+        for (int i = 0; i < C; i++) {
+            const unsigned c = start[i];
+            start[i] = run;
+            run += c;
+        }
+    }
+    __syncthreads();
+    for (int k = t; k < n; k += 1024) a.spill_index[atomicAdd(&start[cls(k)], 1u)] = k;
+}
+
+// Row workgroups per CU behind a lane kernel: with one wave per SIMD (RK2,
+// which divides less, two) the longest systems run at their own pace, and the
+// order has something to choose from.  hhe6 SIE, 8 (all that fit) / 2 / 1 per
+// CU, in list order: 100,003 systems 177 / 144 / 143 ms, 50,003 121 / 111 / 85,
+// 1,000,003 321 / 294 / 299; longest first 169 / 133 / 137, 105 / 102 / 82 and
+// 303 / 278 / 276.  RK2, 100,003 systems 104 / 59 / 83 in list order, 93 / 70 /
+// 95 longest first.
+constexpr int row_tail_per_cu(int method) { return method == WIND_SIE ? 1 : 2; }
+
+// Threads that give each of nsys systems a row.
+inline int row_threads(int nsys) { return 16 * (nsys < (1 << 26) ? nsys : 1 << 26); }
+
 // One system per row, four per wave, taken from the device queue; or (TAIL)
 // the systems that the lane kernel before it handed over (a.spill).
 template <class Net, int METHOD, bool TAIL = false>
@@ -322,8 +370,10 @@ __global__ void __launch_bounds__(256) row_integrate(IntegrateArgs a, typename N
     static_assert(N <= 16, "one equation per lane of a 16-lane row");
     const int li = threadIdx.x & 15;
     const bool mine = li < N;
-    unsigned int *head = reinterpret_cast<unsigned int *>(a.counters + (TAIL ? 3 : 0));
-    const int count = TAIL ? (int)*reinterpret_cast<const unsigned *>(a.counters + 2) : a.nsys;
+    unsigned int *const words = reinterpret_cast<unsigned int *>(a.counters);
+    unsigned int *head = words + (TAIL ? SPILL_ROW_HEAD : 0);
+    const bool second = TAIL && (int)words[SPILL_FIRST] > a.spill_pack;
+    const int count = !TAIL ? a.nsys : (int)words[second ? SPILL_SECOND : SPILL_FIRST];
     RowEval<Net, MathExact> ev(p, li);
     float y[N], c[NC > 0 ? NC : 1], yo = 0.0f, tnow = 0.0f, h = 0.0f;
     int sid = 0, unsolved = 0, attempts = 0, status = WIND_STATUS_OK;
@@ -343,7 +393,9 @@ __global__ void __launch_bounds__(256) row_integrate(IntegrateArgs a, typename N
                 active = got < count;
                 if (active) {
                     if constexpr (TAIL) {
-                        const float *r = a.spill + (size_t)got * spill_record_words(N);
+                        const float *r = a.spill + (size_t)((METHOD == WIND_SIE ? a.spill_index[got] : got) +
+                                                               (second ? a.spill_cap : 0)) *
+                                                      spill_record_words(N);
                         yo = r[mine ? li : 0];
                         tnow = r[N];
                         h = r[N + 1];

@@ -374,15 +374,18 @@ __device__ inline void wave_add_steps(unsigned long long *total, unsigned long l
 
 // The body of lane_integrate, shared with kernels that set other launch
 // bounds or are compiled with other floating-point contraction.
-// Hands the wave's unfinished systems (lanes `busy`) to the row kernel.
-template <int N>
+// Hands the wave's unfinished systems (lanes `busy`) over, into the first
+// list or (SECOND) the second.
+template <int N, bool SECOND>
 __device__ inline void spill_systems(const IntegrateArgs &a, const LaneSys<N> &s, int sid, bool active,
                                      unsigned long long busy) {
     constexpr int R = spill_record_words(N);
     const int lane = __lane_id();
     unsigned base = 0;
-    if (lane == 0) base = atomicAdd(reinterpret_cast<unsigned *>(a.counters + 2), (unsigned)__popcll(busy));
-    base = __shfl(base, 0);
+    if (lane == 0)
+        base = atomicAdd(reinterpret_cast<unsigned *>(a.counters) + (SECOND ? SPILL_SECOND : SPILL_FIRST),
+                         (unsigned)__popcll(busy));
+    base = __shfl(base, 0) + (SECOND ? (unsigned)a.spill_cap : 0u);
     if (!active) return;
     const unsigned long long below = lane ? (~0ull >> (64 - lane)) : 0ull;
     float r[R] = {};
@@ -398,12 +401,15 @@ __device__ inline void spill_systems(const IntegrateArgs &a, const LaneSys<N> &s
     for (int v = 0; v < R / 4; v++) out[v] = make_float4(r[4 * v], r[4 * v + 1], r[4 * v + 2], r[4 * v + 3]);
 }
 
-// SPILL: with a.spill set, the wave's last systems go to the row kernel.
-template <class Net, int METHOD, class M, bool TRACE = false, bool SPILL = false>
+// SPILL: with a.spill set, the wave's last systems are handed over; 2: the
+// second pass, over the systems of the first list.
+template <class Net, int METHOD, class M, bool TRACE = false, int SPILL = 0>
 __device__ inline void lane_integrate_body(const IntegrateArgs &a, const typename Net::Params &p) {
     constexpr int N = Net::N;
     constexpr int NC = Net::NCONST;
-    unsigned int *head = reinterpret_cast<unsigned int *>(a.counters);
+    unsigned int *head = reinterpret_cast<unsigned int *>(a.counters) + (SPILL == 2 ? SPILL_LANE_HEAD : 0);
+    const int count = SPILL == 2 ? (int)reinterpret_cast<const unsigned *>(a.counters)[SPILL_FIRST] : a.nsys;
+    if (SPILL == 2 && count <= a.spill_pack) return;
     LaneSys<N> s;
     float c[NC];
     int sid = 0;
@@ -411,12 +417,20 @@ __device__ inline void lane_integrate_body(const IntegrateArgs &a, const typenam
     unsigned long long steps = 0;
     for (;;) {
         const int got = queue_fetch(head, need);
-        if constexpr (SPILL) dry = dry || __any(need && got >= a.nsys);
+        if constexpr (SPILL != 0) dry = dry || __any(need && got >= count);
         if (need) {
             need = false;
-            active = got < a.nsys;
+            active = got < count;
             if (active) {
-                if (a.records) {
+                if constexpr (SPILL == 2) {
+                    const float *r = a.spill + (size_t)got * spill_record_words(N);
+#pragma unroll
+                    for (int i = 0; i < N; i++) s.y[i] = r[i];
+                    sid = __float_as_int(r[N + 4]);
+                    const float *cs = a.constants + (size_t)sid * a.const_stride;
+#pragma unroll
+                    for (int k = 0; k < NC; k++) c[k] = cs[k];
+                } else if (a.records) {
                     // the system's packed record, read in 16-byte pieces
                     constexpr int R = lane_record_words(N, NC);
                     float r[R];
@@ -447,13 +461,20 @@ __device__ inline void lane_integrate_body(const IntegrateArgs &a, const typenam
                 s.unsolved = 0;
                 s.attempts = 0;
                 s.status = WIND_STATUS_OK;
+                if constexpr (SPILL == 2) {
+                    const float *r = a.spill + (size_t)got * spill_record_words(N);
+                    s.tnow = r[N];
+                    s.h = r[N + 1];
+                    s.unsolved = __float_as_int(r[N + 2]);
+                    s.attempts = __float_as_int(r[N + 3]);
+                }
             }
         }
         const unsigned long long busy = __ballot(active);
         if (busy == 0ull) break;
-        if constexpr (SPILL) {
+        if constexpr (SPILL != 0) {
             if (dry && __popcll(busy) <= a.spill_at) {
-                spill_systems<N>(a, s, sid, active, busy);
+                spill_systems<N, SPILL == 2>(a, s, sid, active, busy);
                 break;
             }
         }
@@ -470,7 +491,7 @@ __device__ inline void lane_integrate_body(const IntegrateArgs &a, const typenam
     wave_add_steps(a.counters + 1, steps);
 }
 
-template <class Net, int METHOD, class M, bool TRACE = false, bool SPILL = false>
+template <class Net, int METHOD, class M, bool TRACE = false, int SPILL = 0>
 __global__ void __launch_bounds__(256) lane_integrate(IntegrateArgs a, typename Net::Params p) {
     lane_integrate_body<Net, METHOD, M, TRACE, SPILL>(a, p);
 }

@@ -80,19 +80,23 @@ int plugin_launch_method(const IntegrateArgs &a, int mode, int kernel, int num_c
                 if (kernel == WIND_KERNEL_AUTO && a.nsys <= row_max_systems<Net, METHOD>(num_cu)) {
                     auto k = row_integrate<Net, METHOD>;
                     int grid = 0;
-                    const int rc = plugin_grid(k, 256, a.nsys * 16, num_cu, share, grid_cap, &grid);
+                    const int rc = plugin_grid(k, 256, row_threads(a.nsys), num_cu, share, grid_cap, &grid);
                     if (rc) return rc;
                     hipLaunchKernelGGL(k, dim3(grid), dim3(256), 0, st, a, p);
                     return hipGetLastError() == hipSuccess ? WIND_OK : WIND_ERR_DEVICE;
                 }
                 if (a.spill) {
-                    auto k = lane_integrate<Net, METHOD, MathExact, false, true>;
+                    auto k = lane_integrate<Net, METHOD, MathExact, false, 1>;
+                    auto k2 = lane_integrate<Net, METHOD, MathExact, false, 2>;
                     auto kt = row_integrate<Net, METHOD, true>;
-                    int grid = 0, grid_t = 0;
-                    int rc = plugin_grid(k, 256, a.nsys, num_cu, share, grid_cap, &grid);
-                    if (!rc) rc = plugin_grid(kt, 256, a.nsys, num_cu, share, grid_cap, &grid_t);
+                    int grid = 0;
+                    const int rc = plugin_grid(k, 256, a.nsys, num_cu, share, grid_cap, &grid);
                     if (rc) return rc;
+                    const int grid_t = row_tail_per_cu(METHOD) * num_cu;
                     hipLaunchKernelGGL(k, dim3(grid), dim3(256), 0, st, a, p);
+                    if (a.spill_cap > a.spill_pack) hipLaunchKernelGGL(k2, dim3(num_cu), dim3(256), 0, st, a, p);
+                    if (METHOD == WIND_SIE)
+                        hipLaunchKernelGGL(spill_order<Net::N>, dim3(1), dim3(1024), 0, st, a);
                     hipLaunchKernelGGL(kt, dim3(grid_t), dim3(256), 0, st, a, p);
                     return hipGetLastError() == hipSuccess ? WIND_OK : WIND_ERR_DEVICE;
                 }

@@ -299,15 +299,19 @@ int activity_hints(int num_cu, const wind_network *net, const IntegrateArgs &a, 
     }
 }
 
-// Lanes of a wave at which, its queue empty, its last systems go to the row
-// kernel (kernels_row.h): a lane wave costs three row waves' instructions
-// whatever its lanes do, and a row attempt takes a third of the time.  With
-// none / 8 / 16 / 24 / 32 / 48 lanes handed over, hhe6 SIE (reference
-// controller, t = 1 Myr) took 100,003 systems 475 / 225 / 160 / 154 / 167 /
-// 164 ms and 1,000,003 (t = 10^4) 634 / 415 / 384 / 374 / 385 / 410; katz96
-// 200,000 2.92 / 2.56 / 2.48 / 2.43 / 2.45 / 2.55; NR_test (N = 2) 200,000
-// 0.50 / 0.52 / 0.64 / 0.89, so only systems of five equations on do it.
-constexpr int kSpillAt = 24;
+// Lanes of a wave at which, its queue empty, its last systems are handed
+// over (to a second lane pass where they still fill waves, more than 32 per
+// CU, and to the row kernel in the end, kernels_row.h): a lane wave costs
+// three row waves' instructions whatever its lanes do, and a row attempt takes
+// a third of the time.  hhe6 SIE, reference controller, 20,000 (t = 1 Myr) /
+// 100,003 (1 Myr) / 1,000,003 systems (10^4 yr): 391 / 475 / 634 ms without
+// hand-over; at 24 / 32 / 40 lanes 77 / 88 / 81, 154 / 137 / 135 and 292 / 276 /
+// 279; at 32 without the second pass 74 / 143 / 357.  katz96 200,000 2.92 ms
+// without, 2.11 at 40, 2.88 at 32 without the second pass; NR_test (N = 2)
+// 200,000 0.50 without, 0.52 to 0.89 with, so only systems of five equations
+// on do it.
+constexpr int kSpillAt = 40;
+constexpr int kSpillPackPerCu = 32;
 bool spills(const wind_network *net, int mode, int nsys, int num_cu) {
     const bool lanes = net->builtin == WIND_NET_KATZ96 || net->builtin == WIND_NET_HHE6 || net->builtin == WIND_NET_PLUGIN;
     return mode == WIND_MODE_EXACT && lanes && net->N >= 5 && net->N <= 8 && nsys > 16 * num_cu;
@@ -336,17 +340,20 @@ int launch_small(int num_cu, const wind_network *net, const IntegrateArgs &a, in
                a.nsys <= row_max_systems<Net, METHOD>(num_cu)) {
         auto k = row_integrate<Net, METHOD>;
         int grid = 0;
-        int rc = persistent_grid(num_cu, k, 256, a.nsys * 16, &grid, sc);
+        int rc = persistent_grid(num_cu, k, 256, row_threads(a.nsys), &grid, sc);
         if (rc) return rc;
         hipLaunchKernelGGL(k, dim3(grid), dim3(256), 0, st, a, p);
     } else if (mode == WIND_MODE_EXACT && a.spill) {
-        auto k = lane_integrate<Net, METHOD, MathExact, false, true>;
+        auto k = lane_integrate<Net, METHOD, MathExact, false, 1>;
+        auto k2 = lane_integrate<Net, METHOD, MathExact, false, 2>;
         auto kt = row_integrate<Net, METHOD, true>;
-        int grid = 0, grid_t = 0;
+        int grid = 0;
         int rc = persistent_grid(num_cu, k, 256, a.nsys, &grid, sc);
-        if (!rc) rc = persistent_grid(num_cu, kt, 256, a.nsys, &grid_t, sc);
         if (rc) return rc;
+        const int grid_t = row_tail_per_cu(METHOD) * num_cu;
         hipLaunchKernelGGL(k, dim3(grid), dim3(256), 0, st, a, p);
+        if (a.spill_cap > a.spill_pack) hipLaunchKernelGGL(k2, dim3(num_cu), dim3(256), 0, st, a, p);
+        if (METHOD == WIND_SIE) hipLaunchKernelGGL(spill_order<Net::N>, dim3(1), dim3(1024), 0, st, a);
         hipLaunchKernelGGL(kt, dim3(grid_t), dim3(256), 0, st, a, p);
     } else if (mode == WIND_MODE_EXACT) {
         auto k = a.trace.capacity > 0 ? lane_integrate<Net, METHOD, MathExact, true>
@@ -978,11 +985,15 @@ int wind_integrate(const wind_network *net, float tnow, float tend, int n_integr
     a.records = pk.rec;
     if (opts.kernel == WIND_KERNEL_AUTO && !opts.trace && spills(net, opts.mode, Nsystems, c.num_cu)) {
         a.spill_at = kSpillAt;
-        // at most 32 waves per CU, each of which hands over once
+        a.spill_pack = kSpillPackPerCu * c.num_cu;
+        // at most 32 waves per CU, each of which hands over once; two lists
         const size_t most = std::min((size_t)Nsystems, (size_t)c.num_cu * 32 * kSpillAt);
-        rc = reserve(sl->spill, sizeof(float) * spill_record_words(Neqn) * most);
+        a.spill_cap = (int)most;
+        const size_t words = (size_t)spill_record_words(Neqn) * 2 * most;
+        rc = reserve(sl->spill, sizeof(float) * (words + most));
         if (rc) return rc;
         a.spill = (float *)sl->spill.ptr;
+        a.spill_index = (int32_t *)(a.spill + words);
     }
     std::vector<TraceCopy> trace_back;
     if (opts.trace) {

@@ -49,12 +49,22 @@ struct IntegrateArgs {
     const float *records = nullptr;
     // optional (lane kernels with a row-kernel tail, kernels_row.h): a wave
     // whose queue is empty and whose unfinished systems are at most
-    // spill_at hands them over: system k's state to record k of
-    // spill_record_words(N) floats, k counted in the low word of counters[2];
-    // the row kernel that follows takes them through counters[3].
+    // spill_at hands them over, each as a record of spill_record_words(N)
+    // floats.  First list: records 0 .. spill_cap - 1 of spill; when it holds
+    // more than spill_pack systems, a second pass of the lane kernel takes
+    // them, packed into full waves again, and hands its own last ones over in
+    // the second list, behind the first.  The row kernel takes the last list.
+    // The lists' lengths and queue heads are 32-bit words of counters
+    // (spill_word).
     float *spill = nullptr;
-    int32_t spill_at = 0;
+    int32_t *spill_index = nullptr;  // the row kernel's start order, [spill_cap]
+    int32_t spill_at = 0, spill_cap = 0, spill_pack = 0;
 };
+
+// 32-bit words of IntegrateArgs::counters for the hand-over: lengths of the
+// two lists, and the heads of the second lane pass's and the row kernel's
+// queues.
+enum SpillWord { SPILL_FIRST = 4, SPILL_SECOND = 5, SPILL_ROW_HEAD = 6, SPILL_LANE_HEAD = 7 };
 
 // Floats per packed record: state, constants and the system id, rounded up
 // to whole 32-byte sectors.
