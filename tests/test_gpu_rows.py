@@ -52,7 +52,7 @@ def test_row_kernel_equals_lane_kernel(name, method, controller, n):
 
 
 @pytest.mark.parametrize("name,n,method,controller", [
-    ("katz96", 16385, api.SIE, api.CTRL_REFERENCE), ("katz96", 4097, api.RK2, api.CTRL_ADAPTIVE),
+    ("katz96", 16385, api.SIE, api.CTRL_REFERENCE), ("hhe6", 4097, api.SIE, api.CTRL_REFERENCE), ("katz96", 4097, api.RK2, api.CTRL_ADAPTIVE),
     ("hhe6", 17001, api.SIE, api.CTRL_ADAPTIVE), ("hhe6", 140001, api.RK2, api.CTRL_REFERENCE),
     ("mixed5", 70001, api.SIE, api.CTRL_REFERENCE), ("katz96", 300007, api.SIE, api.CTRL_REFERENCE)])
 def test_tail_on_rows_equals_lane_kernel(name, n, method, controller):

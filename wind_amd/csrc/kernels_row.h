@@ -309,9 +309,13 @@ constexpr bool row_network() {
 // 0.148 / 0.096, 20000 0.198 / 0.162 (adaptive 8192 0.036 / 0.050); NR_test
 // SIE 4096 0.140 / 0.106, 8192 0.139 / 0.127, 20000 0.147 / 0.239 (adaptive
 // 4096 0.044 / 0.048, 8192 0.044 / 0.063).
+// With a hand-over available (SIE, reference controller, rows / lanes with
+// hand-over) hhe6 4097 systems took 62.7 / 68.1 ms, 5000 71.0 / 65.8, 16384
+// 142 / 72; katz96 8192 0.43 / 0.52, 12000 0.67 / 0.62.
 template <class Net, int METHOD>
-inline int row_max_systems(int num_cu) {
-    return (METHOD == WIND_SIE && Net::N >= 5 ? 64 : 16) * num_cu;
+inline int row_max_systems(int num_cu, bool handover) {
+    if (METHOD != WIND_SIE || Net::N < 5) return 16 * num_cu;
+    return (!handover ? 64 : Net::N == 5 ? 40 : 16) * num_cu;
 }
 
 // Start order of the row kernel's systems (SIE): most remaining attempts

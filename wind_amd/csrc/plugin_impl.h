@@ -77,7 +77,7 @@ int plugin_launch_method(const IntegrateArgs &a, int mode, int kernel, int num_c
     } else if (choice == 0) {
         if constexpr (Net::N <= kGenLaneMaxN) {
             if constexpr (row_network<Net>()) {
-                if (kernel == WIND_KERNEL_AUTO && a.nsys <= row_max_systems<Net, METHOD>(num_cu)) {
+                if (kernel == WIND_KERNEL_AUTO && a.nsys <= row_max_systems<Net, METHOD>(num_cu, a.spill != nullptr)) {
                     auto k = row_integrate<Net, METHOD>;
                     int grid = 0;
                     const int rc = plugin_grid(k, 256, row_threads(a.nsys), num_cu, share, grid_cap, &grid);

@@ -337,7 +337,7 @@ int launch_small(int num_cu, const wind_network *net, const IntegrateArgs &a, in
         const int grid = scaled_grid(num_cu, 32, sc, a.nsys);
         hipLaunchKernelGGL((block_integrate<Net, METHOD>), dim3(grid), dim3(64), 0, st, a, p);
     } else if (mode == WIND_MODE_EXACT && kernel == WIND_KERNEL_AUTO && a.trace.capacity == 0 &&
-               a.nsys <= row_max_systems<Net, METHOD>(num_cu)) {
+               a.nsys <= row_max_systems<Net, METHOD>(num_cu, a.spill != nullptr)) {
         auto k = row_integrate<Net, METHOD>;
         int grid = 0;
         int rc = persistent_grid(num_cu, k, 256, row_threads(a.nsys), &grid, sc);
