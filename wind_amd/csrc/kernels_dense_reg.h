@@ -29,19 +29,27 @@
 //   G = A11^-1, per 16-column panel k, with two barriers:
 //     B: W_kj = G_k A_kj for the row panel (G_k from LDS, A_kj in the
 //        owner's registers; W replaces A_kj and goes to LDS), the column
-//        panel A_ik to LDS, and the forward sweep r_i -= A_ik c_k;
+//        panel A_ik to LDS, and the forward sweep: A_ik c_k is added to the
+//        row's sums, a lane's columns in the lane; row k + 1, complete, is
+//        summed over its lanes;
 //     C: the trailing update A_ij -= A_ik W_kj on the matrix cores
 //        (v_mfma_f32_16x16x4f32, operands from LDS, accumulator in place);
 //        the owner of the next diagonal tile updates it first, inverts it in
 //        registers (Gauss-Jordan on its transpose, which the accumulator
 //        layout holds as rows), publishes G_{k+1} and forms c_{k+1} =
 //        G_{k+1} r_{k+1};
-// * backward sweep x_k = c_k - sum_{j>k} W_kj x_j by columns, one barrier per
-//   block, the W tiles still in registers;
+// * backward sweep x_k = c_k - sum_{j>k} W_kj x_j by columns, its sums kept the
+//   same way, one barrier per block, the W tiles still in registers;
 // * y += h x.
-// Tile matrix-vector products reduce over the 16 lanes of a row with DPP
-// shifts in a fixed order; every result is deterministic and independent of
-// the grid.  The step control is the LDS solver's.
+// The sweeps' sums live in the registers of tiles that are no longer needed
+// and are reduced (DPP shifts over the 16 lanes of a row, then one partial sum
+// per wave column through LDS) once per block row.  Reduced and subtracted in
+// LDS per tile instead, a sub-step took 19.1 instead of 17.6 us per CU at
+// N = 157 with four systems on it and 37.0 instead of 34.0 us alone, 3.92 /
+// 3.81 (four on the CU) and 9.8 / 9.5 (alone) at N = 64, and whole batches 630
+// / 579 ms (1,024 systems, N = 157) and 812 / 719 (4,096, N = 100).  Every
+// result is deterministic and independent of the grid and of the waves'
+// number.  The step control is the LDS solver's.
 #pragma once
 #include "kernels_dense.h"
 
@@ -67,13 +75,16 @@ constexpr int kDenseRegBatch = 8;
 template <int NT>
 constexpr int kDenseRegGW = NT >= 8 ? 2 : 1;
 
+// Wave columns of every shape.
+constexpr int kDenseRegWC = 2;
+
 // LDS layout of the register-resident solver (offsets in floats, 16-byte
-// aligned): per-system vectors, per-reaction rate terms, reactant indices
+// aligned): per-system vectors, the sweeps' partial sums, per-reaction rate terms, reactant indices
 // and rate constants, and a work area shared by the assembly's compact
 // element buffer (cap floats) with f behind it, and the factorisation's panel
 // buffers.  The term lists stay in global memory.
 struct DenseRegOffsets {
-    int y, yw, y1, r, w, hda, hdb, k, ab, work, total;
+    int y, yw, y1, r, part, w, hda, hdb, k, ab, work, total;
 };
 
 __host__ __device__ inline DenseRegOffsets dense_reg_offsets(int NT, int R, int WGS, int cap) {
@@ -89,6 +100,8 @@ __host__ __device__ inline DenseRegOffsets dense_reg_offsets(int NT, int R, int 
     p = up(p + NP);
     o.r = p;
     p = up(p + NP);
+    o.part = p;
+    p = up(p + 3 * kDenseRegWC * 16);
     o.w = p;
     p = up(p + R);
     o.hda = p;
@@ -154,18 +167,14 @@ __device__ inline void tile_invert_acc(f32x4 &m, int lane) {
     m = f32x4{a[0], a[1], a[2], a[3]};
 }
 
-// dst[16 i + 4g + q] (q = 0..3, lanes with c = 15 store) = mode: dst - T v,
-// or T v; T in the accumulator layout, v[c] the lane's column entry.
-template <bool SUBTRACT>
-__device__ inline void tile_matvec_store(const f32x4 &m, float v, float *dst, int lane) {
+// dst[4g + q] (q = 0..3, lanes with c = 15 store) = the sum of m[q] over the
+// 16 lanes of the lane's DPP row (the columns).
+__device__ inline void tile_rowsum_store(const f32x4 &m, float *dst, int lane) {
     const int c = lane & 15, g = lane >> 4;
-    float p[4];
+    f32x4 p;
 #pragma unroll
-    for (int q = 0; q < 4; q++) p[q] = row_sum16(m[q] * v);
-    if (c == 15) {
-#pragma unroll
-        for (int q = 0; q < 4; q++) dst[4 * g + q] = SUBTRACT ? dst[4 * g + q] - p[q] : p[q];
-    }
+    for (int q = 0; q < 4; q++) p[q] = row_sum16(m[q]);
+    if (c == 15) *reinterpret_cast<f32x4 *>(dst + 4 * g) = p;
 }
 
 __device__ inline float uniform(float v) {
@@ -177,6 +186,7 @@ __device__ inline float uniform(float v) {
 template <int NT, int WGS, int WR, int WC, bool TRACE = false>
 __global__ void __launch_bounds__(64 * WR * WC, WGS *WR *WC / 4)
     ma_dense_reg_integrate(IntegrateArgs a, MassActionDevice net) {
+    static_assert(WC == kDenseRegWC, "the sweeps' partial sums are laid out for this");
     constexpr int NP = 16 * NT, T = 64 * WR * WC, NR = (NT + WR - 1) / WR, NC = (NT + WC - 1) / WC;
     extern __shared__ float lds[];
     const int N = net.N, R = net.R, t = threadIdx.x;
@@ -198,7 +208,8 @@ __global__ void __launch_bounds__(64 * WR * WC, WGS *WR *WC / 4)
     float *const cA = Cbuf + wi * 256 + lr * 16 + 4 * g;  // A-operand reads of Cbuf tile i: + ta * RS
     float *const cS = Cbuf + wi * 256 + 64 * g + lr;      // stores to Cbuf tile i: + ta * RS + q * 16
     float *const wB = Wbuf + wj * 256 + lane * 4;          // Wbuf tile j: + tb * CS
-    float *const rI = rv + 16 * wi;                        // rows of tile row i: + 16 * WR * ta
+    float *const fp = lds + o.part, *const bp = fp + 16 * WC;  // partial sums, by wave column: forward; backward, twice
+    float *const xv = work;                                    // the solution (no panel buffer is in use by then)
     for (int r = t; r < R; r += T) {
         ab[r] = make_int2(net.rx[4 * r], net.rx[4 * r + 1]);
         if (WGS == 3) kk[r] = net.k[r];
@@ -319,14 +330,22 @@ __global__ void __launch_bounds__(64 * WR * WC, WGS *WR *WC / 4)
         tile_invert_acc(m, lane);
 #pragma unroll
         for (int q = 0; q < 4; q++) Gbuf[(4 * g + q) * 16 + lr] = m[q];
-        const float v = rv[16 * k + lr];
-        tile_matvec_store<false>(m, v, rv + 16 * k, lane);
+        float v = rv[16 * k + lr];
+#pragma unroll
+        for (int u = 0; u < WC; u++)
+            if (u < k) v -= fp[16 * u + lr];
+#pragma unroll
+        for (int q = 0; q < 4; q++) m[q] *= v;
+        tile_rowsum_store(m, rv + 16 * k, lane);
     };
+
+    // the last tile column of wave column u
+    auto last_col = [](int u) __attribute__((always_inline)) { return NT - 1 - (NT - 1 - u) % WC; };
 
     // Block LU without pivoting with the forward sweep on rv (= f on entry),
     // per 16-column panel k (two barriers): B) the row panel W_kj = G_k A_kj
     // (G_k from LDS; W replaces A_kj and goes to LDS), the column panel A_ik
-    // (i > k) to LDS and r_i -= A_ik c_k; C) A_ij -= A_ik W_kj on the matrix
+    // (i > k) to LDS and the sums of A_ik c_k; C) A_ij -= A_ik W_kj on the matrix
     // cores, the owner of the next diagonal tile updating it first, inverting
     // it and forming c_{k+1} = G_{k+1} r_{k+1}.  Leaves c in rv.
     auto factor = [&]() __attribute__((always_inline)) {
@@ -366,10 +385,22 @@ __global__ void __launch_bounds__(64 * WR * WC, WGS *WR *WC / 4)
                         if (i <= k || i >= NT) continue;
                         const f32x4 m = M[ta][tb];
 #pragma unroll
-                        for (int q = 0; q < 4; q++) cS[ta * RS + q * 16] = -m[q];
-                        tile_matvec_store<true>(m, ck, rI + 16 * WR * ta, lane);
+                        for (int q = 0; q < 4; q++) {
+                            cS[ta * RS + q * 16] = -m[q];
+                            // the row's sum of A_ik c_k over this wave's
+                            // columns, a lane's columns in the lane, in the
+                            // registers of the first of these tiles (each is
+                            // in the panel buffer from here on)
+                            M[ta][0][q] = tb == 0 ? m[q] * ck : fmaf(m[q], ck, M[ta][0][q]);
+                        }
                     }
                 }
+            }
+            // row k + 1 has all its columns
+            if (wi == (k + 1) % WR && wj <= k) {
+#pragma unroll
+                for (int ta = 0; ta < NR; ta++)
+                    if (WR * ta + wi == k + 1) tile_rowsum_store(M[ta][0], fp + 16 * wj, lane);
             }
             __syncthreads();
             const int k1 = k + 1;
@@ -426,27 +457,50 @@ __global__ void __launch_bounds__(64 * WR * WC, WGS *WR *WC / 4)
         }
     };
 
-    // Backward sweep by columns: x_k = c_k, then c_i -= W_ik x_k above.
+    // Backward sweep by columns: x_k = c_k - sum_j W_kj x_j, the sums kept as
+    // in the forward sweep, in the registers of the last of a row's tiles.
+    // Leaves x_k in xv for k > 0 and the partial sums of row 0 in bp.
     auto back = [&]() __attribute__((always_inline)) {
         int wv = wave;
         asm volatile("" : "+s"(wv));
         const int wi = wv / WC, wj = wv % WC;
         for (int k = NT - 1; k >= 1; k--) {
             if (wj == k % WC) {
-                const float xk = rv[16 * k + lr];
+                float xk = rv[16 * k + lr];
+#pragma unroll
+                for (int u = 0; u < WC; u++)
+                    if (last_col(u) > k) xk -= bp[16 * (WC * (k & 1) + u) + lr];
+                if (wi == 0 && g == 0) xv[16 * k + lr] = xk;
 #pragma unroll
                 for (int tb = 0; tb < NC; tb++) {
                     if (WC * tb + wj != k) continue;
 #pragma unroll
                     for (int ta = 0; ta < NR; ta++) {
-                        const int i = WR * ta + wi;
-                        if (i >= k) continue;
-                        tile_matvec_store<true>(M[ta][tb], xk, rI + 16 * WR * ta, lane);
+                        if (WR * ta + wi >= k) continue;
+                        const bool first = k + WC >= NT;
+#pragma unroll
+                        for (int q = 0; q < 4; q++)
+                            M[ta][NC - 1][q] = first ? M[ta][tb][q] * xk : fmaf(M[ta][tb][q], xk, M[ta][NC - 1][q]);
                     }
                 }
             }
+            // row k - 1 has all its columns
+            if (wi == (k - 1) % WR && last_col(wj) >= k) {
+#pragma unroll
+                for (int ta = 0; ta < NR; ta++)
+                    if (WR * ta + wi == k - 1)
+                        tile_rowsum_store(M[ta][NC - 1], bp + 16 * (WC * ((k - 1) & 1) + wj), lane);
+            }
             __syncthreads();
         }
+    };
+    auto solution = [&](int i) __attribute__((always_inline)) {
+        if (i >= 16) return xv[i];
+        float x = rv[i];
+#pragma unroll
+        for (int u = 0; u < WC; u++)
+            if (last_col(u) > 0) x -= bp[16 * u + i];
+        return x;
     };
 
     for (;;) {
@@ -482,7 +536,7 @@ __global__ void __launch_bounds__(64 * WR * WC, WGS *WR *WC / 4)
                 assemble(yw, scale, hs);
                 factor();
                 back();
-                for (int i = t; i < N; i += T) yw[i] = fmaf(hs, rv[i], yw[i]);
+                for (int i = t; i < N; i += T) yw[i] = fmaf(hs, solution(i), yw[i]);
                 __syncthreads();
                 if (pass == 0)
                     for (int i = t; i < N; i += T) y1[i] = yw[i];
