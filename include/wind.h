@@ -219,7 +219,7 @@ enum wind_flags {
                                   lane-per-system ones).  Mass-action networks then use the LDS
                                   LU instead of the blocked MFMA solver.  Exact mode rejects it:
                                   the reference's Gauss-Jordan is unpivoted. */
-    WIND_FLAG_DENSE_LDS = 8    /* fast mode, mass-action SIE with 49 <= N <= 160: keep the matrix in
+    WIND_FLAG_DENSE_LDS = 8    /* fast mode, mass-action SIE with N <= 160: keep the matrix in
                                   LDS (one system per CU at N = 157) instead of the default
                                   register-resident solver (three or four systems per CU); results agree
                                   to rounding */

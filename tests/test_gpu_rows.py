@@ -4,6 +4,7 @@ import numpy as np
 import pytest
 
 import oracle_lib as O
+import test_gpu_trace
 from wind_amd import api
 from wind_amd import networks as W
 
@@ -82,7 +83,7 @@ def test_register_kernel_equals_oracle(N, controller):
     assert same(y, yr) and np.array_equal(steps, sr) and np.array_equal(status, tr)
 
 
-@pytest.mark.parametrize("N", [50, 80, 96, 97, 113, 129, 157])
+@pytest.mark.parametrize("N", [3, 16, 17, 33, 48, 50, 80, 96, 97, 113, 129, 157])
 def test_dense_solver_results_do_not_depend_on_the_batch(N):
     """Fast dense solver: few systems run on eight waves each, many on four; the same bits."""
     n = 560
@@ -94,6 +95,13 @@ def test_dense_solver_results_do_not_depend_on_the_batch(N):
     for m in (1, 200, 512):
         part = run(net, m, y0[:m * N], sc[:m], api.KERNEL_AUTO, **kw)
         assert same(part[0], full[0][:m * N]) and np.array_equal(part[1], full[1][:m])
+
+
+@pytest.mark.parametrize("N", [5, 16, 33, 40, 48])
+def test_dense_solver_attempts_at_few_tiles(N):
+    """Register-resident dense solver at one and three tiles per dimension: per attempt against the float
+    oracle, with the bounds of the other sizes."""
+    test_gpu_trace.test_fast_dense_attempts(N, 16, 200, 0)
 
 
 def test_row_kernel_strides_hints_and_non_finite_states():

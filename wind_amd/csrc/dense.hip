@@ -103,9 +103,15 @@ int launch_dense_reg(int num_cu, const MassActionDevice &d, const IntegrateArgs 
         default: break;
     }
     switch (NT) {
+    case 1:
+        return dense_reg_wgs_dev(d) == 8 ? launch_dense_reg_nt<1, 8>(num_cu, d, a, sc, st)
+                                         : launch_dense_reg_nt<1, 3>(num_cu, d, a, sc, st);
     case 2:
         return dense_reg_wgs_dev(d) == 8 ? launch_dense_reg_nt<2, 8>(num_cu, d, a, sc, st)
                                          : launch_dense_reg_nt<2, 3>(num_cu, d, a, sc, st);
+    case 3:
+        return dense_reg_wgs_dev(d) == 6 ? launch_dense_reg_nt<3, 6>(num_cu, d, a, sc, st)
+                                         : launch_dense_reg_nt<3, 3>(num_cu, d, a, sc, st);
     case 4:
         return dense_reg_wgs_dev(d) == 6 ? launch_dense_reg_nt<4, 6>(num_cu, d, a, sc, st)
                                          : launch_dense_reg_nt<4, 3>(num_cu, d, a, sc, st);

@@ -93,10 +93,13 @@ int launch_dense(int num_cu, const wind::MassActionDevice &d, const wind::Integr
 // Register-resident dense SIE solver (dense.hip): tiles per dimension it is
 // built for, whether it takes this network and choice (fast mode, FP32
 // tiles, no refinement, two workgroups' LDS per CU), and its launch.
-constexpr int kDenseRegMinNT = 2, kDenseRegMaxNT = 10;
-// Tiles per dimension at which the register-resident solver is used: at
-// three (33 <= N <= 48) it measured 7-10% slower than the LDS solver.
-constexpr bool dense_reg_tiles(int NT) { return NT >= kDenseRegMinNT && NT <= kDenseRegMaxNT && NT != 3; }
+constexpr int kDenseRegMinNT = 1, kDenseRegMaxNT = 10;
+// Against the LDS solver, ms for a whole batch of a mixed-size network: N = 12
+// 0.09 / 0.15 (1 system), 13.8 / 24.9 (512), 22.1 / 37.8 (4,096), 52.3 / 71.8
+// (16,384); N = 24 9.2 / 14.8, 32.7 / 53.7, 46.3 / 66.5, 104 / 125; N = 40
+// 11.0 / 18.7, 43.1 / 73.2, 75.2 / 108, 200 / 237: it is the faster one at all
+// of these sizes.
+constexpr bool dense_reg_tiles(int NT) { return NT >= kDenseRegMinNT && NT <= kDenseRegMaxNT; }
 bool dense_reg_eligible(const wind::MassActionDevice &d, const SolverChoice &sc);
 int launch_dense_reg(int num_cu, const wind::MassActionDevice &d, const wind::IntegrateArgs &a, const SolverChoice &sc,
                      hipStream_t st);
