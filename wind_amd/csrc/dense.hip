@@ -58,7 +58,7 @@ bool dense_reg_eligible(const MassActionDevice &d, const SolverChoice &sc) {
     if (sc.solver != WIND_SOLVER_AUTO && sc.solver != WIND_SOLVER_MFMA_F32) return false;
     const int NT = (d.N + 15) / 16;
     if (!dense_reg_tiles(NT)) return false;
-    // three (or four) workgroups per CU must fit, else the LDS-resident solver is the better shape
+    // three workgroups per CU must fit, else the LDS-resident solver is the better shape
     return dense_reg_wgs_dev(d) != 0;
 }
 
@@ -82,6 +82,15 @@ int launch_dense_reg_nt(int num_cu, const MassActionDevice &d, const IntegrateAr
     return WIND_OK;
 }
 
+// The four-wave build for as many workgroups per CU as fit (dense_reg_wgs_for).
+template <int NT>
+int launch_dense_reg_wgs(int num_cu, const MassActionDevice &d, const IntegrateArgs &a, const SolverChoice &sc,
+                         hipStream_t st) {
+    constexpr int want = dense_reg_wgs_want(NT);
+    return dense_reg_wgs_dev(d) == want ? launch_dense_reg_nt<NT, want>(num_cu, d, a, sc, st)
+                                        : launch_dense_reg_nt<NT, 3>(num_cu, d, a, sc, st);
+}
+
 int launch_dense_reg(int num_cu, const MassActionDevice &d, const IntegrateArgs &a, const SolverChoice &sc,
                      hipStream_t st) {
     // Few systems: eight waves each, two workgroups per CU, no register
@@ -103,26 +112,16 @@ int launch_dense_reg(int num_cu, const MassActionDevice &d, const IntegrateArgs 
         default: break;
     }
     switch (NT) {
-    case 1:
-        return dense_reg_wgs_dev(d) == 8 ? launch_dense_reg_nt<1, 8>(num_cu, d, a, sc, st)
-                                         : launch_dense_reg_nt<1, 3>(num_cu, d, a, sc, st);
-    case 2:
-        return dense_reg_wgs_dev(d) == 8 ? launch_dense_reg_nt<2, 8>(num_cu, d, a, sc, st)
-                                         : launch_dense_reg_nt<2, 3>(num_cu, d, a, sc, st);
-    case 3:
-        return dense_reg_wgs_dev(d) == 6 ? launch_dense_reg_nt<3, 6>(num_cu, d, a, sc, st)
-                                         : launch_dense_reg_nt<3, 3>(num_cu, d, a, sc, st);
-    case 4:
-        return dense_reg_wgs_dev(d) == 6 ? launch_dense_reg_nt<4, 6>(num_cu, d, a, sc, st)
-                                         : launch_dense_reg_nt<4, 3>(num_cu, d, a, sc, st);
-    case 5: return launch_dense_reg_nt<5, 3>(num_cu, d, a, sc, st);
-    case 6: return launch_dense_reg_nt<6, 3>(num_cu, d, a, sc, st);
-    case 7: return launch_dense_reg_nt<7, 3>(num_cu, d, a, sc, st);
-    case 8: return launch_dense_reg_nt<8, 3>(num_cu, d, a, sc, st);
-    case 9: return launch_dense_reg_nt<9, 3>(num_cu, d, a, sc, st);
-    case 10:
-        return dense_reg_wgs_dev(d) == 4 ? launch_dense_reg_nt<10, 4>(num_cu, d, a, sc, st)
-                                         : launch_dense_reg_nt<10, 3>(num_cu, d, a, sc, st);
+    case 1: return launch_dense_reg_wgs<1>(num_cu, d, a, sc, st);
+    case 2: return launch_dense_reg_wgs<2>(num_cu, d, a, sc, st);
+    case 3: return launch_dense_reg_wgs<3>(num_cu, d, a, sc, st);
+    case 4: return launch_dense_reg_wgs<4>(num_cu, d, a, sc, st);
+    case 5: return launch_dense_reg_wgs<5>(num_cu, d, a, sc, st);
+    case 6: return launch_dense_reg_wgs<6>(num_cu, d, a, sc, st);
+    case 7: return launch_dense_reg_wgs<7>(num_cu, d, a, sc, st);
+    case 8: return launch_dense_reg_wgs<8>(num_cu, d, a, sc, st);
+    case 9: return launch_dense_reg_wgs<9>(num_cu, d, a, sc, st);
+    case 10: return launch_dense_reg_wgs<10>(num_cu, d, a, sc, st);
     default: return wind_fail(WIND_ERR_UNSUPPORTED, "register-resident dense solver: N out of range");
     }
 }

@@ -55,16 +55,17 @@
 
 namespace wind {
 
-// Workgroups per CU (WGS) the solver is built for: three; four at ten tiles
-// per dimension (N > 144), six at three and four tiles (33 <= N <= 64) and
-// eight below when the network's LDS footprint allows it (dense_reg_wgs_for).
-// Built for more than three, the kernel reads the rate constants from
+// Workgroups per CU (WGS) the solver is built for: four from seven tiles per
+// dimension (N > 96), five at five and six, six at three and four, eight
+// below, when the network's LDS footprint allows it (dense_reg_wgs_for); else
+// three.  Built for more than three, the kernel reads the rate constants from
 // global memory instead of LDS and the compiler keeps it within 512 / WGS
-// VGPRs (at ten tiles spilling some).  Measured: N = 157 four per CU 3%
-// faster than three; N = 64 six per CU 6% faster than three (five, the
-// register-limited occupancy of the three-per-CU build); N = 40, 8,192
-// systems, 112 ms at six per CU, 119 at five and 117 in the three-per-CU
-// build.
+// VGPRs (spilling up to 38 of them).  Measured, whole batches, the
+// three-per-CU build (which may leave room for more) against this choice:
+// 2,048 systems, N = 112 270 / 249 ms, 128 364 / 320, 144 431 / 421, N = 157 3%
+// faster; 8,192 systems, N = 40 117 / 112 (five per CU 119), 80 376 / 344, 96
+// 449 / 419; 64 six per CU 193, five 209.  Where the CU is not full the builds
+// are within 2% of each other.
 
 // Assembly stream words a thread loads at a time (streams are padded to a
 // multiple of it).
@@ -615,13 +616,15 @@ inline size_t dense_reg_lds_bytes(int NT, int R, int WGS, int cap) {
     return sizeof(float) * (size_t)dense_reg_offsets(NT, R, WGS, cap).total;
 }
 
-// The workgroups per CU to build for: four at ten tiles, six at three and
-// four, and eight below when they fit the CU's LDS (max_lds bytes), else three when
-// three fit, else 0 (the solver does not apply).  cap: the network's
-// compact element buffer (floats).
+// The workgroups per CU to build for where their LDS fits.
+constexpr int dense_reg_wgs_want(int NT) { return NT >= 7 ? 4 : NT >= 5 ? 5 : NT >= 3 ? 6 : 8; }
+
+// The workgroups per CU to build for: dense_reg_wgs_want when they fit the
+// CU's LDS (max_lds bytes), else three when three fit, else 0 (the solver
+// does not apply).  cap: the network's compact element buffer (floats).
 inline int dense_reg_wgs_for(int NT, int R, int cap, size_t max_lds) {
-    const int want = NT >= 10 ? 4 : NT == 3 || NT == 4 ? 6 : NT <= 2 ? 8 : 3;
-    if (want != 3 && want * (dense_reg_lds_bytes(NT, R, want, cap) + 256) <= max_lds) return want;
+    const int want = dense_reg_wgs_want(NT);
+    if (want * (dense_reg_lds_bytes(NT, R, want, cap) + 256) <= max_lds) return want;
     return 3 * (dense_reg_lds_bytes(NT, R, 3, cap) + 256) <= max_lds ? 3 : 0;
 }
 
