@@ -97,6 +97,24 @@ def test_dense_solver_results_do_not_depend_on_the_batch(N):
         assert same(part[0], full[0][:m * N]) and np.array_equal(part[1], full[1][:m])
 
 
+@pytest.mark.parametrize("N", [50, 80, 100, 157])
+@pytest.mark.parametrize("controller", [api.CTRL_REFERENCE, api.CTRL_ADAPTIVE])
+def test_dense_hand_over_continues_each_system(N, controller):
+    """The last systems of a call go on on eight waves each: states, sub-steps, status and the sub-steps' total are
+    those of calls that never hand over, also where systems reach max_attempts."""
+    n = 600
+    net = api.Network.mass_action(N, *W.mass_action_network(N, 700 + N))
+    y0, sc = W.mass_action_systems(n, N, 7, W.MIXED_SCALE_RANGE)
+    kw = {"tend": 1e6, "tol": 1e-10, "rel": 8e-5, "mode": api.MODE_FAST, "controller": controller,
+          "max_attempts": 700}
+    y, steps, status = run(net, n, y0, sc, api.KERNEL_AUTO, **kw)
+    print(f"N={N} attempts {steps.min() // 3} .. {steps.max() // 3}", flush=True)
+    for i in range(0, n, 200):
+        part = run(net, 200, y0[i * N:(i + 200) * N], sc[i:i + 200], api.KERNEL_AUTO, **kw)
+        assert same(part[0], y[i * N:(i + 200) * N])
+        assert np.array_equal(part[1], steps[i:i + 200]) and np.array_equal(part[2], status[i:i + 200])
+
+
 @pytest.mark.parametrize("N", [5, 16, 33, 40, 48])
 def test_dense_solver_attempts_at_few_tiles(N):
     """Register-resident dense solver at one and three tiles per dimension: per attempt against the float

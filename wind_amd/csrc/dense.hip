@@ -75,7 +75,7 @@ int launch_dense_reg_nt(int num_cu, const MassActionDevice &d, const IntegrateAr
     int per_cu = 0;
     hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kfn, 64 * WR * WC, lds);
     if (e != hipSuccess) return wind_fail(WIND_ERR_DEVICE, hipGetErrorString(e));
-    const int grid = scaled_grid(num_cu, per_cu, sc, a.nsys);
+    const int grid = scaled_grid(num_cu, per_cu, sc, WR > 2 && a.spill ? a.spill_cap : a.nsys);
     hipLaunchKernelGGL(kfn, dim3(grid), dim3(64 * WR * WC), lds, st, a, d);
     e = hipGetLastError();
     if (e != hipSuccess) return wind_fail(WIND_ERR_DEVICE, hipGetErrorString(e));
@@ -91,27 +91,34 @@ int launch_dense_reg_wgs(int num_cu, const MassActionDevice &d, const IntegrateA
                                         : launch_dense_reg_nt<NT, 3>(num_cu, d, a, sc, st);
 }
 
-int launch_dense_reg(int num_cu, const MassActionDevice &d, const IntegrateArgs &a, const SolverChoice &sc,
-                     hipStream_t st) {
-    // Few systems: eight waves each, two workgroups per CU, no register
-    // spilled.  A system alone on its CU: N = 160 46.6 -> 37.0 us per
-    // sub-step, 128 29.2 -> 24.6, 96 18.4 -> 16.7, 64 10.6 -> 9.8; two per
-    // CU: 56.1 -> 50.3, 35.1 -> 33.2, 21.6 -> 21.8, 12.2 -> 12.7 (512
-    // systems to the end, N = 160 512 -> 450 ms, 128 367 -> 320, 96 159 ->
-    // 152).  With the CU full the four-wave form is the better one (N = 160
-    // 19.1 us per sub-step and CU against 25.2).
-    const int NT = (d.N + 15) / 16;
-    if (a.nsys <= num_cu * (NT >= 6 ? 2 : 1)) switch (NT) {
-        case 4: return launch_dense_reg_nt<4, 2, 4, 2>(num_cu, d, a, sc, st);
-        case 5: return launch_dense_reg_nt<5, 2, 4, 2>(num_cu, d, a, sc, st);
-        case 6: return launch_dense_reg_nt<6, 2, 4, 2>(num_cu, d, a, sc, st);
-        case 7: return launch_dense_reg_nt<7, 2, 4, 2>(num_cu, d, a, sc, st);
-        case 8: return launch_dense_reg_nt<8, 2, 4, 2>(num_cu, d, a, sc, st);
-        case 9: return launch_dense_reg_nt<9, 2, 4, 2>(num_cu, d, a, sc, st);
-        case 10: return launch_dense_reg_nt<10, 2, 4, 2>(num_cu, d, a, sc, st);
-        default: break;
+// Few systems: eight waves each, two workgroups per CU, no register
+// spilled.  A system alone on its CU: N = 160 46.6 -> 37.0 us per
+// sub-step, 128 29.2 -> 24.6, 96 18.4 -> 16.7, 64 10.6 -> 9.8; two per
+// CU: 56.1 -> 50.3, 35.1 -> 33.2, 21.6 -> 21.8, 12.2 -> 12.7 (512
+// systems to the end, N = 160 512 -> 450 ms, 128 367 -> 320, 96 159 ->
+// 152).  With the CU full the four-wave form is the better one (N = 160
+// 19.1 us per sub-step and CU against 25.2).
+//
+// The largest number of systems that the eight-wave form takes; 0: it is not built.
+static int dense_reg_few(int NT, int num_cu) { return NT >= 6 ? 2 * num_cu : NT >= 4 ? num_cu : 0; }
+
+static int launch_dense_reg_few(int num_cu, const MassActionDevice &d, const IntegrateArgs &a, const SolverChoice &sc,
+                         hipStream_t st) {
+    switch ((d.N + 15) / 16) {
+    case 4: return launch_dense_reg_nt<4, 2, 4, 2>(num_cu, d, a, sc, st);
+    case 5: return launch_dense_reg_nt<5, 2, 4, 2>(num_cu, d, a, sc, st);
+    case 6: return launch_dense_reg_nt<6, 2, 4, 2>(num_cu, d, a, sc, st);
+    case 7: return launch_dense_reg_nt<7, 2, 4, 2>(num_cu, d, a, sc, st);
+    case 8: return launch_dense_reg_nt<8, 2, 4, 2>(num_cu, d, a, sc, st);
+    case 9: return launch_dense_reg_nt<9, 2, 4, 2>(num_cu, d, a, sc, st);
+    case 10: return launch_dense_reg_nt<10, 2, 4, 2>(num_cu, d, a, sc, st);
+    default: return wind_fail(WIND_ERR_UNSUPPORTED, "register-resident dense solver: N out of range");
     }
-    switch (NT) {
+}
+
+static int launch_dense_reg_many(int num_cu, const MassActionDevice &d, const IntegrateArgs &a, const SolverChoice &sc,
+                          hipStream_t st) {
+    switch ((d.N + 15) / 16) {
     case 1: return launch_dense_reg_wgs<1>(num_cu, d, a, sc, st);
     case 2: return launch_dense_reg_wgs<2>(num_cu, d, a, sc, st);
     case 3: return launch_dense_reg_wgs<3>(num_cu, d, a, sc, st);
@@ -124,4 +131,25 @@ int launch_dense_reg(int num_cu, const MassActionDevice &d, const IntegrateArgs 
     case 10: return launch_dense_reg_wgs<10>(num_cu, d, a, sc, st);
     default: return wind_fail(WIND_ERR_UNSUPPORTED, "register-resident dense solver: N out of range");
     }
+}
+
+int dense_reg_hand_cap(const wind_network *net, const wind_options &o, const SolverChoice &sc, int nsys, int num_cu) {
+    if (net->builtin != WIND_NET_MASS_ACTION || o.mode != WIND_MODE_FAST || o.method != WIND_SIE || o.trace) return 0;
+    const int few = dense_reg_few((net->N + 15) / 16, num_cu);
+    return nsys > few && dense_reg_eligible(net->ma, sc) ? few : 0;
+}
+
+// More systems than that: four waves each until no more than that are
+// unfinished; where the caller has a list for them (a.spill), those go on
+// on eight waves each, spread over the CUs again (a system's last attempts
+// otherwise run at the pace that its CU's other long systems leave it).
+// Whole batches, ms, handed over never / at 128 / 256 / 384 / 512 / 768 unfinished:
+// N = 157, 1,021 systems, 354 / 334 / 327 / 322 / 308 / 310; 112, 2,000, 221 /
+// 215 / 211 / 211 / 206 / 211; 64, 4,099, 113 / 109 / 106 / 107 / 105 / 109; 80,
+// 1,500, 105 / 103 / 105 / 101 / 101 / 102.
+int launch_dense_reg(int num_cu, const MassActionDevice &d, const IntegrateArgs &a, const SolverChoice &sc,
+                     hipStream_t st) {
+    if (a.nsys <= dense_reg_few((d.N + 15) / 16, num_cu)) return launch_dense_reg_few(num_cu, d, a, sc, st);
+    const int rc = launch_dense_reg_many(num_cu, d, a, sc, st);
+    return rc || !a.spill ? rc : launch_dense_reg_few(num_cu, d, a, sc, st);
 }

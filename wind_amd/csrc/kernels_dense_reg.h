@@ -216,7 +216,8 @@ __global__ void __launch_bounds__(64 * WR * WC, WGS *WR *WC / 4)
         ab[r] = make_int2(net.rx[4 * r], net.rx[4 * r + 1]);
         if (WGS == 3) kk[r] = net.k[r];
     }
-    __shared__ int s_flag, s_sid;
+    __shared__ int s_flag, s_sid, s_rec;
+    __shared__ int s_done;
     __shared__ double s_err[WR * WC];
     f32x4 M[NR][NC];
     unsigned long long steps = 0;
@@ -505,10 +506,18 @@ __global__ void __launch_bounds__(64 * WR * WC, WGS *WR *WC / 4)
         return x;
     };
 
+    unsigned *const words = reinterpret_cast<unsigned *>(a.counters);
+    float *const hand = TRACE || NT < 4 ? nullptr : a.spill;  // (built from four tiles)
     for (;;) {
         if (t == 0) {
-            const unsigned q = atomicAdd(head, 1u);
-            s_sid = q < (unsigned)a.nsys ? (a.index ? a.index[q] : (int)q) : a.nsys;
+            if (WR > 2 && hand) {
+                const unsigned q = atomicAdd(words + DENSE_TAIL_HEAD, 1u);
+                s_rec = (int)q;
+                s_sid = q < words[DENSE_HANDED] ? __float_as_int(hand[(size_t)q * kDenseHandWords]) : a.nsys;
+            } else {
+                const unsigned q = atomicAdd(head, 1u);
+                s_sid = q < (unsigned)a.nsys ? (a.index ? a.index[q] : (int)q) : a.nsys;
+            }
         }
         __syncthreads();
         const int sid = __builtin_amdgcn_readfirstlane(s_sid);
@@ -518,6 +527,14 @@ __global__ void __launch_bounds__(64 * WR * WC, WGS *WR *WC / 4)
         __syncthreads();
         float tnow = a.tnow, h = a.h0;
         int unsolved = 0, attempts = 0, status = WIND_STATUS_OK;
+        bool handed = false;
+        if (WR > 2 && hand) {
+            const float *r = hand + (size_t)__builtin_amdgcn_readfirstlane(s_rec) * kDenseHandWords;
+            tnow = uniform(r[1]);
+            h = uniform(r[2]);
+            unsolved = __builtin_amdgcn_readfirstlane(__float_as_int(r[3]));
+            attempts = __builtin_amdgcn_readfirstlane(__float_as_int(r[4]));
+        }
         const bool replay = TRACE && a.trace.h != nullptr;
         const int rcount = replay ? min(a.trace.count[sid], a.trace.capacity) : 0;
         while (replay ? attempts < rcount : tnow < a.tend) {
@@ -543,7 +560,13 @@ __global__ void __launch_bounds__(64 * WR * WC, WGS *WR *WC / 4)
                 if (pass == 0)
                     for (int i = t; i < N; i += T) y1[i] = yw[i];
             }
-            if (t == 0) s_flag = 0;
+            // every eighth attempt: how many systems are finished (the read's
+            // latency would show if it were every one)
+            const bool look = WR == 2 && hand && (attempts & 7) == 7;
+            if (t == 0) {
+                s_flag = 0;
+                if (look) s_done = (int)__hip_atomic_load(words + DENSE_DONE, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
             __syncthreads();
             bool flag = false;
             double err = 0.0;
@@ -598,10 +621,28 @@ __global__ void __launch_bounds__(64 * WR * WC, WGS *WR *WC / 4)
                 status = WIND_STATUS_EXHAUSTED;
                 break;
             }
+            if (look && tnow < a.tend &&
+                a.nsys - __builtin_amdgcn_readfirstlane(s_done) <= a.spill_cap) {
+                handed = true;
+                break;
+            }
         }
         __syncthreads();
         for (int i = t; i < N; i += T) a.equations[(size_t)sid * N + i] = y[i];
-        if (t == 0) {
+        if (WR == 2 && hand && t == 0) {
+            if (handed) {
+                // at most spill_cap systems are unfinished, so the list holds them
+                float *r = hand + (size_t)atomicAdd(words + DENSE_HANDED, 1u) * kDenseHandWords;
+                r[0] = __int_as_float(sid);
+                r[1] = tnow;
+                r[2] = h;
+                r[3] = __int_as_float(unsolved);
+                r[4] = __int_as_float(attempts);
+            } else {
+                atomicAdd(words + DENSE_DONE, 1u);
+            }
+        }
+        if (t == 0 && !handed) {
             if (a.steps_out) a.steps_out[sid] = 3 * attempts;
             if (a.status_out) a.status_out[sid] = status;
             steps += 3ull * (unsigned long long)attempts;

@@ -994,6 +994,11 @@ int wind_integrate(const wind_network *net, float tnow, float tend, int n_integr
         if (rc) return rc;
         a.spill = (float *)sl->spill.ptr;
         a.spill_index = (int32_t *)(a.spill + words);
+    } else if (const int cap = dense_reg_hand_cap(net, opts, sc, Nsystems, c.num_cu)) {
+        rc = reserve(sl->spill, sizeof(float) * kDenseHandWords * (size_t)cap);
+        if (rc) return rc;
+        a.spill = (float *)sl->spill.ptr;
+        a.spill_cap = cap;
     }
     std::vector<TraceCopy> trace_back;
     if (opts.trace) {

@@ -101,6 +101,9 @@ constexpr int kDenseRegMinNT = 1, kDenseRegMaxNT = 10;
 // of these sizes.
 constexpr bool dense_reg_tiles(int NT) { return NT >= kDenseRegMinNT && NT <= kDenseRegMaxNT; }
 bool dense_reg_eligible(const wind::MassActionDevice &d, const SolverChoice &sc);
+// Systems that this call's last part may hand over (IntegrateArgs::spill of
+// kDenseHandWords words each); 0: it does not.
+int dense_reg_hand_cap(const wind_network *net, const wind_options &o, const SolverChoice &sc, int nsys, int num_cu);
 int launch_dense_reg(int num_cu, const wind::MassActionDevice &d, const wind::IntegrateArgs &a, const SolverChoice &sc,
                      hipStream_t st);
 

@@ -55,7 +55,11 @@ struct IntegrateArgs {
     // them, packed into full waves again, and hands its own last ones over in
     // the second list, behind the first.  The row kernel takes the last list.
     // The lists' lengths and queue heads are 32-bit words of counters
-    // (spill_word).
+    // (SpillWord).
+    // The register dense solver (kernels_dense_reg.h) with spill set: its
+    // four-wave form hands over when at most spill_cap systems are
+    // unfinished, the state in place in equations, the rest as a record of
+    // kDenseHandWords words, and the eight-wave form continues them.
     float *spill = nullptr;
     int32_t *spill_index = nullptr;  // the row kernel's start order, [spill_cap]
     int32_t spill_at = 0, spill_cap = 0, spill_pack = 0;
@@ -65,6 +69,14 @@ struct IntegrateArgs {
 // two lists, and the heads of the second lane pass's and the row kernel's
 // queues.
 enum SpillWord { SPILL_FIRST = 4, SPILL_SECOND = 5, SPILL_ROW_HEAD = 6, SPILL_LANE_HEAD = 7 };
+
+// The same words for the dense solver's hand-over: length of the list, head of
+// the eight-wave form's queue, systems finished in the four-wave form.
+enum DenseHandWord { DENSE_HANDED = 4, DENSE_TAIL_HEAD = 5, DENSE_DONE = 6 };
+
+// Words per system the dense solver hands over: id, tnow, h, refinements in a
+// row, attempts (the rest unused).
+constexpr int kDenseHandWords = 8;
 
 // Floats per packed record: state, constants and the system id, rounded up
 // to whole 32-byte sectors.
