@@ -3,13 +3,17 @@
 // from a generated network header and plugin_impl.h; it exports
 // wind_plugin_get(), which returns a static descriptor.  Core and plugins are
 // built from the same sources, so IntegrateArgs crosses the boundary as is;
-// WIND_PLUGIN_ABI guards against mixing builds.
+// WIND_PLUGIN_ABI guards against mixing builds.  IntegrateArgs has grown at
+// its end since ABI 4: a plugin built before reads the part it knows and
+// runs without the rest, and a core of that time passes only that part,
+// so a plugin takes the members from `spill` on only from a core that has
+// told it how many bytes it passes (wind_plugin_args, optional).
 #pragma once
 #include <hip/hip_runtime.h>
 
 #include "wind_types.h"
 
-#define WIND_PLUGIN_ABI 6
+#define WIND_PLUGIN_ABI 4
 
 struct wind_plugin_desc {
     int abi;          // WIND_PLUGIN_ABI
@@ -34,3 +38,4 @@ struct wind_plugin_desc {
 };
 
 typedef const wind_plugin_desc *(*wind_plugin_get_fn)(void);
+typedef void (*wind_plugin_args_fn)(size_t bytes);

@@ -7,6 +7,10 @@
 // mode and lockstep kernels, the descriptor; no FMA contraction) and
 // WIND_PLUGIN_PART=2 (the fast-mode kernels, with FMA contraction).
 #pragma once
+#include <atomic>
+#include <cstddef>
+#include <cstring>
+
 #include "kernels_generated.h"
 #include "kernels_lockstep.h"
 #include "kernels_small.h"
@@ -114,14 +118,20 @@ int plugin_launch_method(const IntegrateArgs &a, int mode, int kernel, int num_c
     return WIND_ERR_UNSUPPORTED;
 }
 
+// Bytes of IntegrateArgs that the core passes: those of ABI 4's first form
+// until the core names more (wind_plugin_args).
+static std::atomic<size_t> g_args_bytes{offsetof(IntegrateArgs, spill)};
+
 template <class Net>
-int plugin_launch(const IntegrateArgs *a, int method, int mode, int kernel, int num_cu, float share, int grid,
+int plugin_launch(const IntegrateArgs *args, int method, int mode, int kernel, int num_cu, float share, int grid,
                   float *scratch, size_t sbytes, hipStream_t st) {
-    if (a->trace.capacity > 0) return WIND_ERR_UNSUPPORTED;  // no traced kernels in plugins
+    IntegrateArgs a;
+    std::memcpy(&a, args, g_args_bytes.load());
+    if (a.trace.capacity > 0) return WIND_ERR_UNSUPPORTED;  // no traced kernels in plugins
     if (method == WIND_SIE)
-        return plugin_launch_method<Net, WIND_SIE>(*a, mode, kernel, num_cu, share, grid, scratch, sbytes, st);
+        return plugin_launch_method<Net, WIND_SIE>(a, mode, kernel, num_cu, share, grid, scratch, sbytes, st);
     if (method == WIND_RK2)
-        return plugin_launch_method<Net, WIND_RK2>(*a, mode, kernel, num_cu, share, grid, scratch, sbytes, st);
+        return plugin_launch_method<Net, WIND_RK2>(a, mode, kernel, num_cu, share, grid, scratch, sbytes, st);
     return WIND_ERR_ARGUMENT;
 }
 
@@ -189,6 +199,9 @@ int plugin_scratch_fast(int nsys, int method, int kernel, int num_cu, float shar
 
 #if WIND_PLUGIN_PART == 1
 #define WIND_DEFINE_PLUGIN(NET, NAME, NREACT, FLOPS_RHS, FLOPS_JAC)                                      \
+    extern "C" __attribute__((visibility("default"))) void wind_plugin_args(size_t bytes) {               \
+        wind::g_args_bytes = bytes < sizeof(wind::IntegrateArgs) ? bytes : sizeof(wind::IntegrateArgs);   \
+    }                                                                                                      \
     extern "C" __attribute__((visibility("default"))) const wind_plugin_desc *wind_plugin_get(void) {     \
         static const wind_plugin_desc d = {WIND_PLUGIN_ABI,       NET::N,                                  \
                                            NET::NCONST,           NREACT,                                  \

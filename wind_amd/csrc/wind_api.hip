@@ -625,6 +625,7 @@ int wind_network_create_plugin(const char *path, wind_network **out) {
         dlclose(dl);
         return fail(WIND_ERR_ARGUMENT, "not a network plugin of this library version");
     }
+    if (auto args = (wind_plugin_args_fn)dlsym(dl, "wind_plugin_args")) args(sizeof(IntegrateArgs));
     wind_network *n = new wind_network();
     n->builtin = WIND_NET_PLUGIN;
     n->N = d->N;
