@@ -65,6 +65,24 @@ def test_tail_on_rows_equals_lane_kernel(name, n, method, controller):
     assert same(a[0], b[0]) and np.array_equal(a[1], b[1]) and np.array_equal(a[2], b[2])
 
 
+@pytest.mark.parametrize("name", list(NETS))
+@pytest.mark.parametrize("method", [api.SIE, api.RK2])
+def test_lanes_without_a_system_change_nothing(name, method):
+    """Fast lane kernel: lanes that repeat another lane's system once the queue is empty store nothing; each
+    system's state, sub-steps and status are those of the whole call, also where systems reach max_attempts."""
+    make, systems, kw = NETS[name]
+    net, n = make(), 300
+    y0, c = systems(n)
+    N, NC = len(y0) // n, np.size(c) // n
+    kw = {**kw, "mode": api.MODE_FAST, "controller": api.CTRL_ADAPTIVE, "max_attempts": 150}
+    y, steps, status = run(net, n, y0, c, api.KERNEL_AUTO, method=method, **kw)
+    flat = np.ravel(c)
+    for a, b in ((0, 1), (1, 4), (4, 68), (68, 133), (133, 300)):
+        part = run(net, b - a, y0[a * N:b * N], flat[a * NC:b * NC], api.KERNEL_AUTO, method=method, **kw)
+        assert same(part[0], y[a * N:b * N])
+        assert np.array_equal(part[1], steps[a:b]) and np.array_equal(part[2], status[a:b])
+
+
 @pytest.mark.parametrize("N", [1, 2, 7, 8, 9, 16, 31, 33, 40, 41, 55, 57, 63, 64])
 @pytest.mark.parametrize("controller", [api.CTRL_REFERENCE, api.CTRL_ADAPTIVE])
 def test_register_kernel_equals_oracle(N, controller):
