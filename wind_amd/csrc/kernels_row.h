@@ -366,6 +366,13 @@ constexpr int row_tail_per_cu(int method) { return method == WIND_SIE ? 1 : 2; }
 // Threads that give each of nsys systems a row.
 inline int row_threads(int nsys) { return 16 * (nsys < (1 << 26) ? nsys : 1 << 26); }
 
+// v = lane src's value where take is set.
+template <class T>
+__device__ inline void row_take(bool take, int src, T &v) {
+    const T x = __shfl(v, src);
+    v = take ? x : v;
+}
+
 // One system per row, four per wave, taken from the device queue; or (TAIL)
 // the systems that the lane kernel before it handed over (a.spill).
 template <class Net, int METHOD, bool TAIL = false>
@@ -381,7 +388,11 @@ __global__ void __launch_bounds__(256) row_integrate(IntegrateArgs a, typename N
     RowEval<Net, MathExact> ev(p, li);
     float y[N], c[NC > 0 ? NC : 1], yo = 0.0f, tnow = 0.0f, h = 0.0f;
     int sid = 0, unsolved = 0, attempts = 0, status = WIND_STATUS_OK;
-    bool active = false, need = true;
+    // fill: the queue is empty and the row repeats another row's system,
+    // storing nothing: a wave with idle lanes runs slower (lane_integrate_body).
+    // hhe6 SIE 100,003 systems, reference controller, 136 -> 127 ms; Katz96, 80
+    // systems, 263 -> 238 us; NR_test, 1,024, 121 -> 114 us.
+    bool active = false, need = true, fill = false;
     unsigned long long steps = 0;
     // The first system of a row is its own index in the grid; the queue
     // counts on from there, and is not asked where it is empty (its atomics
@@ -419,9 +430,24 @@ __global__ void __launch_bounds__(256) row_integrate(IntegrateArgs a, typename N
                     for (int k = 0; k < NC; k++) c[k] = a.constants[(size_t)sid * a.const_stride + k];
                 }
             }
-            if (!__any(active)) break;
+            const unsigned long long busy = __ballot(active);
+            if (busy == 0ull) break;
+            if (__ballot(active || fill) != ~0ull) {
+                const int src = (__ffsll((long long)busy) - 1) + li;  // the lane's counterpart in the first active row
+                const bool take = !active && !fill;
+                row_take(take, src, yo);
+#pragma unroll
+                for (int i = 0; i < N; i++) row_take(take, src, y[i]);
+#pragma unroll
+                for (int k = 0; k < NC; k++) row_take(take, src, c[k]);
+                row_take(take, src, tnow);
+                row_take(take, src, h);
+                row_take(take, src, unsolved);
+                row_take(take, src, attempts);
+                if (take) status = WIND_STATUS_OK;
+                fill = fill || take;
+            }
         }
-        if (!active) continue;
         const float hh = fminf(a.tend - tnow, h);
         const float tb = tnow + hh;
         const float hs1 = tb - tnow, hs2 = (tb - tnow) / 2.0f;
@@ -447,13 +473,14 @@ __global__ void __launch_bounds__(256) row_integrate(IntegrateArgs a, typename N
             if (attempts < a.max_attempts) continue;
             status = WIND_STATUS_EXHAUSTED;
         }
-        if (mine) a.equations[(size_t)sid * N + li] = yo;
-        if (li == 0) {
+        if (active && mine) a.equations[(size_t)sid * N + li] = yo;
+        if (active && li == 0) {
             if (a.steps_out) a.steps_out[sid] = 3 * attempts;
             if (a.status_out) a.status_out[sid] = status;
             steps += 3ull * (unsigned long long)attempts;
         }
-        active = false;
+        // (a row without a system asks again too, to take another to repeat)
+        active = fill = false;
         need = true;
     }
     wave_add_steps(a.counters + 1, steps);
