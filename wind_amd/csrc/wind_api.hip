@@ -269,7 +269,7 @@ int order_by_hint(Pool &order, const int32_t *d_hint, int n, hipStream_t st, con
 
 bool queue_kernel(const wind_network *net, const wind_options &o) { return wind_queue_kernel(net, o.mode, o.kernel); }
 
-// Batches at least this large start in the order of an initial-state work
+// Calls at least this large start in the order of a work
 // estimate when the caller gives no hints (fast mode, compiled-in
 // networks): the persistent fast lane grid holds 2 x 256 x 256 systems at
 // once, and smaller batches start every system immediately.
@@ -306,7 +306,8 @@ int activity_hints(int num_cu, const wind_network *net, const IntegrateArgs &a, 
 // a third of the time.  hhe6 SIE, reference controller, 20,000 (t = 1 Myr) /
 // 100,003 (1 Myr) / 1,000,003 systems (10^4 yr): 391 / 475 / 634 ms without
 // hand-over; at 24 / 32 / 40 lanes 77 / 88 / 81, 154 / 137 / 135 and 292 / 276 /
-// 279; at 32 without the second pass 74 / 143 / 357.  katz96 200,000 2.92 ms
+// 279; at 32 without the second pass 74 / 143 / 357 (all before the row kernel's
+// idle rows repeated a neighbour's system: 137 -> 127 at 40).  katz96 200,000 2.92 ms
 // without, 2.11 at 40, 2.88 at 32 without the second pass; NR_test (N = 2)
 // 200,000 0.50 without, 0.52 to 0.89 with, so only systems of five equations
 // on do it.
