@@ -1,0 +1,71 @@
+"""wind_integrate's host code on a HIP runtime without a device (fake_hip.cpp)."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+CHILD = r"""
+import ctypes as C, sys
+import numpy as np
+fake = C.CDLL(sys.argv[1], C.RTLD_GLOBAL)
+sys.path.insert(0, sys.argv[2])
+from wind_amd import api
+from wind_amd import networks as W
+
+lib = api.load()
+
+
+def call(net, n, stream, kernel=api.KERNEL_AUTO, mode=api.MODE_EXACT, outputs=True):
+    y, c = W.hhe6_systems(n, 1)
+    before = y.copy()
+    out = [np.zeros(n, np.int32) for _ in range(2)] if outputs else [None, None]
+    o = api.WindOptions()
+    lib.wind_options_init(C.byref(o))
+    o.mode, o.kernel, o.stream = mode, kernel, stream
+    if outputs:
+        o.steps_out, o.status_out = (a.ctypes.data for a in out)
+    rc = lib.wind_integrate(net.handle, 0.0, 1.0, 1, c.ctypes.data, y.ctypes.data, n, 6, 1e-3, 1e-3, C.byref(o))
+    return rc, fake.fake_pending(), np.array_equal(y, before)
+
+
+net = api.Network.builtin(api.NET_HHE6, W.hhe6_params())
+"""
+
+
+@pytest.fixture(scope="module")
+def fake(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("fake") / "libfake_hip.so")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-fPIC", "-shared", "-I/opt/rocm/include", "-Wno-return-type",
+                    os.path.join(ROOT, "tests", "fake_hip.cpp"), "-o", so], check=True)
+    return so
+
+
+def child(fake, body, *args):
+    r = subprocess.run([sys.executable, "-c", CHILD + body, fake, ROOT, *map(str, args)], capture_output=True, text=True)
+    assert r.returncode == 0, r.stdout + r.stderr
+
+
+@pytest.mark.parametrize("n", [300, 5000, 60000])  # one pinned copy each way; the same with a hand-over list; arrays one by one
+@pytest.mark.parametrize("what", ["none", "block", "hipGetLastError", "hipMalloc", "hipMemcpyAsync"])
+def test_a_call_leaves_nothing_queued(fake, n, what):
+    """Also where it fails after it has queued copies: the next call may take its buffers."""
+    child(fake, r"""
+what, n = sys.argv[3], int(sys.argv[4])
+seen = 0
+for k in range(1, 12):  # (each call of the function in turn, until none is left to fail)
+    kw = {"kernel": api.KERNEL_BLOCK, "mode": api.MODE_FAST} if what == "block" else {}
+    if what.startswith("hip"):
+        if what == "hipMalloc":  # the pools keep what they have: grow them
+            n += 1000 if n > 50000 else 0
+        fake.fake_fail(what.encode(), k)
+    rc, pending, same = call(net, n, 0x1000 * k, **kw)
+    fake.fake_fail(what.encode(), 0)
+    assert pending == 0, (what, k, pending)
+    assert same
+    assert rc == 0 or what != "none"
+    seen += rc != 0
+assert (seen > 0) == (what != "none")
+""", what, n)

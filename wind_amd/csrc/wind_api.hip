@@ -242,6 +242,17 @@ struct SlotGuard {
     }
 };
 
+// A call that returns early waits for what it has queued: its copies read and
+// write the slot's pinned image, the caller's arrays and this frame, which
+// others may use as soon as the slot is free.
+struct StreamDrain {
+    hipStream_t st;
+    bool done = false;  // the stream has been synchronised
+    ~StreamDrain() {
+        if (!done) (void)hipStreamSynchronize(st);
+    }
+};
+
 int reserve(Pool &p, size_t bytes) {
     if (bytes <= p.bytes) return WIND_OK;
     if (p.ptr) WIND_HIP(hipFree(p.ptr));
@@ -874,6 +885,7 @@ int wind_integrate(const wind_network *net, float tnow, float tend, int n_integr
     std::unique_lock<std::mutex> scratch_lock(g_scratch_mu, std::defer_lock);
     if (scratch_need) scratch_lock.lock();
     hipStream_t st = opts.stream ? (hipStream_t)opts.stream : sl->stream;
+    StreamDrain drain{st};
 
     const size_t eq_bytes = (size_t)Nsystems * Neqn * sizeof(float);
     // Reads of constants reach (Nsystems - 1) * stride + nconst floats.
@@ -1017,6 +1029,7 @@ int wind_integrate(const wind_network *net, float tnow, float tend, int n_integr
         char *h = (char *)sl->host;
         WIND_HIP(hipMemcpyAsync(h + at_cnt, (char *)sl->io.ptr + at_cnt, at_end - at_cnt, hipMemcpyDeviceToHost, st));
         WIND_HIP(hipStreamSynchronize(st));
+        drain.done = true;
         std::memcpy(equations, h + at_eq, eq_bytes);
         if (opts.steps_out) std::memcpy(opts.steps_out, h + at_steps, n4);
         if (opts.status_out) std::memcpy(opts.status_out, h + at_status, n4);
@@ -1038,6 +1051,7 @@ int wind_integrate(const wind_network *net, float tnow, float tend, int n_integr
                                     hipMemcpyDeviceToHost, st));
     }
     WIND_HIP(hipStreamSynchronize(st));
+    drain.done = true;
     if (opts.kernel_ms) WIND_HIP(hipEventElapsedTime(opts.kernel_ms, sl->ev0, sl->ev1));
     if (opts.total_steps) *opts.total_steps = (int64_t)total;
     return WIND_OK;
