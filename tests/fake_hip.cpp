@@ -13,6 +13,9 @@
 
 static std::map<hipStream_t, std::vector<std::function<void()>>> g_queue;
 static std::map<std::string, int> g_fail;
+static std::map<const void *, std::string> g_kernel;  // device function names
+static std::string g_static_name;                     // kernels with this in their name use g_static bytes of LDS
+static int g_static = 0, g_max_lds = 163840;
 
 static bool fails(const char *name) {
     auto it = g_fail.find(name);
@@ -31,11 +34,18 @@ int fake_pending() {
     return n;
 }
 void fake_fail(const char *name, int n) { g_fail[name] = n; }
+void fake_lds(int max_lds, const char *kernel, int bytes) {
+    g_max_lds = max_lds;
+    g_static_name = kernel;
+    g_static = bytes;
+}
 
 void **__hipRegisterFatBinary(const void *) { return (void **)calloc(1, sizeof(void *)); }
 void __hipUnregisterFatBinary(void **) {}
-void __hipRegisterFunction(void **, const void *, char *, const char *, unsigned, void *, void *, void *, void *,
-                           int *) {}
+void __hipRegisterFunction(void **, const void *host, char *, const char *name, unsigned, void *, void *, void *,
+                           void *, int *) {
+    g_kernel[host] = name;
+}
 void __hipRegisterVar(void **, void *, char *, char *, int, size_t, int, int) {}
 static struct { dim3 grid, block; size_t lds; hipStream_t st; } g_config;
 hipError_t __hipPushCallConfiguration(dim3 grid, dim3 block, size_t lds, hipStream_t st) {
@@ -62,7 +72,12 @@ hipError_t hipGetDevicePropertiesR0600(hipDeviceProp_tR0600 *p, int) {
     return hipSuccess;
 }
 hipError_t hipDeviceGetAttribute(int *v, hipDeviceAttribute_t, int) {
-    *v = 163840;
+    *v = g_max_lds;
+    return hipSuccess;
+}
+hipError_t hipFuncGetAttributes(hipFuncAttributes *a, const void *k) {
+    std::memset(a, 0, sizeof(*a));
+    a->sharedSizeBytes = g_kernel[k].find(g_static_name) != std::string::npos ? g_static : 0;
     return hipSuccess;
 }
 hipError_t hipOccupancyMaxActiveBlocksPerMultiprocessor(int *n, const void *, int, size_t) {

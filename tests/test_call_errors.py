@@ -69,3 +69,31 @@ for k in range(1, 12):  # (each call of the function in turn, until none is left
     seen += rc != 0
 assert (seen > 0) == (what != "none")
 """, what, n)
+
+
+def test_tile_kernel_matrices_leave_room_for_its_own_lds(fake):
+    """The dense fallback's matrices go to LDS only where they fit beside what the kernel declares itself."""
+    child(fake, r"""
+import os
+N, nc, own = 100, 10, 600  # katz96_t20; a kernel's declared LDS
+need = 4 * (5 * N + 12 + 2 * N * N) + own
+p = C.CDLL(os.path.join(api._HERE, "lib", "gen", "katz96_t20", "libwind_net.so"))
+
+
+class Desc(C.Structure):
+    _fields_ = [("abi", C.c_int), ("N", C.c_int), ("nconst", C.c_int), ("nreactions", C.c_int), ("name", C.c_char_p),
+                ("flops_rhs", C.c_longlong), ("flops_jac", C.c_longlong), ("launch", C.c_void_p),
+                ("lockstep", C.c_void_p),
+                ("scratch", C.CFUNCTYPE(C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, C.c_float, C.c_int,
+                                        C.POINTER(C.c_size_t)))]
+
+
+p.wind_plugin_get.restype = C.POINTER(Desc)
+d = p.wind_plugin_get().contents
+assert (d.N, d.nconst) == (N, nc)
+for limit in (need - own + 256, need - 1, need, need + 1000):
+    fake.fake_lds(limit, b"gen_tile_integrate", own)
+    b = C.c_size_t()
+    assert d.scratch(80, api.SIE, api.MODE_EXACT, api.KERNEL_AUTO, 256, 0.0, 0, C.byref(b)) == 0
+    assert (b.value == 0) == (limit >= need), (limit, need, b.value)
+""")

@@ -124,7 +124,9 @@ inline int gen_block_shape(int nsys, int num_cu, float share, int grid_cap, GenB
     const size_t base = sizeof(float) * (size_t)gen_block_base_floats<Net>();
     const size_t mats = sizeof(float) * (FAST ? 1 : 2) * (size_t)N * N;
     auto kfn = gen_block_kernel<Net, METHOD, FAST, PIVOT>(nsys, num_cu, &s->T);
-    s->in_lds = base + mats + 256 <= (size_t)max_lds;
+    hipFuncAttributes own;  // what the kernel declares itself (the tile kernel: 0.2 to 0.6 KB)
+    if (hipFuncGetAttributes(&own, (const void *)kfn) != hipSuccess) return WIND_ERR_DEVICE;
+    s->in_lds = base + mats + own.sharedSizeBytes <= (size_t)max_lds;
     s->lds = base + (s->in_lds ? mats : 0);
     if (s->lds > 65536 &&
         hipFuncSetAttribute((const void *)kfn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)s->lds) != hipSuccess)
