@@ -47,12 +47,14 @@ __device__ inline void row_gather(float v, float (&out)[N]) {
     static_for<0, N>([&](auto i) { out[i] = row_get<i>(v); });
 }
 
-// v[i] with i the lane's index (selects: registers cannot be indexed).
+// v[i] with i the lane's index (selects: registers cannot be indexed.  Constant
+// indices from the start: of a loop over v the compiler made a load by index,
+// v went to LDS by thread, and the workgroup's sizes for that came from the
+// launch packet in host memory, 10 us at the start of every RK2 kernel).
 template <int N>
 __device__ inline float lane_pick(const float (&v)[N], int li) {
     float r = v[0];
-#pragma unroll
-    for (int i = 1; i < N; i++) r = li == i ? v[i] : r;
+    static_for<1, N>([&](auto i) { r = li == i ? v[i] : r; });
     return r;
 }
 
