@@ -279,7 +279,8 @@ __device__ inline bool attempt(const typename Net::Params &p, const IntegrateArg
     double err = 0.0;
     if (a.controller == WIND_CTRL_REFERENCE) {
 #pragma unroll
-        for (int i = 0; i < N; i++) flag = flag || species_fails<METHOD, !M::kFast>(y1[i], y2[i], a.ABS, a.REL);
+        for (int i = 0; i < N; i++)
+            flag = flag || species_fails<METHOD, !M::kFast && METHOD == WIND_SIE>(y1[i], y2[i], a.ABS, a.REL);
     } else if constexpr (M::kFast) {
         err = err_norm_fast<N>(y1, y2, a.ABS, a.REL);
     } else {
