@@ -65,6 +65,44 @@ def test_tail_on_rows_equals_lane_kernel(name, n, method, controller):
     assert same(a[0], b[0]) and np.array_equal(a[1], b[1]) and np.array_equal(a[2], b[2])
 
 
+def num_cu():
+    return pytest.importorskip("torch").cuda.get_device_properties(0).multi_processor_count
+
+
+@pytest.mark.parametrize("name,per_cu,method,controller,cap,tol,hints", [
+    ("hhe6", 17, api.SIE, api.CTRL_REFERENCE, 700, 1e-3, False),
+    ("hhe6", 300, api.SIE, api.CTRL_REFERENCE, 700, 1e-3, False),
+    ("hhe6", 300, api.SIE, api.CTRL_REFERENCE, 700, 1e-3, True),
+    ("hhe6", 40, api.RK2, api.CTRL_REFERENCE, 1200, 1e-3, False),
+    ("hhe6", 300, api.RK2, api.CTRL_ADAPTIVE, 1200, 1e-3, False),
+    ("katz96", 300, api.SIE, api.CTRL_REFERENCE, 700, 1e-5, True),
+    ("mixed5", 9, api.SIE, api.CTRL_ADAPTIVE, 700, 1e-6, False),
+    ("mixed5", 300, api.SIE, api.CTRL_ADAPTIVE, 700, 1e-6, False),
+    ("mixed5", 1400, api.SIE, api.CTRL_REFERENCE, 700, 1e-3, False)])
+def test_long_systems_are_handed_over(name, per_cu, method, controller, cap, tol, hints):
+    """One system in 50 goes on to the attempt cap, far beyond the attempts after which a wave may hand over, the
+    others end soon: the second lane pass and the rows take the long ones over, in index order and in another start
+    order, and also where the queue feeds lanes twice.  The same bits as the lane kernel alone."""
+    make, systems, kw = NETS[name]
+    net, n = make(), per_cu * num_cu() + 3
+    y0, c = systems(n)
+    N, NC = len(y0) // n, np.size(c) // n
+    c = np.ravel(c).reshape(n, NC).copy()
+    kw = dict(kw, method=method, controller=controller, max_attempts=cap, tol=tol)
+    steps = run(net, n, y0, c.ravel(), api.KERNEL_LANE, **kw)[1]
+    order = np.argsort(steps, kind="stable")
+    long, short = order[-(n // 50 + 1):], order[:n // 2]
+    pick = np.resize(short, n)
+    pick[np.random.default_rng(1).permutation(n)[:n // 50]] = np.resize(long, n // 50)
+    y0, c = y0.reshape(n, N)[pick].ravel(), c[pick].ravel()
+    if hints:
+        kw["cost_hint"] = steps[pick].astype(np.int32)
+    a, b = (run(net, n, y0, c, k, **kw) for k in (api.KERNEL_LANE, api.KERNEL_AUTO))
+    print(f"{name} n={n}: attempts {np.percentile(a[1] // 3, [0, 50, 97, 98.5, 100])}", flush=True)
+    assert np.percentile(a[1] // 3, 98.5) >= 128
+    assert same(a[0], b[0]) and np.array_equal(a[1], b[1]) and np.array_equal(a[2], b[2])
+
+
 @pytest.mark.parametrize("name", list(NETS))
 @pytest.mark.parametrize("method", [api.SIE, api.RK2])
 def test_lanes_without_a_system_change_nothing(name, method):

@@ -40,3 +40,12 @@ def test_explicit_row_kernels_declare_no_lds(kernels, kernel):
     """Nothing of theirs is indexed per thread: arrays that the compiler moves to LDS for that cost every launch a
     read of its packet in host memory."""
     assert find(kernels, f"row_integrate<wind::Net{kernel}>")[1] == 0
+
+
+@pytest.mark.parametrize("net", ["Katz96", "HHe6"])
+@pytest.mark.parametrize("method", [0, 1])
+def test_hand_over_leaves_the_lane_kernels_their_waves(kernels, net, method):
+    """As many waves per SIMD (512 VGPRs, given in eights) with the hand-over in the loop as without it."""
+    waves = [512 // (-(-find(kernels, f"lane_integrate<wind::Net{net}, {method}, wind::MathExact, false, {spill}>")[0]
+                       // 8) * 8) for spill in (0, 1)]
+    assert waves[0] == waves[1]

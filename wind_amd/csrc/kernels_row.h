@@ -302,68 +302,26 @@ constexpr bool row_network() {
     return TileOf<Net>::NTILE == 1 && Net::N <= 8;
 }
 
-// Largest batch that the row kernel takes whole: one row wave per SIMD
-// (4 systems each), or four with an implicit method on five or more equations,
-// whose attempts are long enough to pay for the idle lanes.  Kernel times,
-// lane against row kernel (reference controller unless said): hhe6 SIE 1000
-// systems 338 / 60 ms, 4096 375 / 68, 16384 411 / 131; katz96 SIE 80 systems
-// 0.75 / 0.26 ms, 8192 1.13 / 0.44, 20000 1.03 / 0.89; katz96 RK2 4096
-// 0.148 / 0.096, 20000 0.198 / 0.162 (adaptive 8192 0.036 / 0.050); NR_test
-// SIE 4096 0.140 / 0.106, 8192 0.139 / 0.127, 20000 0.147 / 0.239 (adaptive
-// 4096 0.044 / 0.048, 8192 0.044 / 0.063).
-// With a hand-over available (SIE, reference controller, rows / lanes with
-// hand-over) hhe6 4097 systems took 62.7 / 68.1 ms, 5000 71.0 / 65.8, 16384
-// 142 / 72; katz96 8192 0.43 / 0.52, 12000 0.67 / 0.62.
-template <class Net, int METHOD>
-inline int row_max_systems(int num_cu, bool handover) {
-    if (METHOD != WIND_SIE || Net::N < 5) return 16 * num_cu;
-    return (!handover ? 64 : Net::N == 5 ? 40 : 16) * num_cu;
-}
+// Systems per CU up to which rows are the faster form whatever the systems'
+// lengths: the largest batch that the row kernel takes whole, and the number
+// of unfinished systems at which a larger one's go on on rows.  At 16 every
+// SIMD has one row wave (4 systems).  Kernel times, lane against row kernel:
+// hhe6 SIE 1000 systems 338 / 60 ms, 4096 375 / 68, all of 400 attempts 3.1 /
+// 1.0; katz96 SIE 80 systems 0.75 / 0.26; katz96 RK2 4096 0.152 / 0.082; NR_test
+// SIE 4096 0.162 / 0.117, adaptive 0.073 / 0.069.  More rows than that only pay
+// where few systems are long (SIE, 16,384 systems, hhe6 411 / 131, but of one
+// length 3.1 / 3.2, katz96 1.2 / 1.6).  Adaptive calls of five equations make too
+// few attempts for 16 (katz96 to t = 2, 4096 systems, lanes / rows 36 / 40 us).
+constexpr int row_limit_per_cu(int N, int controller) { return N == 5 && controller == WIND_CTRL_ADAPTIVE ? 8 : 16; }
 
-// Start order of the row kernel's systems (SIE): most remaining attempts
-// first, as the attempts so far extrapolate over the time left (rank
-// correlation 0.7 to 0.76 with the true ones on hhe6 after 600 to 5000
-// attempts; RK2's steps grow too unevenly for it).  A counting sort into four
-// classes per octave, one workgroup.
-template <int N>
-__global__ void __launch_bounds__(1024) spill_order(IntegrateArgs a) {
-    constexpr int C = 64;
-    __shared__ unsigned start[C];
-    const unsigned *words = reinterpret_cast<const unsigned *>(a.counters);
-    const bool second = (int)words[SPILL_FIRST] > a.spill_pack;
-    const int n = (int)words[second ? SPILL_SECOND : SPILL_FIRST], t = threadIdx.x;
-    const float *list = a.spill + (size_t)(second ? a.spill_cap : 0) * spill_record_words(N);
-    auto cls = [&](int k) {
-        const float *r = list + (size_t)k * spill_record_words(N);
-        const float est = (float)__float_as_int(r[N + 3]) * (a.tend - r[N]) / fmaxf(r[N] - a.tnow, 1.0e-30f);
-        // exponent and two mantissa bits, from 2^4 up; NaN first, as longest
-        const int b = (int)(__float_as_uint(est) >> 21) - ((127 + 4) << 2);
-        return C - 1 - min(max(b, 0), C - 1);
-    };
-    if (t < C) start[t] = 0;
-    __syncthreads();
-    for (int k = t; k < n; k += 1024) atomicAdd(&start[cls(k)], 1u);
-    __syncthreads();
-    if (t == 0) {
-        unsigned run = 0;
-        for (int i = 0; i < C; i++) {
-            const unsigned c = start[i];
-            start[i] = run;
-            run += c;
-        }
-    }
-    __syncthreads();
-    for (int k = t; k < n; k += 1024) a.spill_index[atomicAdd(&start[cls(k)], 1u)] = k;
+// Where nothing can be handed over (handover false: batches, the server, the
+// output-step driver) an implicit method on five or more equations takes 32:
+// lanes throughout are the only other choice, and at 32 rows are faster whatever
+// the systems' lengths (8192 systems, hhe6 1.7 to 3.6 times, katz96 1.2 to 1.3; at
+// 64 per CU, 0.98 and 0.73 times where all are of one length).
+inline int row_max_systems(int N, int method, int controller, int num_cu, bool handover) {
+    return (!handover && method == WIND_SIE && N >= 5 ? 32 : row_limit_per_cu(N, controller)) * num_cu;
 }
-
-// Row workgroups per CU behind a lane kernel: with one wave per SIMD (RK2,
-// which divides less, two) the longest systems run at their own pace, and the
-// order has something to choose from.  hhe6 SIE, 8 (all that fit) / 2 / 1 per
-// CU, in list order: 100,003 systems 177 / 144 / 143 ms, 50,003 121 / 111 / 85,
-// 1,000,003 321 / 294 / 299; longest first 169 / 133 / 137, 105 / 102 / 82 and
-// 303 / 278 / 276.  RK2, 100,003 systems 104 / 59 / 83 in list order, 93 / 70 /
-// 95 longest first.
-constexpr int row_tail_per_cu(int method) { return method == WIND_SIE ? 1 : 2; }
 
 // Threads that give each of nsys systems a row.
 inline int row_threads(int nsys) { return 16 * (nsys < (1 << 26) ? nsys : 1 << 26); }
@@ -376,7 +334,7 @@ __device__ inline void row_take(bool take, int src, T &v) {
 }
 
 // One system per row, four per wave, taken from the device queue; or (TAIL)
-// the systems that the lane kernel before it handed over (a.spill).
+// the systems that the lane kernels before it handed over (a.spill), a row each.
 template <class Net, int METHOD, bool TAIL = false>
 __global__ void __launch_bounds__(256) row_integrate(IntegrateArgs a, typename Net::Params p) {
     constexpr int N = Net::N, NC = Net::NCONST;
@@ -385,7 +343,7 @@ __global__ void __launch_bounds__(256) row_integrate(IntegrateArgs a, typename N
     const bool mine = li < N;
     unsigned int *const words = reinterpret_cast<unsigned int *>(a.counters);
     unsigned int *head = words + (TAIL ? SPILL_ROW_HEAD : 0);
-    const bool second = TAIL && (int)words[SPILL_FIRST] > a.spill_pack;
+    const bool second = TAIL && (int)words[SPILL_FIRST] > a.spill_rows;
     const int count = !TAIL ? a.nsys : (int)words[second ? SPILL_SECOND : SPILL_FIRST];
     RowEval<Net, MathExact> ev(p, li);
     float y[N], c[NC > 0 ? NC : 1], yo = 0.0f, tnow = 0.0f, h = 0.0f;
@@ -410,9 +368,7 @@ __global__ void __launch_bounds__(256) row_integrate(IntegrateArgs a, typename N
                 active = got < count;
                 if (active) {
                     if constexpr (TAIL) {
-                        const float *r = a.spill + (size_t)((METHOD == WIND_SIE ? a.spill_index[got] : got) +
-                                                               (second ? a.spill_cap : 0)) *
-                                                      spill_record_words(N);
+                        const float *r = a.spill + (size_t)(got + (second ? a.spill_cap : 0)) * spill_record_words(N);
                         yo = r[mine ? li : 0];
                         tnow = r[N];
                         h = r[N + 1];

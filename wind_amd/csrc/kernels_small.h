@@ -373,8 +373,6 @@ __device__ inline void wave_add_steps(unsigned long long *total, unsigned long l
     if (__lane_id() == 0 && v) atomicAdd(total, v);
 }
 
-// The body of lane_integrate, shared with kernels that set other launch
-// bounds or are compiled with other floating-point contraction.
 // Hands the wave's unfinished systems (lanes `busy`) over, into the first
 // list or (SECOND) the second.
 template <int N, bool SECOND>
@@ -402,15 +400,39 @@ __device__ inline void spill_systems(const IntegrateArgs &a, const LaneSys<N> &s
     for (int v = 0; v < R / 4; v++) out[v] = make_float4(r[4 * v], r[4 * v + 1], r[4 * v + 2], r[4 * v + 3]);
 }
 
-// SPILL: with a.spill set, the wave's last systems are handed over; 2: the
-// second pass, over the systems of the first list.
+// Attempts that one of a wave's systems has made before the wave hands over,
+// so that a call whose systems are all short ends in the lane kernel.
+constexpr int spill_after(int N, int method, bool to_rows) {
+    if (method == WIND_SIE) return N > 5 ? 16 : 64;
+    return to_rows && N > 5 ? 64 : 512;
+}
+
+// The body of lane_integrate, shared with kernels that set other launch
+// bounds or are compiled with other floating-point contraction.
+// SPILL: the call's last systems are handed over (IntegrateArgs::spill); 2:
+// the second pass, over the systems of the first list.
 template <class Net, int METHOD, class M, bool TRACE = false, int SPILL = 0>
 __device__ inline void lane_integrate_body(const IntegrateArgs &a, const typename Net::Params &p) {
     constexpr int N = Net::N;
     constexpr int NC = Net::NCONST;
     unsigned int *head = reinterpret_cast<unsigned int *>(a.counters) + (SPILL == 2 ? SPILL_LANE_HEAD : 0);
     const int count = SPILL == 2 ? (int)reinterpret_cast<const unsigned *>(a.counters)[SPILL_FIRST] : a.nsys;
-    if (SPILL == 2 && count <= a.spill_pack) return;
+    if (SPILL == 2 && count <= a.spill_rows) return;
+    // Every lane asks the queue once for its first system and once for each
+    // one it finishes, so the queue's head tells how many are unfinished: at
+    // most the limit from this value on, the queue being empty.  (Waves that
+    // have not asked yet only make it lower.)
+    const unsigned lanes = gridDim.x * blockDim.x, limit = (unsigned)(SPILL == 2 ? a.spill_rows : a.spill_cap);
+    const bool to_rows = SPILL == 2 || a.spill_cap == a.spill_rows;
+    const int after = spill_after(N, METHOD, to_rows);
+    // The head is looked at every 16th attempt once this wave has at most
+    // twice the systems that a wave has on average then, seldom before: a read
+    // waits behind all waves' reads and fetches.  Katz96 SIE to t = 200, 10^6
+    // systems: 9.4 ms, read by every wave at every 16th attempt 14.3, without
+    // hand-over 9.2.
+    const int few = __builtin_amdgcn_readfirstlane(max(8, (int)min(64u, 128u * limit / lanes)));
+    int turn = 0;
+    const unsigned spill_from = (unsigned)count + (lanes > limit ? lanes - limit : 0u);
     LaneSys<N> s;
     float c[NC];
     int sid = 0;
@@ -421,11 +443,10 @@ __device__ inline void lane_integrate_body(const IntegrateArgs &a, const typenam
     // such waves the device runs), so none is left idle: 9,973 systems to 1 Myr
     // 16.7 -> 11.3 ms, 2^20 systems unchanged, RK2 131,072 78.9 -> 76.9 ms.
     constexpr bool FILL = M::kFast && !TRACE;
-    bool active = false, need = true, dry = false, fill = false;
+    bool active = false, need = true, fill = false;
     unsigned long long steps = 0;
     for (;;) {
         const int got = queue_fetch(head, need);
-        if constexpr (SPILL != 0) dry = dry || __any(need && got >= count);
         if (need) {
             need = false;
             active = got < count;
@@ -505,9 +526,16 @@ __device__ inline void lane_integrate_body(const IntegrateArgs &a, const typenam
             }
         }
         if constexpr (SPILL != 0) {
-            if (dry && __popcll(busy) <= a.spill_at) {
-                spill_systems<N, SPILL == 2>(a, s, sid, active, busy);
-                break;
+            turn = __builtin_amdgcn_readfirstlane(turn + 1);
+            if (__builtin_expect((turn & 15) == 0, 0) && (__popcll(busy) <= few || (turn & 255) == 0) &&
+                __any(active && s.attempts >= after)) {
+                int at = 0;  // made opaque, so that the address takes no register elsewhere
+                asm volatile("" : "+v"(at));
+                const unsigned h = __hip_atomic_load(head + at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if ((unsigned)__builtin_amdgcn_readfirstlane((int)h) >= spill_from) {
+                    spill_systems<N, SPILL == 2>(a, s, sid, active, busy);
+                    break;
+                }
             }
         }
         if ((FILL || active) && attempt<Net, METHOD, M, TRACE>(p, a, c, s, sid)) {

@@ -7,7 +7,9 @@
 // its end since ABI 4: a plugin built before reads the part it knows and
 // runs without the rest, and a core of that time passes only that part,
 // so a plugin takes the members from `spill` on only from a core that has
-// told it how many bytes it passes (wind_plugin_args, optional).
+// told it how many bytes it passes (wind_plugin_args2, optional; another
+// meaning of those members takes another name, so that plugins and cores that
+// differ in it do without).
 #pragma once
 #include <hip/hip_runtime.h>
 

@@ -81,7 +81,8 @@ int plugin_launch_method(const IntegrateArgs &a, int mode, int kernel, int num_c
     } else if (choice == 0) {
         if constexpr (Net::N <= kGenLaneMaxN) {
             if constexpr (row_network<Net>()) {
-                if (kernel == WIND_KERNEL_AUTO && a.nsys <= row_max_systems<Net, METHOD>(num_cu, a.spill != nullptr)) {
+                if (kernel == WIND_KERNEL_AUTO &&
+                    a.nsys <= row_max_systems(Net::N, METHOD, a.controller, num_cu, a.spill != nullptr)) {
                     auto k = row_integrate<Net, METHOD>;
                     int grid = 0;
                     const int rc = plugin_grid(k, 256, row_threads(a.nsys), num_cu, share, grid_cap, &grid);
@@ -96,11 +97,10 @@ int plugin_launch_method(const IntegrateArgs &a, int mode, int kernel, int num_c
                     int grid = 0;
                     const int rc = plugin_grid(k, 256, a.nsys, num_cu, share, grid_cap, &grid);
                     if (rc) return rc;
-                    const int grid_t = row_tail_per_cu(METHOD) * num_cu;
+                    const int grid_t = (a.spill_rows + 15) / 16;  // a row each
                     hipLaunchKernelGGL(k, dim3(grid), dim3(256), 0, st, a, p);
-                    if (a.spill_cap > a.spill_pack) hipLaunchKernelGGL(k2, dim3(num_cu), dim3(256), 0, st, a, p);
-                    if (METHOD == WIND_SIE)
-                        hipLaunchKernelGGL(spill_order<Net::N>, dim3(1), dim3(1024), 0, st, a);
+                    if (a.spill_cap > a.spill_rows)
+                        hipLaunchKernelGGL(k2, dim3((a.spill_cap + 255) / 256), dim3(256), 0, st, a, p);
                     hipLaunchKernelGGL(kt, dim3(grid_t), dim3(256), 0, st, a, p);
                     return hipGetLastError() == hipSuccess ? WIND_OK : WIND_ERR_DEVICE;
                 }
@@ -119,7 +119,7 @@ int plugin_launch_method(const IntegrateArgs &a, int mode, int kernel, int num_c
 }
 
 // Bytes of IntegrateArgs that the core passes: those of ABI 4's first form
-// until the core names more (wind_plugin_args).
+// until the core names more (wind_plugin_args2).
 static std::atomic<size_t> g_args_bytes{offsetof(IntegrateArgs, spill)};
 
 template <class Net>
@@ -199,7 +199,7 @@ int plugin_scratch_fast(int nsys, int method, int kernel, int num_cu, float shar
 
 #if WIND_PLUGIN_PART == 1
 #define WIND_DEFINE_PLUGIN(NET, NAME, NREACT, FLOPS_RHS, FLOPS_JAC)                                      \
-    extern "C" __attribute__((visibility("default"))) void wind_plugin_args(size_t bytes) {               \
+    extern "C" __attribute__((visibility("default"))) void wind_plugin_args2(size_t bytes) {               \
         wind::g_args_bytes = bytes < sizeof(wind::IntegrateArgs) ? bytes : sizeof(wind::IntegrateArgs);   \
     }                                                                                                      \
     extern "C" __attribute__((visibility("default"))) const wind_plugin_desc *wind_plugin_get(void) {     \

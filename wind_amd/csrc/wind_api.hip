@@ -74,7 +74,7 @@ struct CallSlot {
     Pool hint, order;  // cost hints copied from the host; start order and class counts
     Pool records;      // systems packed in start order (lane kernels of compiled-in networks)
     Pool activity;     // initial-state work estimates (start order without caller hints)
-    Pool spill;        // systems that a lane kernel hands over to the row kernel
+    Pool spill;        // systems that a kernel hands over to the next one (IntegrateArgs::spill)
     Pool io;           // small host-pointer calls: constants, counters, state, steps and status in one piece
     void *host = nullptr;  // pinned image of io (kStageBytes)
     Pool trace;        // per-attempt trace arrays of host-pointer calls
@@ -310,23 +310,23 @@ int activity_hints(int num_cu, const wind_network *net, const IntegrateArgs &a, 
     }
 }
 
-// Lanes of a wave at which, its queue empty, its last systems are handed
-// over (to a second lane pass where they still fill waves, more than 32 per
-// CU, and to the row kernel in the end, kernels_row.h): a lane wave costs
-// three row waves' instructions whatever its lanes do, and a row attempt takes
-// a third of the time.  hhe6 SIE, reference controller, 20,000 (t = 1 Myr) /
-// 100,003 (1 Myr) / 1,000,003 systems (10^4 yr): 391 / 475 / 634 ms without
-// hand-over; at 24 / 32 / 40 lanes 77 / 88 / 81, 154 / 137 / 135 and 292 / 276 /
-// 279; at 32 without the second pass 74 / 143 / 357 (all before the row kernel's
-// idle rows repeated a neighbour's system: 137 -> 127 at 40).  katz96 200,000 2.92 ms
-// without, 2.11 at 40, 2.88 at 32 without the second pass; NR_test (N = 2)
-// 200,000 0.50 without, 0.52 to 0.89 with, so only systems of five equations
-// on do it.
-constexpr int kSpillAt = 40;
-constexpr int kSpillPackPerCu = 32;
-bool spills(const wind_network *net, int mode, int nsys, int num_cu) {
+// Exact calls larger than the row kernel takes whole hand their last systems
+// over to it when no more are unfinished than it would take (kernels_row.h),
+// and to a second lane pass before that, when no more are unfinished than one
+// full lane wave per SIMD holds.  The count of the whole call decides, not a
+// wave's own: what has been handed over waits for the slowest wave's last
+// system otherwise (handed over wave by wave at 40 systems, calls whose systems
+// are of one length took up to twice as long as without hand-over, hhe6 SIE,
+// 16,384 systems of 400 attempts, 3.1 -> 6.4 ms; now 3.2).  hhe6 SIE, reference
+// controller, without hand-over / so: 20,000 systems (1 Myr) 391 / 65 ms,
+// 100,003 (1 Myr) 475 / 125, at 128 or 512 per CU for the second pass 131 and
+// 191; 1,000,003 (10^4 yr) 634 / 337; katz96, 100,003 (t = 200) 1.60 / 1.31;
+// NR_test (N = 2) gains nothing, so only systems of five equations on do it.
+constexpr int kSpillPackPerCu = 256;
+bool spills(const wind_network *net, const wind_options &o, int nsys, int num_cu) {
     const bool lanes = net->builtin == WIND_NET_KATZ96 || net->builtin == WIND_NET_HHE6 || net->builtin == WIND_NET_PLUGIN;
-    return mode == WIND_MODE_EXACT && lanes && net->N >= 5 && net->N <= 8 && nsys > 16 * num_cu;
+    return o.mode == WIND_MODE_EXACT && o.kernel == WIND_KERNEL_AUTO && !o.trace && lanes && net->N >= 5 &&
+           net->N <= 8 && nsys > row_limit_per_cu(net->N, o.controller) * num_cu;
 }
 
 template <class K>
@@ -349,7 +349,7 @@ int launch_small(int num_cu, const wind_network *net, const IntegrateArgs &a, in
         const int grid = scaled_grid(num_cu, 32, sc, a.nsys);
         hipLaunchKernelGGL((block_integrate<Net, METHOD>), dim3(grid), dim3(64), 0, st, a, p);
     } else if (mode == WIND_MODE_EXACT && kernel == WIND_KERNEL_AUTO && a.trace.capacity == 0 &&
-               a.nsys <= row_max_systems<Net, METHOD>(num_cu, a.spill != nullptr)) {
+               a.nsys <= row_max_systems(Net::N, METHOD, a.controller, num_cu, a.spill != nullptr)) {
         auto k = row_integrate<Net, METHOD>;
         int grid = 0;
         int rc = persistent_grid(num_cu, k, 256, row_threads(a.nsys), &grid, sc);
@@ -362,10 +362,10 @@ int launch_small(int num_cu, const wind_network *net, const IntegrateArgs &a, in
         int grid = 0;
         int rc = persistent_grid(num_cu, k, 256, a.nsys, &grid, sc);
         if (rc) return rc;
-        const int grid_t = row_tail_per_cu(METHOD) * num_cu;
+        const int grid_t = (a.spill_rows + 15) / 16;  // a row each
         hipLaunchKernelGGL(k, dim3(grid), dim3(256), 0, st, a, p);
-        if (a.spill_cap > a.spill_pack) hipLaunchKernelGGL(k2, dim3(num_cu), dim3(256), 0, st, a, p);
-        if (METHOD == WIND_SIE) hipLaunchKernelGGL(spill_order<Net::N>, dim3(1), dim3(1024), 0, st, a);
+        if (a.spill_cap > a.spill_rows)
+            hipLaunchKernelGGL(k2, dim3((a.spill_cap + 255) / 256), dim3(256), 0, st, a, p);
         hipLaunchKernelGGL(kt, dim3(grid_t), dim3(256), 0, st, a, p);
     } else if (mode == WIND_MODE_EXACT) {
         auto k = a.trace.capacity > 0 ? lane_integrate<Net, METHOD, MathExact, true>
@@ -637,7 +637,7 @@ int wind_network_create_plugin(const char *path, wind_network **out) {
         dlclose(dl);
         return fail(WIND_ERR_ARGUMENT, "not a network plugin of this library version");
     }
-    if (auto args = (wind_plugin_args_fn)dlsym(dl, "wind_plugin_args")) args(sizeof(IntegrateArgs));
+    if (auto args = (wind_plugin_args_fn)dlsym(dl, "wind_plugin_args2")) args(sizeof(IntegrateArgs));
     wind_network *n = new wind_network();
     n->builtin = WIND_NET_PLUGIN;
     n->N = d->N;
@@ -997,17 +997,13 @@ int wind_integrate(const wind_network *net, float tnow, float tend, int n_integr
         if (rc) return rc;
     }
     a.records = pk.rec;
-    if (opts.kernel == WIND_KERNEL_AUTO && !opts.trace && spills(net, opts.mode, Nsystems, c.num_cu)) {
-        a.spill_at = kSpillAt;
-        a.spill_pack = kSpillPackPerCu * c.num_cu;
-        // at most 32 waves per CU, each of which hands over once; two lists
-        const size_t most = std::min((size_t)Nsystems, (size_t)c.num_cu * 32 * kSpillAt);
-        a.spill_cap = (int)most;
-        const size_t words = (size_t)spill_record_words(Neqn) * 2 * most;
-        rc = reserve(sl->spill, sizeof(float) * (words + most));
+    if (spills(net, opts, Nsystems, c.num_cu)) {
+        a.spill_rows = row_limit_per_cu(Neqn, opts.controller) * c.num_cu;
+        a.spill_cap = Nsystems > kSpillPackPerCu * c.num_cu ? kSpillPackPerCu * c.num_cu : a.spill_rows;
+        const size_t records = (size_t)a.spill_cap + a.spill_rows;
+        rc = reserve(sl->spill, sizeof(float) * spill_record_words(Neqn) * records);
         if (rc) return rc;
         a.spill = (float *)sl->spill.ptr;
-        a.spill_index = (int32_t *)(a.spill + words);
     } else if (const int cap = dense_reg_hand_cap(net, opts, sc, Nsystems, c.num_cu)) {
         rc = reserve(sl->spill, sizeof(float) * kDenseHandWords * (size_t)cap);
         if (rc) return rc;

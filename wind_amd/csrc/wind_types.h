@@ -47,13 +47,14 @@ struct IntegrateArgs {
     // bits) of system index[q], packed in queue order, so that lanes read the
     // systems they take contiguously instead of gathering them
     const float *records = nullptr;
-    // optional (lane kernels with a row-kernel tail, kernels_row.h): a wave
-    // whose queue is empty and whose unfinished systems are at most
-    // spill_at hands them over, each as a record of spill_record_words(N)
-    // floats.  First list: records 0 .. spill_cap - 1 of spill; when it holds
-    // more than spill_pack systems, a second pass of the lane kernel takes
-    // them, packed into full waves again, and hands its own last ones over in
-    // the second list, behind the first.  The row kernel takes the last list.
+    // optional (lane kernels with a row-kernel tail, kernels_row.h): once the
+    // queue is empty and at most spill_cap systems of the call are unfinished,
+    // every wave hands its systems over, each as a record of
+    // spill_record_words(N) floats, into a list of spill_cap records.  Where
+    // that list holds more than spill_rows systems, a second pass of the lane
+    // kernel takes them, packed into full waves again, and hands over in the
+    // same way at spill_rows unfinished, into a second list of spill_rows
+    // records behind the first.  The row kernel takes the last list.
     // The lists' lengths and queue heads are 32-bit words of counters
     // (SpillWord).
     // The register dense solver (kernels_dense_reg.h) with spill set: its
@@ -61,8 +62,7 @@ struct IntegrateArgs {
     // unfinished, the state in place in equations, the rest as a record of
     // kDenseHandWords words, and the eight-wave form continues them.
     float *spill = nullptr;
-    int32_t *spill_index = nullptr;  // the row kernel's start order, [spill_cap]
-    int32_t spill_at = 0, spill_cap = 0, spill_pack = 0;
+    int32_t spill_cap = 0, spill_rows = 0;
 };
 
 // 32-bit words of IntegrateArgs::counters for the hand-over: lengths of the
