@@ -314,13 +314,16 @@ constexpr bool row_network() {
 // few attempts for 16 (katz96 to t = 2, 4096 systems, lanes / rows 36 / 40 us).
 constexpr int row_limit_per_cu(int N, int controller) { return N == 5 && controller == WIND_CTRL_ADAPTIVE ? 8 : 16; }
 
+// Equations from which on a call's last systems are handed over (IntegrateArgs::spill).
+constexpr int kSpillMinN = 5;
+
 // Where nothing can be handed over (handover false: batches, the server, the
 // output-step driver) an implicit method on five or more equations takes 32:
 // lanes throughout are the only other choice, and at 32 rows are faster whatever
 // the systems' lengths (8192 systems, hhe6 1.7 to 3.6 times, katz96 1.2 to 1.3; at
 // 64 per CU, 0.98 and 0.73 times where all are of one length).
 inline int row_max_systems(int N, int method, int controller, int num_cu, bool handover) {
-    return (!handover && method == WIND_SIE && N >= 5 ? 32 : row_limit_per_cu(N, controller)) * num_cu;
+    return (!handover && method == WIND_SIE && N >= kSpillMinN ? 32 : row_limit_per_cu(N, controller)) * num_cu;
 }
 
 // Threads that give each of nsys systems a row.

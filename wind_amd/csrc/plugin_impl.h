@@ -90,19 +90,21 @@ int plugin_launch_method(const IntegrateArgs &a, int mode, int kernel, int num_c
                     hipLaunchKernelGGL(k, dim3(grid), dim3(256), 0, st, a, p);
                     return hipGetLastError() == hipSuccess ? WIND_OK : WIND_ERR_DEVICE;
                 }
-                if (a.spill) {
-                    auto k = lane_integrate<Net, METHOD, MathExact, false, 1>;
-                    auto k2 = lane_integrate<Net, METHOD, MathExact, false, 2>;
-                    auto kt = row_integrate<Net, METHOD, true>;
-                    int grid = 0;
-                    const int rc = plugin_grid(k, 256, a.nsys, num_cu, share, grid_cap, &grid);
-                    if (rc) return rc;
-                    const int grid_t = (a.spill_rows + 15) / 16;  // a row each
-                    hipLaunchKernelGGL(k, dim3(grid), dim3(256), 0, st, a, p);
-                    if (a.spill_cap > a.spill_rows)
-                        hipLaunchKernelGGL(k2, dim3((a.spill_cap + 255) / 256), dim3(256), 0, st, a, p);
-                    hipLaunchKernelGGL(kt, dim3(grid_t), dim3(256), 0, st, a, p);
-                    return hipGetLastError() == hipSuccess ? WIND_OK : WIND_ERR_DEVICE;
+                if constexpr (Net::N >= kSpillMinN) {
+                    if (a.spill) {
+                        auto k = lane_integrate<Net, METHOD, MathExact, false, 1>;
+                        auto k2 = lane_integrate<Net, METHOD, MathExact, false, 2>;
+                        auto kt = row_integrate<Net, METHOD, true>;
+                        int grid = 0;
+                        const int rc = plugin_grid(k, 256, a.nsys, num_cu, share, grid_cap, &grid);
+                        if (rc) return rc;
+                        const int grid_t = (a.spill_rows + 15) / 16;  // a row each
+                        hipLaunchKernelGGL(k, dim3(grid), dim3(256), 0, st, a, p);
+                        if (a.spill_cap > a.spill_rows)
+                            hipLaunchKernelGGL(k2, dim3((a.spill_cap + 255) / 256), dim3(256), 0, st, a, p);
+                        hipLaunchKernelGGL(kt, dim3(grid_t), dim3(256), 0, st, a, p);
+                        return hipGetLastError() == hipSuccess ? WIND_OK : WIND_ERR_DEVICE;
+                    }
                 }
             }
             auto k = lane_integrate<Net, METHOD, MathExact>;

@@ -325,7 +325,7 @@ int activity_hints(int num_cu, const wind_network *net, const IntegrateArgs &a, 
 constexpr int kSpillPackPerCu = 256;
 bool spills(const wind_network *net, const wind_options &o, int nsys, int num_cu) {
     const bool lanes = net->builtin == WIND_NET_KATZ96 || net->builtin == WIND_NET_HHE6 || net->builtin == WIND_NET_PLUGIN;
-    return o.mode == WIND_MODE_EXACT && o.kernel == WIND_KERNEL_AUTO && !o.trace && lanes && net->N >= 5 &&
+    return o.mode == WIND_MODE_EXACT && o.kernel == WIND_KERNEL_AUTO && !o.trace && lanes && net->N >= kSpillMinN &&
            net->N <= 8 && nsys > row_limit_per_cu(net->N, o.controller) * num_cu;
 }
 
@@ -356,17 +356,19 @@ int launch_small(int num_cu, const wind_network *net, const IntegrateArgs &a, in
         if (rc) return rc;
         hipLaunchKernelGGL(k, dim3(grid), dim3(256), 0, st, a, p);
     } else if (mode == WIND_MODE_EXACT && a.spill) {
-        auto k = lane_integrate<Net, METHOD, MathExact, false, 1>;
-        auto k2 = lane_integrate<Net, METHOD, MathExact, false, 2>;
-        auto kt = row_integrate<Net, METHOD, true>;
-        int grid = 0;
-        int rc = persistent_grid(num_cu, k, 256, a.nsys, &grid, sc);
-        if (rc) return rc;
-        const int grid_t = (a.spill_rows + 15) / 16;  // a row each
-        hipLaunchKernelGGL(k, dim3(grid), dim3(256), 0, st, a, p);
-        if (a.spill_cap > a.spill_rows)
-            hipLaunchKernelGGL(k2, dim3((a.spill_cap + 255) / 256), dim3(256), 0, st, a, p);
-        hipLaunchKernelGGL(kt, dim3(grid_t), dim3(256), 0, st, a, p);
+        if constexpr (Net::N >= kSpillMinN) {
+            auto k = lane_integrate<Net, METHOD, MathExact, false, 1>;
+            auto k2 = lane_integrate<Net, METHOD, MathExact, false, 2>;
+            auto kt = row_integrate<Net, METHOD, true>;
+            int grid = 0;
+            int rc = persistent_grid(num_cu, k, 256, a.nsys, &grid, sc);
+            if (rc) return rc;
+            const int grid_t = (a.spill_rows + 15) / 16;  // a row each
+            hipLaunchKernelGGL(k, dim3(grid), dim3(256), 0, st, a, p);
+            if (a.spill_cap > a.spill_rows)
+                hipLaunchKernelGGL(k2, dim3((a.spill_cap + 255) / 256), dim3(256), 0, st, a, p);
+            hipLaunchKernelGGL(kt, dim3(grid_t), dim3(256), 0, st, a, p);
+        }
     } else if (mode == WIND_MODE_EXACT) {
         auto k = a.trace.capacity > 0 ? lane_integrate<Net, METHOD, MathExact, true>
                                       : lane_integrate<Net, METHOD, MathExact>;
