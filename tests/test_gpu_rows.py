@@ -218,6 +218,22 @@ def test_tiled_network_equals_oracle_also_where_a_tile_overflows(tiles, method, 
     assert same(y, yr) and np.array_equal(steps, sr) and np.array_equal(status, tr)
 
 
+def test_explicit_tiles_on_both_sides_of_their_limit():
+    """RK2 on a tiled network whose matrices are beyond LDS: the tile kernel up to a system per CU, the block kernel
+    above, the same bits."""
+    tiles = 50
+    N, n = 5 * tiles, num_cu() + 1
+    rng = np.random.default_rng(tiles)
+    y0 = np.tile(np.resize(W.KATZ96_FIXTURE_Y, 5 * n).reshape(n, 5), (1, tiles))
+    y0 = (y0 * rng.uniform(0.5, 1.5, y0.shape)).astype(np.float32).reshape(-1)
+    c = np.resize(W.KATZ96_FIXTURE_C, 10 * n).astype(np.float32)
+    kw = {"tend": 0.5, "tol": 5e-3, "method": api.RK2, "max_attempts": 20}
+    net = api.Network.plugin(f"katz96_t{tiles}")
+    y, steps, status = run(net, n, y0, c, api.KERNEL_AUTO, **kw)
+    part = run(net, n - 1, y0[:-N], c[:-10], api.KERNEL_AUTO, **kw)
+    assert same(part[0], y[:-N]) and np.array_equal(part[1], steps[:-1]) and np.array_equal(part[2], status[:-1])
+
+
 @pytest.mark.parametrize("n", [1, 3, 32000, 33500])
 def test_host_arrays_equal_device_arrays(n):
     """Host-pointer calls on both sides of the staging limit (1 MiB; 32 bytes a system here), outputs optional."""

@@ -94,12 +94,32 @@ __global__ void __launch_bounds__(row_tile_threads<Net>()) gen_tile_integrate(In
     });
 }
 
+// Whether an exact RK2 launch of a tiled network takes the tile kernel.  There
+// is no inverse to save, and a row does a tile's work in 16 lanes; it pays where
+// the block kernel's matrices (in LDS or scratch with either method) hold its
+// workgroups back, or a CU has one system.  Katz96, block against tile kernel:
+// N = 250, matrices beyond LDS, 256 systems 73 / 59 us, 257 72 / 83, 3000 132 /
+// 403; in LDS, 20,000 systems, N = 20 272 / 167, 25 275 / 230, 50 495 / 349, 100
+// 3036 / 1768.
+template <class Net>
+inline bool rk2_takes_tiles(int nsys, int num_cu) {
+    constexpr bool in_lds =
+        sizeof(float) * (gen_block_base_floats<Net>() + 2 * (size_t)Net::N * Net::N) + 1024 <= 160 * 1024;
+    return in_lds || nsys <= num_cu;
+}
+
 // The kernel of a launch and its threads per workgroup.
 template <class Net, int METHOD, bool FAST, bool PIVOT>
 inline auto gen_block_kernel(int nsys, int num_cu, int *threads) {
     if constexpr (!FAST && row_tile_network<Net>()) {
         *threads = row_tile_threads<Net>();
-        return gen_tile_integrate<Net, METHOD>;
+        auto kfn = gen_tile_integrate<Net, METHOD>;
+        if constexpr (METHOD == WIND_RK2)
+            if (!rk2_takes_tiles<Net>(nsys, num_cu)) {
+                *threads = block_threads(Net::N, nsys, num_cu);
+                kfn = gen_block_integrate<Net, METHOD, FAST, PIVOT>;
+            }
+        return kfn;
     } else {
         *threads = block_threads(Net::N, nsys, num_cu);
         return gen_block_integrate<Net, METHOD, FAST, PIVOT>;
