@@ -100,7 +100,7 @@ int launch_dense_reg_wgs(int num_cu, const MassActionDevice &d, const IntegrateA
 // 19.1 us per sub-step and CU against 25.2).
 //
 // The largest number of systems that the eight-wave form takes; 0: it is not built.
-static int dense_reg_few(int NT, int num_cu) { return NT >= 6 ? 2 * num_cu : NT >= 4 ? num_cu : 0; }
+static int dense_reg_few(int NT, int num_cu) { return NT >= 6 ? 2 * num_cu : NT >= kDenseRegMinNT8 ? num_cu : 0; }
 
 static int launch_dense_reg_few(int num_cu, const MassActionDevice &d, const IntegrateArgs &a, const SolverChoice &sc,
                          hipStream_t st) {

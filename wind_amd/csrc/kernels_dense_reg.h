@@ -507,7 +507,7 @@ __global__ void __launch_bounds__(64 * WR * WC, WGS *WR *WC / 4)
     };
 
     unsigned *const words = reinterpret_cast<unsigned *>(a.counters);
-    float *const hand = TRACE || NT < 4 ? nullptr : a.spill;  // (built from four tiles)
+    float *const hand = TRACE || NT < 4 ? nullptr : a.spill;  // (eight waves from four tiles on)
     for (;;) {
         if (t == 0) {
             if (WR > 2 && hand) {

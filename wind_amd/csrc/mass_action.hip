@@ -3,7 +3,8 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <map>
+#include <cstring>
+#include <functional>
 #include <string>
 #include <vector>
 
@@ -17,13 +18,35 @@ using namespace wind;
 
 namespace {
 
-int upload(void **dst, const void *src, size_t bytes) {
-    if (bytes == 0) bytes = 4;
-    hipError_t e = hipMalloc(dst, bytes);
+// The tables of a network, in one device allocation (each on a 256-byte
+// boundary) and one copy: the first table's address is the allocation's.
+struct Table {
+    void **dst;
+    const void *src;
+    size_t bytes;
+};
+int upload(const std::vector<Table> &tables) {
+    auto part = [](size_t b) { return (b + 255) & ~(size_t)255; };
+    size_t total = 256;
+    for (const Table &t : tables) total += part(t.bytes);
+    std::vector<char> host(total);
+    size_t at = 0;
+    for (const Table &t : tables) {
+        if (t.bytes) std::memcpy(host.data() + at, t.src, t.bytes);
+        at += part(t.bytes);
+    }
+    char *dev = nullptr;
+    hipError_t e = hipMalloc((void **)&dev, total);
     if (e != hipSuccess) return wind_fail(WIND_ERR_DEVICE, hipGetErrorString(e));
-    if (src) {
-        e = hipMemcpy(*dst, src, bytes, hipMemcpyHostToDevice);
-        if (e != hipSuccess) return wind_fail(WIND_ERR_DEVICE, hipGetErrorString(e));
+    e = hipMemcpy(dev, host.data(), total, hipMemcpyHostToDevice);
+    if (e != hipSuccess) {
+        (void)hipFree(dev);
+        return wind_fail(WIND_ERR_DEVICE, hipGetErrorString(e));
+    }
+    at = 0;
+    for (const Table &t : tables) {
+        *t.dst = dev + at;
+        at += part(t.bytes);
     }
     return WIND_OK;
 }
@@ -42,26 +65,63 @@ static bool ma_wave_fits(int N, int R) {
     return N <= 64 && sizeof(float) * ma_wave_lds_floats((N + 7) & ~7, R) <= 65536 - 64;
 }
 
-// Deals elements (their terms' words) to `threads` streams, most terms first
-// to the least-loaded thread; streams padded with `pad` to the longest,
-// rounded up to `batch`, and interleaved: word j of thread t at
-// [j * threads + t].
-static std::vector<int32_t> deal_streams(std::vector<std::vector<uint32_t>> &items, int threads, int batch,
-                                         uint32_t pad, int *len) {
-    std::stable_sort(items.begin(), items.end(), [](const auto &p1, const auto &p2) { return p1.size() > p2.size(); });
-    std::vector<std::vector<uint32_t>> per(threads);
-    for (auto &it : items) {
-        size_t th = 0;
-        for (size_t u = 1; u < per.size(); u++)
-            if (per[u].size() < per[th].size()) th = u;
-        per[th].insert(per[th].end(), it.begin(), it.end());
+// Lists of words, list z the words ptr[z] .. ptr[z + 1] - 1.
+struct WordLists {
+    std::vector<int32_t> key, ptr = {0};
+    std::vector<uint32_t> word;
+    size_t size() const { return ptr.size() - 1; }
+    void close() { ptr.push_back((int32_t)word.size()); }
+};
+
+// The words of each key (< nkeys) in their order in `word`, the non-empty keys ascending.
+static WordLists lists_by_key(int nkeys, const std::vector<int32_t> &key, const std::vector<uint32_t> &word) {
+    std::vector<int32_t> at(nkeys + 1, 0);
+    for (int32_t k : key) at[k + 1]++;
+    WordLists l;
+    for (int k = 0; k < nkeys; k++) {
+        if (at[k + 1]) {
+            l.key.push_back(k);
+            l.ptr.push_back(at[k] + at[k + 1]);
+        }
+        at[k + 1] += at[k];
     }
-    size_t n = batch;
-    for (auto &p : per) n = std::max(n, (p.size() + batch - 1) / batch * batch);
-    std::vector<int32_t> out(n * threads, (int32_t)pad);
-    for (int th = 0; th < threads; th++)
-        for (size_t j = 0; j < per[th].size(); j++) out[j * threads + th] = (int32_t)per[th][j];
-    *len = (int)n;
+    l.word.resize(word.size());
+    for (size_t i = 0; i < word.size(); i++) l.word[at[key[i]]++] = word[i];
+    return l;
+}
+
+// Deals elements (their terms' words) to `threads` streams, most terms first
+// to the least-loaded thread (the first of equals); streams padded with `pad`
+// to the longest, rounded up to `batch`, and interleaved: word j of thread t at
+// [j * threads + t].
+static std::vector<int32_t> deal_streams(const WordLists &items, int threads, int batch, uint32_t pad, int *len) {
+    auto terms = [&](int z) { return items.ptr[z + 1] - items.ptr[z]; };
+    int most = 0;
+    for (size_t z = 0; z < items.size(); z++) most = std::max(most, terms((int)z));
+    // by falling number of terms, equals in order (a counting sort)
+    std::vector<int32_t> start(most + 2, 0), order(items.size());
+    for (size_t z = 0; z < items.size(); z++) start[most - terms((int)z) + 1]++;
+    for (int c = 0; c <= most; c++) start[c + 1] += start[c];
+    for (size_t z = 0; z < items.size(); z++) order[start[most - terms((int)z)]++] = (int32_t)z;
+    // the threads with their loads, the least-loaded on top
+    using Load = std::pair<int32_t, int32_t>;
+    std::vector<Load> heap(threads);
+    for (int th = 0; th < threads; th++) heap[th] = {0, th};
+    std::vector<Load> place(items.size());  // first word's place in the stream, thread
+    int longest = 1;
+    for (int32_t z : order) {
+        std::pop_heap(heap.begin(), heap.end(), std::greater<Load>());
+        Load &top = heap.back();
+        place[z] = top;
+        top.first += terms(z);
+        longest = std::max(longest, top.first);
+        std::push_heap(heap.begin(), heap.end(), std::greater<Load>());
+    }
+    *len = (longest + batch - 1) / batch * batch;
+    std::vector<int32_t> out((size_t)*len * threads, (int32_t)pad);
+    for (size_t z = 0; z < items.size(); z++)
+        for (int j = 0; j < terms((int)z); j++)
+            out[(size_t)(place[z].first + j) * threads + place[z].second] = (int32_t)items.word[items.ptr[z] + j];
     return out;
 }
 
@@ -70,27 +130,32 @@ int mass_action_build(wind_network *n, int N, int R, const int32_t *rx, const fl
     n->k.assign(k, k + R);
     // Contribution lists in the order of a serial sweep over reactions.
     std::vector<std::vector<int32_t>> flist(N);
-    std::map<int, std::vector<int32_t>> jlist;
-    for (int r = 0; r < R; r++) {
-        const int32_t *x = rx + 4 * r;
-        for (int slot = 0; slot < 4; slot++) {
-            const int neg = slot < 2 ? 1 : 0;
-            flist[x[slot]].push_back(r * 2 + neg);
-            jlist[x[0] * N + x[slot]].push_back(((r * 2 + 0) * 2) + neg);
-            jlist[x[1] * N + x[slot]].push_back(((r * 2 + 1) * 2) + neg);
+    WordLists jlist;
+    {
+        std::vector<int32_t> key;
+        std::vector<uint32_t> ent;
+        key.reserve(8 * (size_t)R);
+        ent.reserve(8 * (size_t)R);
+        for (int r = 0; r < R; r++) {
+            const int32_t *x = rx + 4 * r;
+            for (int slot = 0; slot < 4; slot++) {
+                const int neg = slot < 2 ? 1 : 0;
+                flist[x[slot]].push_back(r * 2 + neg);
+                for (int which = 0; which < 2; which++) {
+                    key.push_back(x[which] * N + x[slot]);
+                    ent.push_back((uint32_t)(((r * 2 + which) * 2) + neg));
+                }
+            }
         }
+        jlist = lists_by_key(N * N, key, ent);
     }
     std::vector<int32_t> f_ptr(N + 1, 0), f_ent;
     for (int i = 0; i < N; i++) {
         f_ent.insert(f_ent.end(), flist[i].begin(), flist[i].end());
         f_ptr[i + 1] = (int32_t)f_ent.size();
     }
-    std::vector<int32_t> j_pos, j_ptr(1, 0), j_ent;
-    for (auto &kv : jlist) {
-        j_pos.push_back(kv.first);
-        j_ent.insert(j_ent.end(), kv.second.begin(), kv.second.end());
-        j_ptr.push_back((int32_t)j_ent.size());
-    }
+    const std::vector<int32_t> &j_pos = jlist.key, &j_ptr = jlist.ptr;
+    const std::vector<int32_t> j_ent(jlist.word.begin(), jlist.word.end());
     std::vector<std::vector<int32_t>> rows(N);
     for (size_t z = 0; z < j_pos.size(); z++) rows[j_pos[z] % N].push_back((int32_t)z);
     std::vector<int32_t> r_ptr(N + 1, 0), r_z;
@@ -124,25 +189,33 @@ int mass_action_build(wind_network *n, int N, int R, const int32_t *rx, const fl
     if (dense_reg_tiles(NT)) {
         const DenseRegOffsets lo = dense_reg_offsets(NT, R, 3, 0);
         bool ok = lo.hdb + R < 65536;
-        std::map<std::pair<int, int>, std::vector<uint32_t>> elem;  // (row, col) -> words without last
-        for (int i = 0; i < N && ok; i++)
-            for (int32_t e : flist[i]) {
-                const int r = e >> 1, neg = e & 1;
-                const int32_t *x = rx + 4 * r;
-                for (int which = 0; which < 2; which++) {
-                    const uint32_t hd = (uint32_t)((which ? lo.hdb : lo.hda) + r);
-                    elem[{i, x[which]}].push_back((hd << 16) | ((x[which] == i ? 1u : 0u) << 2) | (uint32_t)!neg);
+        WordLists elem;  // by row * N + col
+        if (ok) {
+            std::vector<int32_t> key;
+            std::vector<uint32_t> word;
+            key.reserve(8 * (size_t)R);
+            word.reserve(8 * (size_t)R);
+            for (int i = 0; i < N; i++)
+                for (int32_t e : flist[i]) {
+                    const int r = e >> 1, neg = e & 1;
+                    const int32_t *x = rx + 4 * r;
+                    for (int which = 0; which < 2; which++) {
+                        const uint32_t hd = (uint32_t)((which ? lo.hdb : lo.hda) + r);
+                        key.push_back(i * N + x[which]);
+                        word.push_back((hd << 16) | ((x[which] == i ? 1u : 0u) << 2) | (uint32_t)!neg);
+                    }
                 }
-            }
+            elem = lists_by_key(N * N, key, word);
+        }
         // the q present per (tile, lane), then the offsets
         std::vector<uint32_t> mask4((size_t)NT * NT * 64, 0);
         auto slot = [&](int row, int col, int *tl, int *q) {
             *tl = ((row >> 4) * NT + (col >> 4)) * 64 + 16 * ((row & 15) >> 2) + (col & 15);
             *q = row & 3;
         };
-        for (auto &kv : elem) {
+        for (int32_t key : elem.key) {
             int tl, q;
-            slot(kv.first.first, kv.first.second, &tl, &q);
+            slot(key / N, key % N, &tl, &q);
             mask4[tl] |= 1u << q;
         }
         sc_tile.resize(mask4.size());
@@ -154,31 +227,28 @@ int mass_action_build(wind_network *n, int N, int R, const int32_t *rx, const fl
         // (+1: an owner lane reads one place past its elements, unused)
         sc_cap = (int)((nnz + 1 + 3) & ~3u);
         ok = ok && sc_cap + 16 * NT <= 8192;
-        std::vector<std::vector<uint32_t>> items;
-        for (auto &kv : elem) {
-            int tl, q;
-            slot(kv.first.first, kv.first.second, &tl, &q);
-            const uint32_t dest = (sc_tile[tl] >> 4) + (uint32_t)__builtin_popcount(mask4[tl] & ((1u << q) - 1));
-            std::vector<uint32_t> w = kv.second;
-            for (auto &x : w) x |= dest << 3;
-            w.front() |= 2u;
-            items.push_back(std::move(w));
-        }
-        for (int i = 0; i < N && ok; i++) {
-            std::vector<uint32_t> w;
-            for (int32_t e : flist[i])
-                w.push_back((uint32_t)(lo.w + (e >> 1)) << 16 | (uint32_t)(sc_cap + i) << 3 | (uint32_t)(e & 1));
-            if (w.empty()) continue;
-            w.front() |= 2u;
-            items.push_back(std::move(w));
-        }
-        sc_ent = deal_streams(items, 256, kDenseRegBatch, nnz << 3, &sc_len);
-        sc_ent2 = deal_streams(items, 512, kDenseRegBatch, nnz << 3, &sc_len2);
-        if (!ok) {
-            sc_ent.clear();
-            sc_ent2.clear();
+        if (ok) {
+            for (size_t z = 0; z < elem.size(); z++) {
+                int tl, q;
+                slot(elem.key[z] / N, elem.key[z] % N, &tl, &q);
+                const uint32_t dest = (sc_tile[tl] >> 4) + (uint32_t)__builtin_popcount(mask4[tl] & ((1u << q) - 1));
+                for (int32_t j = elem.ptr[z]; j < elem.ptr[z + 1]; j++) elem.word[j] |= dest << 3;
+                elem.word[elem.ptr[z]] |= 2u;
+            }
+            for (int i = 0; i < N; i++) {
+                if (flist[i].empty()) continue;
+                const size_t first = elem.word.size();
+                for (int32_t e : flist[i])
+                    elem.word.push_back((uint32_t)(lo.w + (e >> 1)) << 16 | (uint32_t)(sc_cap + i) << 3 |
+                                        (uint32_t)(e & 1));
+                elem.word[first] |= 2u;
+                elem.close();
+            }
+            sc_ent = deal_streams(elem, 256, kDenseRegBatch, nnz << 3, &sc_len);
+            if (NT >= kDenseRegMinNT8) sc_ent2 = deal_streams(elem, 512, kDenseRegBatch, nnz << 3, &sc_len2);
+        } else {
             sc_tile.clear();
-            sc_len = sc_len2 = sc_cap = 0;
+            sc_cap = 0;
         }
     }
     // Assembly of the exact register kernel (ma_wave_integrate): f's and the
@@ -190,51 +260,55 @@ int mass_action_build(wind_network *n, int N, int R, const int32_t *rx, const fl
     if (ma_wave_fits(N, R)) {
         const int NP = (N + 7) & ~7;
         const uint32_t f0 = NP * NP + 3 * NP, w0 = f0 + NP;
-        std::vector<std::vector<uint32_t>> items;
+        WordLists items;
         for (int i = 0; i < N; i++) {
-            std::vector<uint32_t> w;
-            for (int32_t e : flist[i]) w.push_back((w0 + (uint32_t)(e >> 1)) << 16 | (f0 + i) << 3 | (uint32_t)(e & 1));
-            if (!w.empty()) items.push_back(std::move(w));
+            if (flist[i].empty()) continue;
+            for (int32_t e : flist[i])
+                items.word.push_back((w0 + (uint32_t)(e >> 1)) << 16 | (f0 + i) << 3 | (uint32_t)(e & 1));
+            items.word.back() |= 2u;
+            items.close();
         }
-        for (auto &kv : jlist) {
-            const uint32_t dest = (uint32_t)(kv.first / N * NP + kv.first % N);
-            std::vector<uint32_t> w;
-            for (int32_t e : kv.second)
-                w.push_back((w0 + (uint32_t)(R * ((e & 2) ? 2 : 1) + (e >> 2))) << 16 | dest << 3 | (uint32_t)(e & 1));
-            items.push_back(std::move(w));
+        for (size_t z = 0; z < jlist.size(); z++) {
+            const uint32_t dest = (uint32_t)(j_pos[z] / N * NP + j_pos[z] % N);
+            for (int32_t j = j_ptr[z]; j < j_ptr[z + 1]; j++) {
+                const int32_t e = j_ent[j];
+                items.word.push_back((w0 + (uint32_t)(R * ((e & 2) ? 2 : 1) + (e >> 2))) << 16 | dest << 3 |
+                                     (uint32_t)(e & 1));
+            }
+            items.word.back() |= 2u;
+            items.close();
         }
-        for (auto &w : items) w.back() |= 2u;
         ex_ent = deal_streams(items, 128, kMaWaveBatch, 0, &ex_len);
     }
     MassActionDevice &d = n->ma;
     d.N = N;
     d.R = R;
     d.nnz = (int)j_pos.size();
-    int rc = upload((void **)&d.rx, rx, sizeof(int32_t) * 4 * R);
-    if (!rc) rc = upload((void **)&d.k, k, sizeof(float) * R);
-    if (!rc) rc = upload((void **)&d.f_ptr, f_ptr.data(), sizeof(int32_t) * f_ptr.size());
-    if (!rc) rc = upload((void **)&d.f_ent, f_ent.data(), sizeof(int32_t) * f_ent.size());
-    if (!rc) rc = upload((void **)&d.j_pos, j_pos.data(), sizeof(int32_t) * j_pos.size());
-    if (!rc) rc = upload((void **)&d.j_ptr, j_ptr.data(), sizeof(int32_t) * j_ptr.size());
-    if (!rc) rc = upload((void **)&d.j_ent, j_ent.data(), sizeof(int32_t) * j_ent.size());
-    if (!rc) rc = upload((void **)&d.r_ptr, r_ptr.data(), sizeof(int32_t) * r_ptr.size());
-    if (!rc) rc = upload((void **)&d.r_z, r_z.data(), sizeof(int32_t) * r_z.size());
-    if (!rc && !sc_ent.empty()) rc = upload((void **)&d.sc_ent, sc_ent.data(), sizeof(int32_t) * sc_ent.size());
-    if (!rc && !sc_ent.empty()) rc = upload((void **)&d.sc_tile, sc_tile.data(), sizeof(uint32_t) * sc_tile.size());
-    if (!rc && !ex_ent.empty()) rc = upload((void **)&d.ex_ent, ex_ent.data(), sizeof(int32_t) * ex_ent.size());
-    d.ex_len = ex_len;
-    if (!rc && !sc_ent2.empty()) rc = upload((void **)&d.sc_ent2, sc_ent2.data(), sizeof(int32_t) * sc_ent2.size());
-    d.sc_len2 = sc_len2;
     d.sc_len = sc_len;
     d.sc_cap = sc_cap;
-    return rc;
+    d.sc_len2 = sc_len2;
+    d.ex_len = ex_len;
+    std::vector<Table> tables = {{(void **)&d.rx, rx, sizeof(int32_t) * 4 * R}, {(void **)&d.k, k, sizeof(float) * R}};
+    auto add = [&](auto &dst, const auto &v) { tables.push_back({(void **)&dst, v.data(), sizeof(v[0]) * v.size()}); };
+    add(d.f_ptr, f_ptr);
+    add(d.f_ent, f_ent);
+    add(d.j_pos, j_pos);
+    add(d.j_ptr, j_ptr);
+    add(d.j_ent, j_ent);
+    add(d.r_ptr, r_ptr);
+    add(d.r_z, r_z);
+    if (!sc_ent.empty()) {
+        add(d.sc_ent, sc_ent);
+        add(d.sc_tile, sc_tile);
+    }
+    if (!sc_ent2.empty()) add(d.sc_ent2, sc_ent2);
+    if (!ex_ent.empty()) add(d.ex_ent, ex_ent);
+    return upload(tables);
 }
 
 void mass_action_release(wind_network *n) {
     MassActionDevice &d = n->ma;
-    void *ptrs[] = {d.rx, d.k, d.f_ptr, d.f_ent, d.j_pos, d.j_ptr, d.j_ent, d.r_ptr, d.r_z, d.sc_ent, d.sc_tile, d.sc_ent2, d.ex_ent};
-    for (void *p : ptrs)
-        if (p) (void)hipFree(p);
+    if (d.rx) (void)hipFree(d.rx);  // the allocation of all tables (upload)
     d = MassActionDevice();
 }
 

@@ -31,7 +31,7 @@ struct MassActionDevice {
     int32_t *sc_ent = nullptr;
     uint32_t *sc_tile = nullptr;
     int sc_len = 0, sc_cap = 0;
-    int32_t *sc_ent2 = nullptr;  // the streams of 512 threads, sc_len2 words each
+    int32_t *sc_ent2 = nullptr;  // the streams of 512 threads, sc_len2 words each (kDenseRegMinNT8)
     int sc_len2 = 0;
     // Exact register kernel (N <= 64, format in mass_action_build): word j
     // of thread t's term stream at ex_ent[j * 128 + t], ex_len words each.
@@ -94,6 +94,7 @@ int launch_dense(int num_cu, const wind::MassActionDevice &d, const wind::Integr
 // built for, whether it takes this network and choice (fast mode, FP32
 // tiles, no refinement, two workgroups' LDS per CU), and its launch.
 constexpr int kDenseRegMinNT = 1, kDenseRegMaxNT = 10;
+constexpr int kDenseRegMinNT8 = 4;  // built for eight waves per system from here on
 // Against the LDS solver, ms for a whole batch of a mixed-size network: N = 12
 // 0.09 / 0.15 (1 system), 13.8 / 24.9 (512), 22.1 / 37.8 (4,096), 52.3 / 71.8
 // (16,384); N = 24 9.2 / 14.8, 32.7 / 53.7, 46.3 / 66.5, 104 / 125; N = 40
