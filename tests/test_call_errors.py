@@ -44,7 +44,8 @@ def fake(tmp_path_factory):
 
 
 def child(fake, body, *args):
-    r = subprocess.run([sys.executable, "-c", CHILD + body, fake, ROOT, *map(str, args)], capture_output=True, text=True)
+    r = subprocess.run([sys.executable, "-c", CHILD + body, fake, ROOT, *map(str, args)], capture_output=True, text=True,
+                       timeout=60)
     assert r.returncode == 0, r.stdout + r.stderr
 
 
@@ -96,4 +97,20 @@ for limit in (need - own + 256, need - 1, need, need + 1000):
     b = C.c_size_t()
     assert d.scratch(80, api.SIE, api.MODE_EXACT, api.KERNEL_AUTO, 256, 0.0, 0, C.byref(b)) == 0
     assert (b.value == 0) == (limit >= need), (limit, need, b.value)
+""")
+
+
+def test_network_tables_go_up_in_one_allocation(fake):
+    """A mass-action network's tables: the only allocation failing is an error of the call, and a later one works."""
+    child(fake, r"""
+for N, R in ((1, 0), (9, 0), (3, 12), (64, 256), (170, 680)):
+    rx, k = W.mass_action_network(N, 5, R=R)
+    for what, fails in (("hipMalloc", 1), ("hipMalloc", 2)):
+        fake.fake_fail(what.encode(), fails)
+        try:
+            api.Network.mass_action(N, rx, k).close()
+            assert fails == 2, (N, R)
+        except api.WindError:
+            assert fails == 1, (N, R)
+        fake.fake_fail(what.encode(), 0)
 """)

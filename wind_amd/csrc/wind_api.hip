@@ -616,7 +616,10 @@ int wind_network_create_mass_action(int N, int R, const int32_t *rx, const float
     n->nconst = 1;
     rc = mass_action_build(n, N, R, rx, k);
     if (rc) {
-        wind_network_destroy(n);
+        // (not wind_network_destroy: it takes the lock held here, and no cache
+        // knows the network yet)
+        mass_action_release(n);
+        delete n;
         return rc;
     }
     *out = n;
