@@ -441,8 +441,10 @@ __device__ inline void lane_integrate_body(const IntegrateArgs &a, const typenam
     // lanes runs slower than a full one (hhe6 SIE, one attempt of a wave alone
     // on its SIMD: 1.9 us with 64 lanes, 2.1 to 6.2 us with one, by how many
     // such waves the device runs), so none is left idle: 9,973 systems to 1 Myr
-    // 16.7 -> 11.3 ms, 2^20 systems unchanged, RK2 131,072 78.9 -> 76.9 ms.
-    constexpr bool FILL = M::kFast && !TRACE;
+    // 16.7 -> 11.3 ms, 2^20 systems unchanged, RK2 131,072 78.9 -> 76.9 ms; three
+    // species 9973 systems 0.98 -> 0.71 ms.  Two species' attempts are too short to
+    // pay for it (NR_test 140,000 systems 232 / 251 us without / with).
+    constexpr bool FILL = M::kFast && !TRACE && N > 2;
     bool active = false, need = true, fill = false;
     unsigned long long steps = 0;
     for (;;) {
