@@ -15,7 +15,8 @@ the bound) are reported beside it, and so is the same integration with the
 previous step's per-system sub-step counts as cost hints (longest systems
 first; bit-identical results), the case of a caller that integrates the
 same cells again.
-Also reported (one JSON line): the final-state relative error of a
+Also reported (one JSON line with the main figures, all of them in the --detail
+file): the final-state relative error of a
 512-system sample against FP64 Radau solutions (tests/golden/truth_hhe6.npz),
 per-step latency p50/p99, the integration kernel's roofline position, the
 reference algorithm as the reference runs it (exact arithmetic, reference
@@ -668,6 +669,32 @@ def _spearman(a, b):
     return float((ra * rb).sum() / np.sqrt((ra * ra).sum() * (rb * rb).sum()))
 
 
+LINE_MAX = 4000  # characters of the printed line: a captured output's tail holds all of it
+
+
+def compact(line, limit=LINE_MAX):
+    """The report as one JSON line of at most `limit` characters: numbers to six digits, and beside the headline's
+    own fields the legs as deep as there is room for (the --detail file has all of them)."""
+    def prune(v, depth):
+        if isinstance(v, float):
+            return float(f"{v:.6g}")
+        if isinstance(v, dict):
+            if depth == 0:
+                return None
+            kept = {k: prune(x, depth - 1) for k, x in v.items() if not (isinstance(x, str) and len(x) > 40)}
+            return {k: x for k, x in kept.items() if x is not None} or None
+        return None if isinstance(v, (list, tuple)) else v
+
+    own = ("metric", "value", "unit", "n_gpus", "steps", "warmup", "ms_per_step", "higher_is_better", "scaling",
+           "vs_baseline", "dtype", "data", "config", "latency_ms")
+    for depth in range(6, -1, -1):
+        text = json.dumps({k: v if k in own else prune(v, depth) for k, v in line.items()
+                           if k in own or prune(v, depth) is not None})
+        if len(text) <= limit:
+            break
+    return text
+
+
 def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--gpus", type=int, default=1)
@@ -700,6 +727,8 @@ def main():
                     help="timed steps of the headline with the previous step's sub-step counts as cost hints")
     ap.add_argument("--copy-probe", type=int, default=0,
                     help="only copy this many bytes device to device three times (HBM counter calibration)")
+    ap.add_argument("--detail", default=os.path.join(ROOT, "bench_detail.json"),
+                    help="file for the whole report; the printed line holds its main figures")
     a = ap.parse_args()
     if a.gpus != 1:
         print(f"bench.py measures one GPU only (--gpus {a.gpus} requested): systems are independent, so "
@@ -941,7 +970,9 @@ def main():
         "cpu_baseline": cpu, "cpu_same_algorithm": cpu_same,
         "wind_published_katz96": wind_pub, "mixed_batch": mixed, "dense_157": dense, "dense_157_precision": precision, "serving": serve,
     }
-    print(json.dumps(line))
+    with open(a.detail, "w") as f:
+        json.dump(line, f, indent=1)
+    print(compact(line))
 
 
 if __name__ == "__main__":
