@@ -3,12 +3,12 @@
 // (2 x 2, or 4 x 2 for few systems, dense.hip) owns one system at a time,
 // systems taken from a device queue, and the matrix A = I - hJ lives in the
 // waves' registers instead of LDS: wave (wi, wj) holds the 16x16 tiles (i, j)
-// with i = wi (mod WR), j = wj (mod WC), each in the MFMA accumulator layout (lane l holds rows 4(l/16) + q, q = 0..3, of
-// column l % 16).  Without the matrix in LDS a workgroup needs a third
-// (N > 144 and few enough reactions: a quarter) of a CU's LDS and
-// registers, so three (four) systems share a CU and each one's serial
-// parts (the pivot chain of a diagonal block, the barriers) overlap with
-// the others' work.
+// with i = wi (mod WR), j = wj (mod WC), each in the MFMA accumulator layout
+// (lane l holds rows 4(l/16) + q, q = 0..3, of column l % 16).  Without the
+// matrix in LDS a workgroup needs a third to an eighth of a CU's LDS and
+// registers (dense_reg_wgs_for), so three to eight systems share a CU and each
+// one's serial parts (the pivot chain of a diagonal block, the barriers)
+// overlap with the others' work.
 //
 // Per pass (step-doubling sub-step) of an attempt:
 // * assembly: the per-reaction rate terms and f as in the LDS solver

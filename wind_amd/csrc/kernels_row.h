@@ -454,9 +454,12 @@ __global__ void __launch_bounds__(256) row_integrate(IntegrateArgs a, typename N
 // zeros, which changes no non-zero bit, and a zero's sign cannot reach the
 // result (the mat-vec's sums start at +0).  That holds for finite values; in
 // the dense elimination an infinity or a NaN of one tile reaches the others
-// through those zeros.  Every non-finite matrix, inverse or f entry makes
-// its tile's sub-step result non-finite, so a system with a non-finite
-// result is integrated again by the dense path (dense(sid)).
+// through those zeros.  A non-finite f or inverse entry makes its tile's
+// sub-step result non-finite, and so does a non-finite matrix entry, through
+// the pivot that it meets, but for an infinite diagonal alone: it scales its
+// own row to zeros, in the dense elimination as here.  So a system with a
+// non-finite result is integrated again, from its start, by the dense path
+// (dense(sid)).
 // The tiles share the step control, and the first tile's state where the
 // network's temporaries read it; both go through LDS, with one barrier per
 // attempt for each.

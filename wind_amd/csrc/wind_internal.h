@@ -92,7 +92,7 @@ int launch_dense(int num_cu, const wind::MassActionDevice &d, const wind::Integr
 
 // Register-resident dense SIE solver (dense.hip): tiles per dimension it is
 // built for, whether it takes this network and choice (fast mode, FP32
-// tiles, no refinement, two workgroups' LDS per CU), and its launch.
+// tiles, no refinement, three workgroups' LDS per CU), and its launch.
 constexpr int kDenseRegMinNT = 1, kDenseRegMaxNT = 10;
 constexpr int kDenseRegMinNT8 = 4;  // built for eight waves per system from here on
 // Against the LDS solver, ms for a whole batch of a mixed-size network: N = 12
