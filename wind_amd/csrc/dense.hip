@@ -92,12 +92,10 @@ int launch_dense_reg_wgs(int num_cu, const MassActionDevice &d, const IntegrateA
 }
 
 // Few systems: eight waves each, two workgroups per CU, no register
-// spilled.  A system alone on its CU: N = 160 46.6 -> 37.0 us per
-// sub-step, 128 29.2 -> 24.6, 96 18.4 -> 16.7, 64 10.6 -> 9.8; two per
-// CU: 56.1 -> 50.3, 35.1 -> 33.2, 21.6 -> 21.8, 12.2 -> 12.7 (512
-// systems to the end, N = 160 512 -> 450 ms, 128 367 -> 320, 96 159 ->
-// 152).  With the CU full the four-wave form is the better one (N = 160
-// 19.1 us per sub-step and CU against 25.2).
+// spilled.  Four waves against eight, us per sub-step of a system alone on its
+// CU: N = 160 42.0 / 31.7, 128 24.6 / 21.0, 96 15.6 / 14.8, 64 9.5 / 9.1; two per CU:
+// 49.5 / 39.7, 29.1 / 26.3, 18.0 / 18.5 (512 systems to the end 144 ms in either
+// form), 10.8 / 11.6; three: 56.7 / 67.3, 33.4 / 44.0, 20.4 / 34.0, 12.2 / 20.0.
 //
 // The largest number of systems that the eight-wave form takes; 0: it is not built.
 static int dense_reg_few(int NT, int num_cu) { return NT >= 6 ? 2 * num_cu : NT >= kDenseRegMinNT8 ? num_cu : 0; }
