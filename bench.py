@@ -677,7 +677,7 @@ def compact(line, limit=LINE_MAX):
     own fields the legs as deep as there is room for (the --detail file has all of them)."""
     def prune(v, depth):
         if isinstance(v, float):
-            return float(f"{v:.6g}")
+            return float(f"{v:.6g}") if np.isfinite(v) else None
         if isinstance(v, dict):
             if depth == 0:
                 return None
