@@ -65,6 +65,19 @@ def test_dense_hand_over_from_the_smallest_batch_that_does(N):
                        controller=api.CTRL_ADAPTIVE, max_attempts=300)
 
 
+@pytest.mark.parametrize("method", [api.SIE, api.RK2])
+@pytest.mark.parametrize("controller", [api.CTRL_REFERENCE, api.CTRL_ADAPTIVE])
+@pytest.mark.parametrize("per_cu", [0, 16, 20, 300])
+def test_eight_equations_on_rows(method, controller, per_cu):
+    """The largest network that rows take: small batches, the largest that is rows throughout, and hand-overs with
+    and without the second lane pass, against the lane kernel."""
+    net, n = api.Network.plugin("mass_action8"), per_cu * num_cu() + (5 if per_cu != 16 else 0)
+    y0, c = W.mass_action_systems(n, 8, 11, W.MIXED_SCALE_RANGE)
+    kw = {"tend": 1e7, "tol": 1e-8, "rel": 1e-4, "method": method, "controller": controller, "max_attempts": 700}
+    a, b = (run(net, n, y0, c, k, **kw) for k in (api.KERNEL_LANE, api.KERNEL_AUTO))
+    assert same(a[0], b[0]) and np.array_equal(a[1], b[1]) and np.array_equal(a[2], b[2])
+
+
 def test_plugin_that_does_not_know_the_grown_arguments(tmp_path):
     """A plugin file without the entry that tells it of them reads the part it knows: the same bits, no hand-over."""
     built = os.path.join(os.path.dirname(api.LIB_PATH), "gen", "mixed5", "libwind_net.so")

@@ -217,7 +217,8 @@ def katz96_scaling_systems(ntile: int, nsystem_tile: int = 20):
 
 def generated_specs():
     """Descriptions of the networks that the build generates: the mixed
-    workload's N = 5 and N = 10 networks (as "mixed5", "mixed10"), a small
+    workload's N = 5 and N = 10 networks (as "mixed5", "mixed10"), one of the
+    largest size that exact calls give 16 lanes per system ("mass_action8"), a small
     network with one- and two-body reactions and two constants per system
     ("demo_decay"), that network tiled three times ("demo_decay_t3"), and the
     reference's networks from their expressions: Katz96 ("katz96_gen"), Katz96
@@ -231,6 +232,7 @@ def generated_specs():
     for N in GENERATED_MIXED:
         rx, k = mixed_network(N)
         specs.append(codegen.mass_action_spec(f"mixed{N}", N, rx, k))
+    specs.append(codegen.mass_action_spec("mass_action8", 8, *mass_action_network(8, seed=1008)))
     demo = {
         "name": "demo_decay", "species": 4, "nconst": 2,
         "reactions": [
