@@ -14,6 +14,7 @@
 static std::map<hipStream_t, std::vector<std::function<void()>>> g_queue;
 static std::map<std::string, int> g_fail;
 static std::map<const void *, std::string> g_kernel;  // device function names
+static std::string g_launched;  // their names, in order, one a line
 static std::string g_static_name;                     // kernels with this in their name use g_static bytes of LDS
 static int g_static = 0, g_max_lds = 163840;
 
@@ -34,6 +35,13 @@ int fake_pending() {
     return n;
 }
 void fake_fail(const char *name, int n) { g_fail[name] = n; }
+// The kernels launched since the last call.
+const char *fake_launched() {
+    static std::string out;
+    out.swap(g_launched);
+    g_launched.clear();
+    return out.c_str();
+}
 void fake_lds(int max_lds, const char *kernel, int bytes) {
     g_max_lds = max_lds;
     g_static_name = kernel;
@@ -56,7 +64,8 @@ hipError_t __hipPopCallConfiguration(dim3 *grid, dim3 *block, size_t *lds, hipSt
     *grid = g_config.grid, *block = g_config.block, *lds = g_config.lds, *st = g_config.st;
     return hipSuccess;
 }
-hipError_t hipLaunchKernel(const void *, dim3, dim3, void **, size_t, hipStream_t s) {
+hipError_t hipLaunchKernel(const void *k, dim3, dim3, void **, size_t, hipStream_t s) {
+    g_launched += g_kernel[k] + "\n";
     g_queue[s].push_back([] {});
     return hipSuccess;
 }

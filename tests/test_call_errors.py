@@ -100,6 +100,22 @@ for limit in (need - own + 256, need - 1, need, need + 1000):
 """)
 
 
+@pytest.mark.parametrize("N,R,form", [(32, 716, (2, 8)), (32, 2018, (2, 3)), (64, 734, (4, 6)), (64, 1586, (4, 3))])
+def test_dense_forms_reach_the_networks_that_their_lds_allows(fake, N, R, form):
+    """The largest networks that the register solver takes with its full number of workgroups per CU, and at all."""
+    child(fake, r"""
+import re
+N, R, form = int(sys.argv[3]), int(sys.argv[4]), sys.argv[5]
+net = api.Network.mass_action(N, *W.mass_action_network(N, 5, R=R))
+y, c = W.mass_action_systems(3000, N, 1)
+fake.fake_launched.restype = C.c_char_p
+fake.fake_launched()
+api.integrate(net, 0.0, 1.0, 1, c, y, 3000, 1e-3, 1e-3, mode=api.MODE_FAST, controller=api.CTRL_ADAPTIVE)
+names = fake.fake_launched().decode()
+assert "ma_dense_reg_integrateILi%sELi%sE" % tuple(form.split(",")) in names, names
+""", N, R, "%d,%d" % form)
+
+
 def test_network_tables_go_up_in_one_allocation(fake):
     """A mass-action network's tables: the only allocation failing is an error of the call, and a later one works."""
     child(fake, r"""

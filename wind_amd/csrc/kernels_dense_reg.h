@@ -81,10 +81,11 @@ constexpr int kDenseRegGW = NT >= 8 ? 2 : 1;
 constexpr int kDenseRegWC = 2;
 
 // LDS layout of the register-resident solver (offsets in floats, 16-byte
-// aligned): per-system vectors, the sweeps' partial sums, per-reaction rate terms, reactant indices
-// and rate constants, and a work area shared by the assembly's compact
-// element buffer (cap floats) with f behind it, and the factorisation's panel
-// buffers.  The term lists stay in global memory.
+// aligned): per-system vectors, per-reaction rate terms (the sweeps' partial
+// sums in the same place later), reactant indices and rate constants, and a work
+// area shared by the assembly's compact element buffer (cap floats) with f
+// behind it, and the factorisation's panel buffers.  The term lists stay in
+// global memory.
 struct DenseRegOffsets {
     int y, yw, y1, r, part, w, hda, hdb, k, ab, work, total;
 };
@@ -102,14 +103,18 @@ __host__ __device__ inline DenseRegOffsets dense_reg_offsets(int NT, int R, int 
     p = up(p + NP);
     o.r = p;
     p = up(p + NP);
-    o.part = p;
-    p = up(p + 3 * kDenseRegWC * 16);
     o.w = p;
     p = up(p + R);
     o.hda = p;
     p = up(p + R);
     o.hdb = p;
     p = up(p + R);
+    // the sweeps' partial sums, in the rate terms' place where it is large
+    // enough: the terms are read for the last time two barriers before the first
+    // of the sums is written, and written again after the sums' last barrier
+    constexpr int sums = 3 * kDenseRegWC * 16;
+    o.part = p - o.w >= sums ? o.w : p;
+    if (p - o.w < sums) p = up(p + sums);
     o.k = p;
     if (WGS == 3) p = up(p + R);  // rate constants in LDS
     o.ab = p;
